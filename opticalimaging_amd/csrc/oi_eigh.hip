@@ -1,16 +1,35 @@
-// Float64 Hermitian eigensolver: parallel two-sided cyclic Jacobi.
+// Float64 Hermitian eigensolver: parallel two-sided block Jacobi.
 //
-// Indices are paired by the round-robin (circle) schedule: m = n rounded up to
-// even, m-1 rounds per sweep, m/2 disjoint pairs per round (index n, when n is
-// odd, is a dummy).  A round computes all m/2 rotations from the current
-// matrix, then updates every 2x2 block (pair i, pair j) as U_i^H A_ij U_j and
-// the eigenvector columns as V U_j.  For pair (p, q) with c = A_pq = |c| e^{i phi},
-//   tau = (A_qq - A_pp) / (2|c|),  t = sign(tau) / (|tau| + sqrt(1 + tau^2)),
-//   cs = 1/sqrt(1 + t^2), sn = t cs,
-//   U = [[cs, sn], [-sn e^{-i phi}, cs e^{-i phi}]]
-// zeroes A_pq (phase removal followed by the real Jacobi rotation).  Sweeps
+// The indices are cut into blocks of kEb = 16.  Blocks are paired by the
+// round-robin (circle) schedule: m = block count rounded up to even, m - 1
+// outer rounds per sweep, m/2 disjoint block pairs per round (block m - 1 is a
+// dummy when the count is odd; indices past n read as zero and are never
+// written).  One outer round is two launches:
+//   k_solve   one workgroup per block pair: the 32 x 32 diagonal submatrix S of
+//             the pair in LDS, 16 rounds of 16 disjoint rotations that meet
+//             every index of one block with every index of the other (the
+//             first outer round of a sweep runs the 31 rounds that also meet
+//             the indices inside a block), their product U accumulated beside
+//             it.  S goes back to A as rotated, with exact zeros at the last
+//             round's pairs.
+//   k_update  tiles (pair I, pair J), I < J: A_IJ <- U_I^H A_IJ U_J (and its
+//             conjugate transpose at (J, I)); V's 32-row tiles: V_J <- V_J U_J.
+//             Two 32 x 32 x 32 complex products on the float64 matrix cores.
+// A rotation of indices (p, q) is U = [[c, g], [-conj g, c]], c^2 + |g|^2 = 1,
+// the one of the two that zero A_pq whose angle is at most 45 degrees.  Sweeps
 // stop when the off-diagonal Frobenius norm falls below tol times the diagonal
 // norm.
+//
+// What bounds it: latency.  n = 120 .. 600 is far too little work for the
+// chip, and a sweep is a chain of n - 1 dependent rounds.  As two launches per
+// rotation round the chain ran at launch latency (about 6 us a round); sixteen
+// rounds per launch pair run at LDS latency (k_solve 11.4 us = 0.65 us a round,
+// k_update 5.6-6.3 us up to n = 240, 12 us at n = 588).  16 x 16 blocks: with
+// 32 a round moves 128 KB through LDS and takes as long as two rounds here.
+// Rank-deficient graded matrices (the hardest of the tests), launch pair per
+// round -> blocks: n = 120 13.7 -> 3.8 ms, 240 40.8 -> 8.2 ms, 588 138 -> 27 ms,
+// 1024 316 -> 53 ms, eigenvalue errors 3.5e-14 / 7.7e-14 / 2.3e-13 / 3.0e-13
+// -> 3.1e-14 / 5.6e-14 / 7.8e-14 / 1.0e-13 of the largest.
 #include <cfloat>
 #include <cmath>
 #include <string>
@@ -19,11 +38,29 @@
 
 namespace oi {
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kEb = 16;            // indices per block
+constexpr int kEw = 2 * kEb;       // width of a pair's submatrix
+constexpr int kNormBlocks = 64;    // partial sums of the norms
+
+// A rotation U = [[c, g], [-conj g, c]] of indices (p, q); c = 0 never occurs.
 struct Rot {
-  double c, s, er, ei;  // cos, sin, e^{i phi}
+  double c, gx, gy;
 };
 
-__device__ __forceinline__ void pair_of(int i, int s, int m, int& p, int& q) {
+// Convergence state of a solve on the device: the norms of the last check,
+// whether they met the tolerance (later launches then return at once) and the
+// number of sweeps begun.
+struct EigState {
+  double off, diag;
+  int done, sweeps;
+};
+
+__host__ __device__ inline int eig_blocks(int n) { return (n + kEb - 1) / kEb; }
+__host__ __device__ inline int eig_pairs(int n) { return (eig_blocks(n) + 1) / 2; }
+
+__host__ __device__ __forceinline__ void pair_of(int i, int s, int m, int& p, int& q) {
   if (i == 0) {
     p = 0;
     q = 1 + pmod(s - 1, m - 1);
@@ -33,15 +70,63 @@ __device__ __forceinline__ void pair_of(int i, int s, int m, int& p, int& q) {
   }
 }
 
-__device__ __forceinline__ double2 zmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 zconj(double2 a) { return make_double2(a.x, -a.y); }
 __device__ __forceinline__ double2 zadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ double2 zscale(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
+// 1 / sqrt(x) for normal positive x: the hardware estimate (about 2^-28) and
+// two Newton steps (a square root's and a division's full sequences would sit
+// on every round's critical path).
+__device__ __forceinline__ double rsq2(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * fma(-x * r, r, 1.0), r, r);
+  return fma(0.5 * fma(-x * r, r, 1.0), r, r);
+}
 
-__global__ void k_eye(double2* __restrict__ V, int n) {
+// The rotation that zeroes A_pq = b between the diagonal values app and aqq.
+// With d = aqq - app and r = sqrt(d^2 + 4 |b|^2), cos 2theta = |d| / r and
+// sin 2theta = 2 |b| / r, so c = sqrt((1 + |d| / r) / 2) and
+// g = sign(d) b / (r c): two reciprocal square roots, no division, no phase.
+__device__ __forceinline__ Rot rotation(double app, double aqq, double2 b) {
+  double d = aqq - app;
+  double h = fma(d, d, 4.0 * fma(b.x, b.x, b.y * b.y));
+  if (!(h > 1e-280 && h < 1e290)) {          // squares near the ends of the range
+    const double big = fmax(fabs(d), fmax(fabs(b.x), fabs(b.y)));
+    if (!(big > 0.0)) return Rot{1.0, 0.0, 0.0};
+    int e;
+    (void)frexp(big, &e);
+    d = ldexp(d, -e);
+    b = make_double2(ldexp(b.x, -e), ldexp(b.y, -e));
+    h = fma(d, d, 4.0 * fma(b.x, b.x, b.y * b.y));
+  }
+  const double ir = rsq2(h);
+  const double c2 = fma(0.5 * fabs(d), ir, 0.5);
+  const double ic = rsq2(c2);
+  const double f = d >= 0.0 ? ir * ic : -(ir * ic);
+  return Rot{c2 * ic, b.x * f, b.y * f};
+}
+
+// The value of lane + 1 within each row of 16 lanes (lane 15 takes lane 0's).
+__device__ __forceinline__ double row_next(double v) {
+  constexpr int kRor15 = 0x12F;              // row rotate right by 15
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, kRor15, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, lo, kRor15, 0xf, 0xf, false));
+}
+__device__ __forceinline__ double2 row_next(double2 v) { return make_double2(row_next(v.x), row_next(v.y)); }
+
+// (a, b) <- (a, b) U for a pair of columns, and U^H applied to a pair of rows.
+__device__ __forceinline__ void rot_cols(const Rot& r, double2& a, double2& b) {
+  const double2 x = a, y = b;
+  a = make_double2(r.c * x.x - (r.gx * y.x + r.gy * y.y), r.c * x.y - (r.gx * y.y - r.gy * y.x));
+  b = make_double2(r.c * y.x + (r.gx * x.x - r.gy * x.y), r.c * y.y + (r.gx * x.y + r.gy * x.x));
+}
+__device__ __forceinline__ void rot_rows(const Rot& r, double2& a, double2& b) {
+  const double2 x = a, y = b;
+  a = make_double2(r.c * x.x - (r.gx * y.x - r.gy * y.y), r.c * x.y - (r.gx * y.y + r.gy * y.x));
+  b = make_double2(r.c * y.x + (r.gx * x.x + r.gy * x.y), r.c * y.y + (r.gx * x.y - r.gy * x.x));
+}
+
+__global__ void k_eye(double2* __restrict__ V, int n, EigState* __restrict__ state) {
   const size_t total = (size_t)n * n;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *state = EigState{0.0, 0.0, 0, 0};
   for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
        e += (size_t)gridDim.x * blockDim.x) {
     const int r = (int)(e / n), c = (int)(e - (size_t)r * n);
@@ -49,122 +134,262 @@ __global__ void k_eye(double2* __restrict__ V, int n) {
   }
 }
 
-__global__ void k_rot(const double2* __restrict__ A, int n, int m, int s, Rot* __restrict__ rot) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m / 2) return;
-  int p, q;
-  pair_of(i, s, m, p, q);
-  Rot r{1.0, 0.0, 1.0, 0.0};
-  if (p < n && q < n) {
-    const double app = A[(size_t)p * n + p].x, aqq = A[(size_t)q * n + q].x;
-    const double2 apq = A[(size_t)p * n + q];
-    const double mag = hypot(apq.x, apq.y);
-    if (mag > 0.0) {
-      const double tau = (aqq - app) / (2.0 * mag);
-      const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-      r.c = 1.0 / sqrt(1.0 + t * t);
-      r.s = t * r.c;
-      r.er = apq.x / mag;
-      r.ei = apq.y / mag;
-    }
-  }
-  rot[i] = r;
+// Index of a pair's local position (< kEw) in the matrix.
+__device__ __forceinline__ int eig_index(int P, int Q, int l) {
+  return l < kEb ? P * kEb + l : Q * kEb + l - kEb;
 }
 
-// Applies one round: items [0, h*h) are 2x2 blocks of A, items [h*h, h*h + n*h)
-// are (row, pair) updates of V.  h = m/2.
-__global__ void k_apply(double2* __restrict__ A, double2* __restrict__ V, int n, int m, int s,
-                        const Rot* __restrict__ rot) {
-  const int h = m / 2;
-  const size_t nblk = (size_t)h * h;
-  const size_t total = nblk + (size_t)n * h;
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-       e += (size_t)gridDim.x * blockDim.x) {
-    if (e < nblk) {
-      const int i = (int)(e / h), j = (int)(e - (size_t)i * h);
-      int pi, qi, pj, qj;
-      pair_of(i, s, m, pi, qi);
-      pair_of(j, s, m, pj, qj);
-      const Rot ri = rot[i], rj = rot[j];
-      const int R[2] = {pi, qi}, C[2] = {pj, qj};
-      double2 X[2][2];
+// Waves 0-3 rotate S (thread (i, j) owns the 2 x 2 block of index pairs i and
+// j, from one LDS buffer to the other, one barrier per round), waves 4-7
+// rotate U's 32 rows.  Every lane forms the rotation of its own pair j from S;
+// that of pair i comes from lane i of the wave.  In the rounds between two
+// blocks a lane keeps U's column j and passes the other block's columns to
+// its neighbour (they move by one per round), so U stays in registers; the
+// rounds that also pair inside a block (FULL) rotate U in LDS.
+template <bool FULL>
+__global__ __launch_bounds__(512) void k_solve(double2* __restrict__ A, int n, int m, int s,
+                                               double2* __restrict__ Uout,
+                                               const EigState* __restrict__ state) {
+  __shared__ double2 S[2][kEw * kEw];
+  __shared__ double2 U[FULL ? kEw * kEw : 1];
+  const int done = state->done;
+  int P, Q;
+  pair_of(blockIdx.x, s, m, P, Q);
+  const int tid = threadIdx.x;
+  constexpr int kLoads = kEw * kEw / 512;
+  double2 in[kLoads];
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          X[a][b] = (R[a] < n && C[b] < n) ? A[(size_t)R[a] * n + C[b]] : make_double2(0.0, 0.0);
-      // T = X U_j with U_j = [[c, s], [-s conj(e), c conj(e)]]
-      const double2 ej = zconj(make_double2(rj.er, rj.ei));
-      double2 T[2][2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        T[a][0] = zadd(zscale(X[a][0], rj.c), zscale(zmul(X[a][1], ej), -rj.s));
-        T[a][1] = zadd(zscale(X[a][0], rj.s), zscale(zmul(X[a][1], ej), rj.c));
-      }
-      // Y = U_i^H T with U_i^H = [[c, -s e], [s, c e]]
-      const double2 ei = make_double2(ri.er, ri.ei);
-      double2 Y[2][2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        Y[0][b] = zadd(zscale(T[0][b], ri.c), zscale(zmul(T[1][b], ei), -ri.s));
-        Y[1][b] = zadd(zscale(T[0][b], ri.s), zscale(zmul(T[1][b], ei), ri.c));
-      }
-      if (i == j) {
-        Y[0][1] = make_double2(0.0, 0.0);
-        Y[1][0] = make_double2(0.0, 0.0);
-        Y[0][0].y = 0.0;
-        Y[1][1].y = 0.0;
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          if (R[a] < n && C[b] < n) A[(size_t)R[a] * n + C[b]] = Y[a][b];
-    } else {
-      const size_t f = e - nblk;
-      const int k = (int)(f / h), j = (int)(f - (size_t)k * h);
-      int pj, qj;
-      pair_of(j, s, m, pj, qj);
-      if (pj >= n || qj >= n) continue;
-      const Rot rj = rot[j];
-      const double2 ej = zconj(make_double2(rj.er, rj.ei));
-      const double2 vp = V[(size_t)k * n + pj], vq = V[(size_t)k * n + qj];
-      const double2 vqe = zmul(vq, ej);
-      V[(size_t)k * n + pj] = zadd(zscale(vp, rj.c), zscale(vqe, -rj.s));
-      V[(size_t)k * n + qj] = zadd(zscale(vp, rj.s), zscale(vqe, rj.c));
-    }
+  for (int u = 0; u < kLoads; ++u) {
+    const int e = tid + 512 * u;
+    const int r = eig_index(P, Q, e / kEw), c = eig_index(P, Q, e % kEw);
+    in[u] = (r < n && c < n) ? A[(size_t)r * n + c] : make_double2(0.0, 0.0);
   }
-}
-
-// out[0] = sum_{p != q} |A_pq|^2, out[1] = sum_p A_pp^2 (single block).
-__global__ __launch_bounds__(1024) void k_offnorm(const double2* __restrict__ A, int n,
-                                                  double* __restrict__ out) {
-  __shared__ double so[1024], sd[1024];
-  double off = 0.0, dg = 0.0;
-  const size_t total = (size_t)n * n;
-  for (size_t e = threadIdx.x; e < total; e += blockDim.x) {
-    const int r = (int)(e / n), c = (int)(e - (size_t)r * n);
-    const double2 v = A[e];
-    const double a2 = v.x * v.x + v.y * v.y;
-    if (r == c)
-      dg += a2;
-    else
-      off += a2;
+  if (done) return;                          // uniform over the grid
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int e = tid + 512 * u;
+    S[0][e] = in[u];
+    if constexpr (FULL) U[e] = make_double2(e / kEw == e % kEw ? 1.0 : 0.0, 0.0);
   }
-  so[threadIdx.x] = off;
-  sd[threadIdx.x] = dg;
+  const int j = tid & 15;
+  const int i = (tid >> 4) & 15;             // pair of the block row (waves 0-3), U row (4-7)
+  // U rows i and i + 16, columns j and 16 + ((j + k) & 15) in round k
+  double2 ua[2], ub[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    ua[h] = make_double2(h == 0 && i == j ? 1.0 : 0.0, 0.0);
+    ub[h] = make_double2(h == 1 && i == j ? 1.0 : 0.0, 0.0);
+  }
   __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      so[threadIdx.x] += so[threadIdx.x + w];
-      sd[threadIdx.x] += sd[threadIdx.x + w];
+  constexpr int kRounds = FULL ? kEw - 1 : kEb;
+  for (int k = 0; k < kRounds; ++k) {
+    const double2* src = S[k & 1];
+    double2* dst = S[(k + 1) & 1];
+    int pi, qi, pj, qj;
+    if (FULL) {
+      pair_of(i, k, kEw, pi, qi);
+      pair_of(j, k, kEw, pj, qj);
+    } else {
+      pi = i;
+      qi = kEb + ((i + k) & 15);
+      pj = j;
+      qj = kEb + ((j + k) & 15);
+    }
+    const Rot rj = rotation(src[pj * kEw + pj].x, src[qj * kEw + qj].x, src[pj * kEw + qj]);
+    if (tid < 256) {
+      const Rot ri{__shfl(rj.c, i), __shfl(rj.gx, i), __shfl(rj.gy, i)};
+      double2 x00 = src[pi * kEw + pj], x01 = src[pi * kEw + qj];
+      double2 x10 = src[qi * kEw + pj], x11 = src[qi * kEw + qj];
+      rot_cols(rj, x00, x01);
+      rot_cols(rj, x10, x11);
+      rot_rows(ri, x00, x10);
+      rot_rows(ri, x01, x11);
+      if (i == j) {
+        x01 = x10 = make_double2(0.0, 0.0);
+        x00.y = x11.y = 0.0;
+      }
+      dst[pi * kEw + pj] = x00;
+      dst[pi * kEw + qj] = x01;
+      dst[qi * kEw + pj] = x10;
+      dst[qi * kEw + qj] = x11;
+    } else if (FULL) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        double2* row = U + (i + kEb * h) * kEw;
+        double2 a = row[pj], b = row[qj];
+        rot_cols(rj, a, b);
+        row[pj] = a;
+        row[qj] = b;
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        rot_cols(rj, ua[h], ub[h]);
+        ub[h] = row_next(ub[h]);
+      }
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    out[0] = so[0];
-    out[1] = sd[0];
+  const double2* last = S[kRounds & 1];
+  double2* out = Uout + (size_t)blockIdx.x * kEw * kEw;
+  for (int e = tid; e < kEw * kEw; e += 512) {
+    const int r = eig_index(P, Q, e / kEw), c = eig_index(P, Q, e % kEw);
+    if (r < n && c < n) A[(size_t)r * n + c] = last[e];
+    if constexpr (FULL) out[e] = U[e];
   }
+  if (!FULL && tid >= 256) {                 // after 16 shifts the columns are home again
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      out[(i + kEb * h) * kEw + j] = ua[h];
+      out[(i + kEb * h) * kEw + kEb + j] = ub[h];
+    }
+  }
+}
+
+// C = X Y (conj-transposed X when XH) for 32 x 32 operands in LDS, this
+// wave's 16 x 16 quadrant (r0, c0) in MFMA layout: lane l holds column l & 15
+// and rows (l >> 4) + 4 i.  xs, ys: row strides.
+template <bool XH>
+__device__ __forceinline__ void quad_product(const double2* X, int xs, const double2* Y, int ys,
+                                             int r0, int c0, f64x4& re, f64x4& im) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  // four accumulators, so that consecutive products do not wait for each other
+  f64x4 r2 = f64x4{0, 0, 0, 0}, i2 = f64x4{0, 0, 0, 0};
+  re = f64x4{0, 0, 0, 0};
+  im = f64x4{0, 0, 0, 0};
+#pragma unroll
+  for (int k0 = 0; k0 < kEw; k0 += 4) {
+    const int k = k0 + lk;
+    double2 a = XH ? X[k * xs + r0 + li] : X[(r0 + li) * xs + k];
+    if (XH) a.y = -a.y;
+    const double2 b = Y[k * ys + c0 + li];
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, im, 0, 0, 0);
+    r2 = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, r2, 0, 0, 0);
+    i2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, i2, 0, 0, 0);
+  }
+  re += r2;
+  im += i2;
+}
+
+// Workgroups [0, h (h - 1) / 2): tiles (I, J), I < J, of A; the rest: V's
+// tiles (32 rows x pair J).  h = pairs.  Every tile is read and written by its
+// own workgroup only.
+constexpr int kXs = kEw + 1;       // row stride of the operand read by rows
+__global__ __launch_bounds__(256) void k_update(double2* __restrict__ A, double2* __restrict__ V,
+                                                int n, int m, int s,
+                                                const double2* __restrict__ Uall,
+                                                const EigState* __restrict__ state) {
+  const int done = state->done;
+  __shared__ double2 X[kEw * kXs];
+  __shared__ double2 UI[kEw * kEw], UJ[kEw * kEw];
+  const int h = m / 2, ntile = h * (h - 1) / 2;
+  const int tid = threadIdx.x;
+  const bool onA = (int)blockIdx.x < ntile;
+  int I = 0, J, row0 = 0;
+  if (onA) {
+    int rem = blockIdx.x;
+    while (rem >= h - 1 - I) {
+      rem -= h - 1 - I;
+      ++I;
+    }
+    J = I + 1 + rem;
+  } else {
+    const int f = (int)blockIdx.x - ntile;
+    J = f % h;
+    row0 = (f / h) * kEw;
+  }
+  int PI = 0, QI = 0, PJ, QJ;
+  if (onA) pair_of(I, s, m, PI, QI);
+  pair_of(J, s, m, PJ, QJ);
+  // every load is issued before the flag is looked at and the first value stored
+  constexpr int kLoads = kEw * kEw / 256;
+  const double2* M = onA ? A : V;
+  double2 x[kLoads], uj[kLoads], ui[kLoads];
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int e = tid + 256 * u;
+    const int lr = e / kEw, lc = e % kEw;
+    const int r = onA ? eig_index(PI, QI, lr) : row0 + lr, c = eig_index(PJ, QJ, lc);
+    x[u] = (r < n && c < n) ? M[(size_t)r * n + c] : make_double2(0.0, 0.0);
+    uj[u] = Uall[(size_t)J * kEw * kEw + e];
+    ui[u] = Uall[(size_t)I * kEw * kEw + e];  // I = 0 for V's tiles: not used there
+  }
+  if (done) return;                          // uniform over the grid
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int e = tid + 256 * u;
+    X[(e / kEw) * kXs + e % kEw] = x[u];
+    UJ[e] = uj[u];
+    UI[e] = ui[u];
+  }
+  __syncthreads();
+  const int wave = tid >> 6, lane = tid & 63;
+  const int r0 = (wave >> 1) * 16, c0 = (wave & 1) * 16, li = lane & 15, lk = lane >> 4;
+  f64x4 re, im;
+  quad_product<false>(X, kXs, UJ, kEw, r0, c0, re, im);
+  if (!onA) {                                // uniform over the workgroup
+    const int c = eig_index(PJ, QJ, c0 + li);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = row0 + r0 + lk + 4 * i;
+      if (r < n && c < n) V[(size_t)r * n + c] = make_double2(re[i], im[i]);
+    }
+    return;
+  }
+  __syncthreads();                           // X is read
+#pragma unroll
+  for (int i = 0; i < 4; ++i) X[(r0 + lk + 4 * i) * kXs + c0 + li] = make_double2(re[i], im[i]);
+  __syncthreads();
+  quad_product<true>(UI, kEw, X, kXs, r0, c0, re, im);
+  const int c = eig_index(PJ, QJ, c0 + li);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = eig_index(PI, QI, r0 + lk + 4 * i);
+    if (r < n && c < n) {
+      A[(size_t)r * n + c] = make_double2(re[i], im[i]);
+      A[(size_t)c * n + r] = make_double2(re[i], -im[i]);
+    }
+  }
+}
+
+// Partial sums of |A_pq|^2 (p != q) and A_pp^2, one pair per workgroup.
+__global__ __launch_bounds__(256) void k_offnorm(const double2* __restrict__ A, int n,
+                                                 double2* __restrict__ part) {
+  __shared__ double2 red[256];
+  double off = 0.0, dg = 0.0;
+  for (int r = blockIdx.x; r < n; r += gridDim.x)
+    for (int c = threadIdx.x; c < n; c += 256) {
+      const double2 v = A[(size_t)r * n + c];
+      const double a2 = v.x * v.x + v.y * v.y;
+      if (r == c)
+        dg += a2;
+      else
+        off += a2;
+    }
+  red[threadIdx.x] = make_double2(off, dg);
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] = zadd(red[threadIdx.x], red[threadIdx.x + w]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+
+// The norms from the partial sums (in a fixed order), and whether they meet
+// the tolerance; otherwise one more sweep begins.
+__global__ void k_offnorm_total(const double2* __restrict__ part, int nparts, double tol,
+                                EigState* __restrict__ state) {
+  const int t = threadIdx.x;                 // one wave, nparts <= 64
+  double2 s = t < nparts ? part[t] : make_double2(0.0, 0.0);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    s = zadd(s, make_double2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
+  if (t != 0) return;
+  state->off = s.x;
+  state->diag = s.y;
+  state->done = !(s.x > tol * tol * s.y);
+  if (!state->done) ++state->sweeps;
 }
 
 __global__ void k_diag(const double2* __restrict__ A, int n, double* __restrict__ w) {
@@ -184,8 +409,8 @@ using namespace oi;
 
 extern "C" size_t oi_eigh_work_bytes(int n) {
   if (n < 1) return 0;
-  const int m = n + (n & 1);
-  return (size_t)(m / 2) * sizeof(Rot) + 2 * sizeof(double);
+  return (size_t)eig_pairs(n) * kEw * kEw * sizeof(double2) + kNormBlocks * sizeof(double2) +
+         sizeof(EigState);
 }
 
 extern "C" int oi_eigh_hermitian(void* A, int n, double* w, void* V, int max_sweeps, double tol,
@@ -195,43 +420,52 @@ extern "C" int oi_eigh_hermitian(void* A, int n, double* w, void* V, int max_swe
   hipStream_t st = (hipStream_t)stream;
   double2* a = static_cast<double2*>(A);
   double2* v = static_cast<double2*>(V);
-  const int m = n + (n & 1);
-  Rot* rot = static_cast<Rot*>(work);
-  double* norms = reinterpret_cast<double*>(static_cast<char*>(work) + (size_t)(m / 2) * sizeof(Rot));
-  hipLaunchKernelGGL(k_eye, dim3(blocks_for((size_t)n * n)), dim3(256), 0, st, v, n);
+  const int h = eig_pairs(n), m = 2 * h;
+  double2* U = static_cast<double2*>(work);
+  double2* part = U + (size_t)h * kEw * kEw;
+  EigState* state = reinterpret_cast<EigState*>(part + kNormBlocks);
+  hipLaunchKernelGGL(k_eye, dim3(blocks_for((size_t)n * n)), dim3(256), 0, st, v, n, state);
   OI_LAUNCH_CHECK("eigh_eye");
-  int sweep = 0;
+  int sweeps = 0;
   if (n > 1) {
-    const int h = m / 2;
-    const int rb = (h + 255) / 256;
-    const int ab = blocks_for((size_t)h * h + (size_t)n * h);
+    const int parts = n < kNormBlocks ? n : kNormBlocks;
+    const int tiles = h * (h - 1) / 2 + ((n + kEw - 1) / kEw) * h;
     // A sweep count that runs out still passes when the off-diagonal norm is
     // at the rounding level of an n x n rotation sequence.
     const double acc = tol > 4.0 * n * DBL_EPSILON ? tol : 4.0 * n * DBL_EPSILON;
-    for (;; ++sweep) {
-      hipLaunchKernelGGL(k_offnorm, dim3(1), dim3(1024), 0, st, a, n, norms);
+    for (int sweep = 0;; ++sweep) {
+      hipLaunchKernelGGL(k_offnorm, dim3(parts), dim3(256), 0, st, a, n, part);
+      hipLaunchKernelGGL(k_offnorm_total, dim3(1), dim3(64), 0, st, part, parts, tol, state);
       OI_LAUNCH_CHECK("eigh_offnorm");
-      double host[2];
-      OI_HIP_CHECK(hipMemcpyAsync(host, norms, sizeof(host), hipMemcpyDeviceToHost, st));
-      OI_HIP_CHECK(hipStreamSynchronize(st));
-      if (!std::isfinite(host[0]) || !std::isfinite(host[1]))
-        return fail(OI_ERR_RUNTIME, "eigh_hermitian: matrix norm is not finite");
-      if (!(host[0] > tol * tol * host[1])) break;
-      if (sweep == max_sweeps) {
-        if (host[0] > acc * acc * host[1])
-          return fail(OI_ERR_RUNTIME, "eigh_hermitian: no convergence in " +
-                                          std::to_string(max_sweeps) + " sweeps");
-        break;
+      // No matrix that has to be decomposed converges in two sweeps, and one
+      // that does skips the rest on the device: the host waits from then on.
+      if (sweep >= 2 || sweep == max_sweeps) {
+        EigState host;
+        OI_HIP_CHECK(hipMemcpyAsync(&host, state, sizeof(host), hipMemcpyDeviceToHost, st));
+        OI_HIP_CHECK(hipStreamSynchronize(st));
+        if (!std::isfinite(host.off) || !std::isfinite(host.diag))
+          return fail(OI_ERR_RUNTIME, "eigh_hermitian: matrix norm is not finite");
+        sweeps = host.done ? host.sweeps : host.sweeps - 1;
+        if (host.done) break;
+        if (sweep == max_sweeps) {
+          if (host.off > acc * acc * host.diag)
+            return fail(OI_ERR_RUNTIME, "eigh_hermitian: no convergence in " +
+                                            std::to_string(max_sweeps) + " sweeps");
+          break;
+        }
       }
       for (int s = 0; s < m - 1; ++s) {
-        hipLaunchKernelGGL(k_rot, dim3(rb), dim3(256), 0, st, a, n, m, s, rot);
-        hipLaunchKernelGGL(k_apply, dim3(ab), dim3(256), 0, st, a, v, n, m, s, rot);
+        if (s == 0)
+          hipLaunchKernelGGL(k_solve<true>, dim3(h), dim3(512), 0, st, a, n, m, s, U, state);
+        else
+          hipLaunchKernelGGL(k_solve<false>, dim3(h), dim3(512), 0, st, a, n, m, s, U, state);
+        hipLaunchKernelGGL(k_update, dim3(tiles), dim3(256), 0, st, a, v, n, m, s, U, state);
       }
       OI_LAUNCH_CHECK("eigh_round");
     }
   }
   hipLaunchKernelGGL(k_diag, dim3((n + 255) / 256), dim3(256), 0, st, a, n, w);
   OI_LAUNCH_CHECK("eigh_diag");
-  if (sweeps_out) *sweeps_out = sweep;
+  if (sweeps_out) *sweeps_out = sweeps;
   return OI_OK;
 }

@@ -301,6 +301,14 @@ size_t oi_eigh_work_bytes(int n);
 int oi_eigh_hermitian(void* A, int n, double* w, void* V, int max_sweeps, double tol,
                       void* work, int* sweeps_out, void* stream);
 
+/* Whether the smallest eigenvalue of the real symmetric G (float64 [n][n],
+ * lower triangle read, overwritten) exceeds rel times its trace: above[0]
+ * (device) = 1 or 0, from a Cholesky factorisation of G - rel trace(G) I.
+ * Exact but for rounding of about n eps trace(G); 0 for a G with values that
+ * are not finite.  work: oi_sym_above_work_bytes(n) bytes. */
+size_t oi_sym_above_work_bytes(int n);
+int oi_sym_above(void* G, int n, double rel, void* work, int* above, void* stream);
+
 /* -------------------------------------------------------------- elementwise
  * Fringe Zernike wavefront W(rho, theta) (Projection.py:13-128, Orientation
  * already applied to coeffs).  rho, theta, out : float32 [n].              */

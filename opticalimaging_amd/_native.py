@@ -96,6 +96,8 @@ SIGNATURES = {
     "oi_eigh_work_bytes": (c_size_t, [c_int]),
     "oi_eigh_hermitian": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_double, c_void_p,
                                   P_int, c_void_p]),
+    "oi_sym_above_work_bytes": (c_size_t, [c_int]),
+    "oi_sym_above": (c_int, [c_void_p, c_int, c_double, c_void_p, c_void_p, c_void_p]),
     "oi_zernike": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p]),
     "oi_char_matrix": (c_int, [c_void_p, c_void_p, c_int, c_double, c_double, c_void_p, c_void_p]),
     "oi_socs_adjoint_work_bytes": (c_size_t, [c_void_p, c_int, c_int]),

@@ -397,6 +397,134 @@ __global__ void k_diag(const double2* __restrict__ A, int n, double* __restrict_
   if (i < n) w[i] = A[(size_t)i * n + i].x;
 }
 
+// ------------------------------------------------ smallest eigenvalue above
+// lambda_min(G) > rel trace(G) for a real symmetric G: G - rel trace(G) I has a
+// Cholesky factor.  32-wide panels, one launch each: with panel k factored
+// (its inverse factor Linv_k kept), tile (I, J), k < J <= I, takes
+// A_IJ -= L_I L_J^T with L_I = A_Ik Linv_k^T formed in place by every tile (no
+// launch between panel and update), and tile (k + 1, k + 1) factors itself.
+// Bound by the 32 dependent pivots of each panel (about 13 us a launch, 0.1 ms
+// at n = 240, where the eigenvalues cost 4.1 ms); the factor is not kept.
+constexpr int kCb = 32, kCs = kCb + 1;
+
+// In LDS: S (lower triangle) is factored, W = the factor's inverse.  False
+// when a pivot is not positive.  Every thread of the 256 calls.
+__device__ bool chol_panel(double* S, double* W, double* rs) {
+  const int tid = threadIdx.x;
+  bool ok = true;
+  for (int e = tid; e < kCb * kCb; e += 256) W[(e / kCb) * kCs + e % kCb] = e / kCb == e % kCb ? 1.0 : 0.0;
+  for (int c = 0; c < kCb; ++c) {
+    __syncthreads();
+    const double piv = S[c * kCs + c];
+    ok = ok && piv > 0.0;                    // uniform over the workgroup (NaN: false)
+    const double inv = ok ? 1.0 / piv : 0.0;
+    if (tid == 0) rs[c] = sqrt(inv);
+    for (int e = tid; e < kCb * kCb; e += 256) {
+      const int i = e / kCb, j = e % kCb;
+      if (i <= c) continue;
+      const double l = S[i * kCs + c] * inv;
+      if (j > c && j <= i) S[i * kCs + j] -= l * S[j * kCs + c];
+      if (j <= c) W[i * kCs + j] -= l * W[c * kCs + j];
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < kCb * kCb; e += 256) W[(e / kCb) * kCs + e % kCb] *= rs[e / kCb];
+  __syncthreads();
+  return ok;
+}
+
+// shift[0] = rel trace(G); ok[0] = 1.
+__global__ __launch_bounds__(256) void k_chol_begin(const double* __restrict__ G, int n, double rel,
+                                                    double* __restrict__ shift, int* __restrict__ ok) {
+  __shared__ double red[256];
+  double t = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) t += G[(size_t)i * n + i];
+  red[threadIdx.x] = t;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    shift[0] = rel * red[0];
+    ok[0] = 1;
+  }
+}
+
+// k = -1: tile (0, 0) alone is factored.
+__global__ __launch_bounds__(256) void k_chol_panel(double* __restrict__ G, int n, int k,
+                                                    const double* __restrict__ shift,
+                                                    double* __restrict__ Linv, int* __restrict__ ok) {
+  __shared__ double S[kCb * kCs], W[kCb * kCs], LI[kCb * kCs], LJ[kCb * kCs], rs[kCb];
+  // Workgroup 0 (tile (k + 1, k + 1)) may clear the flag while others of this
+  // launch start: one thread reads it, so that a workgroup decides as one, and
+  // what is then computed or not is not used by any later launch.
+  __shared__ int go;
+  if (threadIdx.x == 0) go = ok[0];
+  __syncthreads();
+  if (!go) return;
+  int I = k + 1, J = k + 1, rem = blockIdx.x;
+  while (rem > I - (k + 1)) {                // pairs J <= I row by row
+    rem -= I - k;
+    ++I;
+  }
+  J = k + 1 + rem;
+  const int tid = threadIdx.x;
+  auto at = [&](int r, int c) -> double {
+    return r < n && c < n ? G[(size_t)r * n + c] : (r == c ? 1.0 : 0.0);   // past n: identity
+  };
+  if (k >= 0) {
+    for (int e = tid; e < kCb * kCb; e += 256) {
+      const int r = e / kCb, c = e % kCb;
+      LI[r * kCs + c] = at(I * kCb + r, k * kCb + c);
+      LJ[r * kCs + c] = at(J * kCb + r, k * kCb + c);
+      W[r * kCs + c] = Linv[(size_t)k * kCb * kCb + e];
+    }
+    __syncthreads();
+    // rows of the panel times Linv^T, one output column per pass and thread
+    double li[4], lj[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + 256 * u, r = e / kCb, c = e % kCb;
+      double a = 0.0, b = 0.0;
+      for (int t = 0; t <= c; ++t) {
+        a = fma(LI[r * kCs + t], W[c * kCs + t], a);
+        b = fma(LJ[r * kCs + t], W[c * kCs + t], b);
+      }
+      li[u] = a;
+      lj[u] = b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + 256 * u, r = e / kCb, c = e % kCb;
+      LI[r * kCs + c] = li[u];
+      LJ[r * kCs + c] = lj[u];
+    }
+    __syncthreads();
+  }
+  const bool diag = I == k + 1 && J == k + 1;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = tid + 256 * u, r = e / kCb, c = e % kCb;
+    double v = at(I * kCb + r, J * kCb + c);
+    // the shift enters each diagonal element once, before its first update
+    if (k <= 0 && I == J && r == c && I * kCb + r < n && (k < 0 || I > 0)) v -= shift[0];
+    if (k >= 0)
+      for (int t = 0; t < kCb; ++t) v = fma(-LI[r * kCs + t], LJ[c * kCs + t], v);
+    if (diag)
+      S[r * kCs + c] = v;
+    else if (I * kCb + r < n && J * kCb + c < n)
+      G[(size_t)(I * kCb + r) * n + J * kCb + c] = v;
+  }
+  if (!diag) return;                         // uniform over the workgroup
+  __syncthreads();
+  const bool good = chol_panel(S, W, rs);
+  if (!good && tid == 0) ok[0] = 0;
+  for (int e = tid; e < kCb * kCb; e += 256)
+    Linv[(size_t)(k + 1) * kCb * kCb + e] = W[(e / kCb) * kCs + e % kCb];
+}
+
 static int blocks_for(size_t total) {
   size_t b = (total + 255) / 256;
   if (b > 4096) b = 4096;
@@ -467,5 +595,27 @@ extern "C" int oi_eigh_hermitian(void* A, int n, double* w, void* V, int max_swe
   hipLaunchKernelGGL(k_diag, dim3((n + 255) / 256), dim3(256), 0, st, a, n, w);
   OI_LAUNCH_CHECK("eigh_diag");
   if (sweeps_out) *sweeps_out = sweeps;
+  return OI_OK;
+}
+
+extern "C" size_t oi_sym_above_work_bytes(int n) {
+  if (n < 1) return 0;
+  return (size_t)((n + kCb - 1) / kCb) * kCb * kCb * sizeof(double) + sizeof(double);
+}
+
+extern "C" int oi_sym_above(void* G, int n, double rel, void* work, int* above, void* stream) {
+  if (!G || !work || !above || n < 1) return fail(OI_ERR_INVALID, "sym_above: bad arguments");
+  hipStream_t st = (hipStream_t)stream;
+  double* g = static_cast<double*>(G);
+  const int nb = (n + kCb - 1) / kCb;
+  double* Linv = static_cast<double*>(work);
+  double* shift = Linv + (size_t)nb * kCb * kCb;
+  hipLaunchKernelGGL(k_chol_begin, dim3(1), dim3(256), 0, st, g, n, rel, shift, above);
+  for (int k = -1; k < nb - 1; ++k) {
+    const int left = nb - 1 - k;             // tile rows past panel k
+    const int tiles = k < 0 ? 1 : left * (left + 1) / 2;
+    hipLaunchKernelGGL(k_chol_panel, dim3(tiles), dim3(256), 0, st, g, n, k, shift, Linv, above);
+  }
+  OI_LAUNCH_CHECK("sym_above");
   return OI_OK;
 }

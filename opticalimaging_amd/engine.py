@@ -180,6 +180,18 @@ def kernel_set_of(kernels) -> "KernelSet":
     return KernelSet.from_dense(torch.as_tensor(kernels))
 
 
+def _sym_above(G: torch.Tensor, rel: float) -> bool:
+    """Whether the smallest eigenvalue of the real symmetric float64 G exceeds
+    rel times its trace (oi_sym_above)."""
+    n = int(G.shape[0])
+    lib = nat.load()
+    work = torch.empty(int(lib.oi_sym_above_work_bytes(n)), dtype=torch.uint8, device=G.device)
+    above = torch.empty(1, dtype=torch.int32, device=G.device)
+    g = G.to(torch.float64).contiguous().clone()
+    nat.check(lib.oi_sym_above(nat.ptr(g), n, float(rel), nat.ptr(work), nat.ptr(above), nat.stream()))
+    return bool(above.item())
+
+
 PAIR_MAX_K = 512        # larger sets are imaged as they are (the 2K x 2K eigenproblem grows)
 
 
@@ -217,6 +229,12 @@ def real_mask_kernels(ks: KernelSet, rel_tol: float = 1e-10) -> KernelSet:
     X = torch.cat([(phi + jphi) * 0.5, (phi - jphi) * (-0.5j)], 0)
     G = (X.conj() @ X.transpose(0, 1)).real
     G = 0.5 * (G + G.transpose(0, 1))
+    # r >= 2K - 1 (nothing to gain) follows when every eigenvalue exceeds half
+    # the part of the trace that may be dropped: a Cholesky factorisation shows
+    # it in 0.2 ms at K = 120 where the eigenvalues take 4 (2 % above the half,
+    # far more than its rounding of 2K eps)
+    if _sym_above(G, 0.51 * rel_tol):
+        return ks
     lam, Q = eigen_desc(G.to(torch.complex128))
     if float(Q.imag.abs().max()) > 1e-9:
         return ks

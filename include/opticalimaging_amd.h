@@ -94,7 +94,8 @@ typedef struct oi_geometry {
   int rows;
   int direct;
   int qr, qc;
-  int path;       /* 0: generic kernels; 1: compile-time-size kernels, one
+  int path;       /* 0: generic kernels, or (image lengths without
+                   * compile-time transforms) matrix products; 1: compile-time-size kernels, one
                      pass over the coarse grid; 2: compile-time-size kernels,
                      two-pass coherent sum (coarse 144, 256 or 512)          */
   int max_kernels;

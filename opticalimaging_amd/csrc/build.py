@@ -22,7 +22,7 @@ LIB_NAME = "libopticalimaging_amd.so"
 LIB_PATH = os.path.join(PKG, LIB_NAME)
 ARCH = os.environ.get("OI_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["oi_api.hip", "oi_imaging.hip", "oi_fastpath.hip", "oi_pupil.hip", "oi_tcc.hip",
+SOURCES = ["oi_api.hip", "oi_imaging.hip", "oi_fastpath.hip", "oi_dft.hip", "oi_pupil.hip", "oi_tcc.hip",
            "oi_eigh.hip", "oi_adjoint.hip", "oi_ilt.hip", "oi_rcwa.hip"]
 
 COMMON_FLAGS = [

@@ -1,6 +1,7 @@
 // Adjoint (mask gradient) of the SOCS image: internal interface.
 #pragma once
 
+#include "oi_dft.h"
 #include "oi_internal.h"
 
 namespace oi {
@@ -11,6 +12,7 @@ struct AdjGeom {
   int lr, lc, qr, qc;
   int direct;
   FftDesc fx, fy, flr, flc;
+  DftTable tab_x, tab_y;
 };
 
 size_t adjoint_work_bytes(const AdjGeom& g, int batch, int nkern);

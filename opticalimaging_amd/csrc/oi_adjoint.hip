@@ -565,6 +565,11 @@ static int adj_half(int k0, int w) {
   return a > b ? a : b;
 }
 
+// both image lengths have a fast transform: in registers or as a product
+static bool adj_image_ok(const AdjGeom& g) {
+  return (fp_image_size_ok(g.ny) || g.tab_y.fcos) && (fp_image_size_ok(g.nx) || g.tab_x.fcos);
+}
+
 size_t adjoint_work_bytes(const AdjGeom& g, int batch, int nkern) {
   const size_t B = (size_t)batch, K = (size_t)nkern;
   const size_t gq = g.direct ? 0 : (size_t)(2 * g.qr + 1) * (2 * g.qc + 1);
@@ -601,8 +606,8 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
   if (g.direct) return fail(OI_ERR_INVALID, "adjoint: no band spectrum on a direct plan");
   const int wgc = 2 * g.qc + 1, wgr = 2 * g.qr + 1;
   float2* Tg = static_cast<float2*>(work);     // the first region of the work buffer
-  if (fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx)) {
-    // register transforms of the image sizes (same spectrum, scale and layout)
+  if (adj_image_ok(g)) {
+    // the fast path's transforms of the image sizes (same spectrum, scale and layout)
     FpArgs a{};
     a.field = img;
     a.kind = OI_FIELD_REAL;
@@ -618,6 +623,8 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
     a.wc = wgc;
     a.tw_x = g.fx.tw;
     a.tw_y = g.fy.tw;
+    a.tab_x = g.tab_x;
+    a.tab_y = g.tab_y;
     a.T = Tg;
     a.spec = out;
     return fp_spectrum(a, st);
@@ -631,8 +638,7 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
 
 bool adjoint_chain_ok(const AdjGeom& g) {
   const int qrm = adj_half(g.k0r, g.wr), qcm = adj_half(g.k0c, g.wc);
-  return fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx) && 2 * qrm + 1 <= g.ny &&
-         2 * qcm + 1 <= g.nx;
+  return adj_image_ok(g) && 2 * qrm + 1 <= g.ny && 2 * qcm + 1 <= g.nx;
 }
 
 int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int batch,
@@ -744,6 +750,8 @@ int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int ba
     a.qc = qcm;
     a.tw_x = g.fx.tw;
     a.tw_y = g.fy.tw;
+    a.tab_x = g.tab_x;
+    a.tab_y = g.tab_y;
     a.Ihat = F;
     a.U = U;
     a.out = grad;

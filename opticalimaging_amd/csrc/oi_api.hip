@@ -110,6 +110,8 @@ struct oi_plan {
   float2* Ihat = nullptr;
   float* part = nullptr;    // residual sums of the image-row pass, [B][ny]
   float2* Bbuf = nullptr;   // two-pass column fields of max_batch x max_kernels kernels
+  float* dft = nullptr;     // product tables of the image lengths (dft_bytes)
+  DftTable tab_x, tab_y;
   size_t bytes = 0;
   std::vector<hipEvent_t> ev;  // slots * (kStages + 1)
   int slots = 0, next = 0, recorded = 0;
@@ -134,15 +136,21 @@ static void plan_free(oi_plan* p) {
   if (!p) return;
   for (hipEvent_t e : p->ev) (void)hipEventDestroy(e);
   for (void* ptr : {(void*)p->T, (void*)p->spec, (void*)p->R, (void*)p->U, (void*)p->Ic,
-                    (void*)p->Ihat, (void*)p->part, (void*)p->Bbuf})
+                    (void*)p->Ihat, (void*)p->part, (void*)p->Bbuf, (void*)p->dft})
     if (ptr) (void)hipFree(ptr);
   free_twiddles(p->pool);
   delete p;
 }
 
+static bool image_lengths_tabled(const oi_geometry& g) {
+  return fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx);
+}
+
 // Validates a geometry and fills the library-chosen fields (coarse grid,
-// path, rows, kernel groups, band half-widths); allocates nothing.
-static int plan_geometry(const oi_geometry& in, oi_geometry& g) {
+// path, rows, kernel groups, band half-widths); allocates nothing.  generic:
+// image lengths without register transforms take the generic kernels
+// throughout (no product tables).
+static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = false) {
   g = in;
   if (g.ny <= 0 || g.nx <= 0 || g.wr <= 0 || g.wc <= 0 || g.nchan <= 0 || g.nchan > 3 ||
       g.max_batch <= 0)
@@ -178,10 +186,13 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g) {
   g.lc = lc;
   g.qr = g.direct ? 0 : band_r - 1;
   g.qc = g.direct ? 0 : band_c - 1;
-  // Compile-time-size path: both image sizes tabled and a tabled square coarse
-  // grid L >= 2 band - 1 in both directions, smaller than the image.
+  // Compile-time-size path: a tabled square coarse grid L >= 2 band - 1 in both
+  // directions, smaller than the image (any image size: lengths without a
+  // register transform take matrix products).
   g.path = 0;
-  if (!g.direct && in.lr <= 0 && in.lc <= 0 && fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx)) {
+  const bool fast = !g.direct && in.lr <= 0 && in.lc <= 0 &&
+                    (!generic || image_lengths_tabled(g));
+  if (fast) {
     const int need = (2 * band_r - 1) > (2 * band_c - 1) ? 2 * band_r - 1 : 2 * band_c - 1;
     const int L = fp_coarse_choose(need);
     if (L > 0 && L < g.ny && L < g.nx && fp_coherent_rows_fit(L) &&
@@ -193,7 +204,7 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g) {
   }
   // Two-pass path: coarse grids beyond one workgroup's reach (L = 256, 512)
   // when the window folds onto them without collisions.
-  if (g.path == 0 && !g.direct && in.lr <= 0 && in.lc <= 0) {
+  if (g.path == 0 && fast) {
     const int need = (2 * band_r - 1) > (2 * band_c - 1) ? 2 * band_r - 1 : 2 * band_c - 1;
     // coarse grids past one workgroup's reach, and those the one-pass kernel
     // does not serve when the two-pass table has them (144)
@@ -264,6 +275,30 @@ static ScratchLayout scratch_layout(const oi_geometry& g, size_t B) {
   return s;
 }
 
+// Bytes of the product tables of a geometry's image lengths (0 where the length
+// has a register transform), and their orders: every order that a transform of
+// that length meets (window and image band).
+static int half_width(int k0, int w) { return -k0 > k0 + w - 1 ? -k0 : k0 + w - 1; }
+
+static size_t dft_bytes(const oi_geometry& g, bool cols) {
+  if (!g.path || fp_image_size_ok(cols ? g.ny : g.nx)) return 0;
+  const int h = cols ? half_width(g.k0r, g.wr) : half_width(g.k0c, g.wc);
+  const int q = cols ? g.qr : g.qc;
+  return dft_table_bytes(cols ? g.ny : g.nx, h > q ? h : q);
+}
+
+// Builds the plan's tables in p->dft (of dft_bytes of both lengths).
+static int dft_build(oi_plan* p, hipStream_t st) {
+  const oi_geometry& g = p->g;
+  const size_t bx = dft_bytes(g, false), by = dft_bytes(g, true);
+  const int hx = half_width(g.k0c, g.wc), hy = half_width(g.k0r, g.wr);
+  int rc = OI_OK;
+  if (bx) rc = dft_table_build(p->fx.tw, g.nx, hx > g.qc ? hx : g.qc, p->dft, p->tab_x, st);
+  if (!rc && by)
+    rc = dft_table_build(p->fy.tw, g.ny, hy > g.qr ? hy : g.qr, p->dft + bx / sizeof(float), p->tab_y, st);
+  return rc;
+}
+
 extern "C" int oi_plan_create(oi_geometry* geo, oi_plan** out) {
   if (!geo || !out) return fail(OI_ERR_INVALID, "plan_create: null argument");
   *out = nullptr;
@@ -294,6 +329,7 @@ extern "C" int oi_plan_create(oi_geometry* geo, oi_plan** out) {
       {(void**)&p->T, sl.T},       {(void**)&p->spec, sl.spec}, {(void**)&p->R, sl.R},
       {(void**)&p->U, sl.U},       {(void**)&p->Ic, sl.Ic},     {(void**)&p->Ihat, sl.Ihat},
       {(void**)&p->part, sl.part}, {(void**)&p->Bbuf, sl.Bbuf},
+      {(void**)&p->dft, dft_bytes(g, false) + dft_bytes(g, true)},
   };
   p->bytes = p->pool.bytes;
   for (auto& w : want) {
@@ -304,7 +340,17 @@ extern "C" int oi_plan_create(oi_geometry* geo, oi_plan** out) {
     }
     p->bytes += w.bytes;
   }
+  rc = dft_build(p, nullptr);
+  if (!rc && p->dft && hipStreamSynchronize(nullptr) != hipSuccess)   // read from any stream
+    rc = fail(OI_ERR_RUNTIME, "plan_create: table set-up failed");
+  if (rc) {
+    plan_free(p);
+    return rc;
+  }
   *geo = g;
+  // a one-pass coarse grid behind matrix products is reported as generic: it has
+  // no compile-time image transforms and none of their fused passes
+  if (g.path == 1 && !image_lengths_tabled(g)) geo->path = 0;
   *out = p;
   return OI_OK;
 }
@@ -363,6 +409,8 @@ static FpArgs fast_args(oi_plan* p, int batch, hipStream_t st) {
   a.tw_x = p->fx.tw;
   a.tw_y = p->fy.tw;
   a.tw_l = p->flr.tw;
+  a.tab_x = p->tab_x;
+  a.tab_y = p->tab_y;
   a.T = p->T;
   a.spec = p->spec;
   a.R = p->R;
@@ -437,7 +485,7 @@ static int spectrum_impl(oi_plan* p, const void* field, int kind, int cin, const
   int rc;
   const oi_geometry& g = p->g;
   mark(p, 0, st);
-  if (g.path == 1 || (g.path == 2 && fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx))) {
+  if (g.path) {
     FpArgs a = fast_args(p, batch, st);
     a.field = field;
     a.kind = kind;
@@ -470,8 +518,7 @@ extern "C" int oi_coherent_image(oi_plan* p, const void* spec, int batch, const 
 // writes 2 (I - target) and its partial sums).
 static bool residual_fused(const oi_plan* p) {
   const oi_geometry& g = p->g;
-  return (g.path == 1 || g.path == 2) && fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx) &&
-         fp_urows_blocks(g.ny, g.nx, 1) <= g.ny;
+  return g.path && image_lengths_tabled(g) && fp_urows_blocks(g.ny, g.nx, 1) <= g.ny;
 }
 
 // target non-null: out = 2 (I - target), partial sums of (I - target)^2 in p->part.
@@ -504,37 +551,17 @@ static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* ke
     c.wr = g.wr;
     c.k0c = g.k0c;
     c.wc = g.wc;
-    const bool fast_io = fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx);
     const int nkc = nkern * g.nchan;
-    c.groups = fast_io ? (groups < nkc ? groups : nkc) : 1;
+    c.groups = groups < nkc ? groups : nkc;
     c.qc = g.qc;
     c.tw_l = p->flr.tw;
     c.tw_m = p->flr.tw;
     c.R = p->R;
-    int rc = fp_two_pass(a, c, p->Bbuf, fast_io ? 0 : 1, st);
+    int rc = fp_two_pass(a, c, p->Bbuf, st);
     if (rc) return rc;
     if (band_only) return fp_band(a, c.groups, st);
     mark(p, 3, st);
-    if (fast_io) {
-      rc = fp_interp(a, c.groups, st);
-    } else {
-      InterpArgs ia{};
-      ia.R = p->R;
-      ia.groups = 1;
-      ia.lr = g.lr;
-      ia.lc = g.lc;
-      ia.ny = g.ny;
-      ia.nx = g.nx;
-      ia.qr = g.qr;
-      ia.qc = g.qc;
-      ia.scale = 1.0f / ((float)g.lr * (float)g.lc);
-      ia.flr = p->flr;
-      ia.fny = p->fy;
-      ia.fnx = p->fx;
-      ia.U = p->U;
-      ia.out = out;
-      rc = launch_interp(ia, batch, st, mark_cb, &g_mark_ctx);
-    }
+    rc = fp_interp(a, c.groups, st);
     mark_done(p);
     return rc;
   }
@@ -725,6 +752,8 @@ static AdjGeom adj_geom(const oi_plan* p) {
   a.fy = p->fy;
   a.flr = p->flr;
   a.flc = p->flc;
+  a.tab_x = p->tab_x;
+  a.tab_y = p->tab_y;
   return a;
 }
 
@@ -941,6 +970,15 @@ static size_t aligned_total(const ScratchLayout& s) {
          align_up(s.Ihat) + align_up(s.part) + align_up(s.Bbuf);
 }
 
+// Scratch of one image with its tables, at most (twiddle tables counted once
+// per transform length, shared or not).
+static size_t noalloc_bytes(const oi_geometry& g) {
+  const size_t tw = align_up(2 * (size_t)g.nx * sizeof(float2)) + align_up(2 * (size_t)g.ny * sizeof(float2)) +
+                    align_up(2 * (size_t)g.lr * sizeof(float2)) + align_up(2 * (size_t)g.lc * sizeof(float2)) +
+                    align_up(2 * (size_t)g.rows * sizeof(float2));
+  return tw + align_up(dft_bytes(g, false) + dft_bytes(g, true)) + aligned_total(scratch_layout(g, 1));
+}
+
 extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, int kind, int cin,
                                      const int* chans, int batch, const void* kern, int nkern,
                                      float* out, void* stream) {
@@ -955,6 +993,10 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   oi_geometry g;
   int rc = plan_geometry(in, g);
   if (rc) return rc;
+  // the tables and buffers of image lengths without a register transform may
+  // not fit beside one image: those sizes then take the generic kernels, whose
+  // scratch is smaller
+  if (noalloc_bytes(g) > kNoAllocScratch && (rc = plan_geometry(in, g, true))) return rc;
   // twiddle tables first, one per distinct length
   const int sizes[5] = {g.nx, g.ny, g.lr, g.lc, g.rows};
   FftDesc d[5];
@@ -969,6 +1011,8 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
       if (sizes[j] == sizes[i]) tw_off[i] = tw_off[j];
     if (tw_off[i] == used) used += align_up(2 * (size_t)sizes[i] * sizeof(float2));
   }
+  const size_t dft_off = used;
+  used += align_up(dft_bytes(g, false) + dft_bytes(g, true));
   const size_t per_image = aligned_total(scratch_layout(g, 1));
   if (used + per_image > kNoAllocScratch)
     return fail(OI_ERR_INVALID, "socs_image_noalloc: one image needs " +
@@ -1002,6 +1046,8 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   pl.flr = d[2];
   pl.flc = d[3];
   pl.frows = d[4];
+  pl.dft = reinterpret_cast<float*>(base + dft_off);
+  if ((rc = dft_build(&pl, st))) return rc;
   const ScratchLayout sl = scratch_layout(pl.g, (size_t)chunk);
   unsigned char* cur = base + used;
   auto carve = [&cur](size_t bytes) -> unsigned char* {

@@ -1,6 +1,7 @@
 // Fast-path (compile-time transform sizes) imaging launches.
 #pragma once
 
+#include "oi_dft.h"
 #include "oi_internal.h"
 
 namespace oi {
@@ -30,6 +31,7 @@ struct FpArgs {
   const float2* tw_x;  // exp(-2 pi i m / nx)
   const float2* tw_y;  // exp(-2 pi i m / ny)
   const float2* tw_l;  // exp(-2 pi i m / L)
+  DftTable tab_x, tab_y;  // product tables of the lengths without register transforms
   float2* T;      // [B][C][wc][ny]
   float2* spec;   // [B][C][wr][wc]
   float2* R;      // [B][G][L][qc+1]
@@ -56,7 +58,7 @@ struct FpCoh {
   float2* R;
 };
 
-bool fp_image_size_ok(int n);
+bool fp_image_size_ok(int n);            // n has a register transform
 bool fp_coarse_size_ok(int l);
 // Radices (R1, R2) of the two-stage register transform of length n, false
 // when n has none.  Twiddle tables of length n carry 2n entries: [0, n) holds
@@ -102,11 +104,10 @@ size_t ilt_target_const_scratch(int batch);
 int ilt_target_const(const float* target, size_t npix, const float2* tband, size_t nband,
                      int batch, void* scratch, float* tconst, hipStream_t st);
 // Two-pass coherent sum for coarse grids L in {256, 512}: B holds
-// batch * nkern * nchan * wc * L c64; R in [img][q][t] (generic_layout = 0) or
-// [img][t][q] (1).
+// batch * nkern * nchan * wc * L c64; R in [img][group][q][t].
 bool fp_two_pass_size_ok(int l);
 int fp_two_pass_choose(int need);
 size_t fp_two_pass_lds(int L, int wc);
-int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, int generic_layout, hipStream_t st);
+int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st);
 
 }  // namespace oi

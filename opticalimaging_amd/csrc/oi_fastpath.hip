@@ -1,7 +1,8 @@
 // Imaging kernels with compile-time transform sizes (register FFTs, one LDS
 // exchange per transform).  Same mathematics and data flow as the generic
-// kernels of oi_imaging.hip; used when the image sizes and the coarse grid are
-// in the size tables below.
+// kernels of oi_imaging.hip; used when the coarse grid is in the size tables
+// below.  Image lengths outside the table take the matrix products of
+// oi_dft.hip for their four stages.
 //
 //   k_fp_rows_real<P>   mask rows -> T[img][j][r] = sum_m h[r][m] e^{+2 pi i (k0c+j) m / nx}
 //   k_fp_rows_c64<P>    same for one channel of a complex channels-last field
@@ -677,8 +678,7 @@ __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ 
 }
 
 // Blocks (row group, img, grp) sum the (kernel, channel) pairs kc = grp,
-// grp + groups, ... into their own partial R[img][grp] (groups = 1 for the
-// generic layout).
+// grp + groups, ... into their own partial R[img][grp].
 // Four waves per SIMD (at most 128 registers) up to coarse 256: four
 // workgroups then share a CU, as their 34 KB of LDS allow (ILT step 0.355 ->
 // 0.348 ms).  From 450 on the LDS (about 70 KB) holds two workgroups per CU
@@ -691,7 +691,7 @@ constexpr int brows_min_blocks() {
 
 template <class PL>
 __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(const float2* __restrict__ B, int nkc, int k0c,
-                                                     int wc, int qc, int generic_layout,
+                                                     int wc, int qc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ R, int batch,
                                                      int groups) {
@@ -751,8 +751,7 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
   for (int m = 0; m < VL; ++m) {
     const int x = t + TL * m;
     if (x > qc) continue;
-    if (generic_layout) R[((size_t)img * L + row) * nq + x] = v[m];   // [img][t][q] (one group)
-    else R[(((size_t)img * groups + grp) * nq + x) * L + row] = v[m];  // [img][grp][q][t]
+    R[(((size_t)img * groups + grp) * nq + x) * L + row] = v[m];  // [img][grp][q][t]
   }
 }
 
@@ -1256,8 +1255,7 @@ static size_t two_pass_rows_lds(int wc) {
 }
 
 template <class PL>
-static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, int generic_layout,
-                        hipStream_t st) {
+static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st) {
   constexpr int G = groups_per_block<PL>();
   const size_t lds1 = rows_lds<PL>();
   int rc = allow(k_fp_bcols<PL>, lds1);
@@ -1269,10 +1267,9 @@ static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, int generic_
   const size_t lds2 = two_pass_rows_lds<PL>(a.wc);
   rc = allow(k_fp_brows<PL>, lds2);
   if (rc) return rc;
-  if (generic_layout && c.groups != 1) return fail(OI_ERR_INVALID, "two-pass path: one group in the generic layout");
   const int items = ((PL::N + G - 1) / G) * a.batch * c.groups;
   hipLaunchKernelGGL(k_fp_brows<PL>, dim3(xcd_grid(items)), dim3(kBlock), lds2, st, B,
-                     c.nkern * c.nchan, a.k0c, a.wc, a.qc, generic_layout, a.tw_l, c.R, a.batch,
+                     c.nkern * c.nchan, a.k0c, a.wc, a.qc, a.tw_l, c.R, a.batch,
                      c.groups);
   OI_LAUNCH_CHECK("fp_brows");
   return OI_OK;
@@ -1303,9 +1300,9 @@ size_t fp_two_pass_lds(int L, int wc) {
   return (size_t)-1;
 }
 
-int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, int generic_layout, hipStream_t st) {
+int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st) {
   int rc = OI_ERR_UNSUPPORTED;
-#define X(NN, A, B_) if (a.L == NN) rc = fp::run_two_pass<reg::GFFT<NN, A, B_>>(a, c, B, generic_layout, st);
+#define X(NN, A, B_) if (a.L == NN) rc = fp::run_two_pass<reg::GFFT<NN, A, B_>>(a, c, B, st);
   OI_TWO_PASS_PLANS(X)
 #undef X
   if (rc == OI_ERR_UNSUPPORTED) return fail(rc, "two-pass path: unsupported coarse size");
@@ -1327,19 +1324,42 @@ int fp_band(const FpArgs& a, int groups, hipStream_t st) {
   return OI_OK;
 }
 
+// A stage of an image size: the register transform where the length has one,
+// else the matrix product of its table.
+#define OI_IMAGE_STAGE(n, table, reg_run, product)                                         \
+  int rc = OI_ERR_UNSUPPORTED;                                                              \
+  if (table.fcos) return product(a, st);                                                     \
+  OI_IMAGE_PLANS(reg_run)                                                                   \
+  return rc == OI_ERR_UNSUPPORTED ? fail(rc, "image length without a transform") : rc;
+
+static int stage_rows(const FpArgs& a, hipStream_t st) {
+#define X(NN, PT) if (a.nx == NN) rc = fp::run_rows<fp::PT>(a, st);
+  OI_IMAGE_STAGE(a.nx, a.tab_x, X, dft_rows)
+#undef X
+}
+static int stage_cols(const FpArgs& a, hipStream_t st) {
+#define X(NN, PT) if (a.ny == NN) rc = fp::run_cols<fp::PT>(a, st);
+  OI_IMAGE_STAGE(a.ny, a.tab_y, X, dft_cols)
+#undef X
+}
+static int stage_ucols(const FpArgs& a, hipStream_t st) {
+#define X(NN, PT) if (a.ny == NN) rc = fp::run_ucols<fp::PT>(a, st);
+  OI_IMAGE_STAGE(a.ny, a.tab_y, X, dft_ucols)
+#undef X
+}
+static int stage_urows(const FpArgs& a, hipStream_t st) {
+#define X(NN, PT) if (a.nx == NN) rc = fp::run_urows<fp::PT>(a, st);
+  OI_IMAGE_STAGE(a.nx, a.tab_x, X, dft_urows)
+#undef X
+}
+
 int fp_interp(const FpArgs& a, int groups, hipStream_t st) {
   int rc = fp_band(a, groups, st);
   if (rc) return rc;
-  rc = OI_ERR_UNSUPPORTED;
-#define X(NN, PT) if (a.ny == NN) rc = fp::run_ucols<fp::PT>(a, st);
-  OI_IMAGE_PLANS(X)
-#undef X
+  rc = stage_ucols(a, st);
   if (rc) return rc;
   if (a.mark) a.mark(a.mark_ctx, 4);
-  rc = OI_ERR_UNSUPPORTED;
-#define X(NN, PT) if (a.nx == NN) rc = fp::run_urows<fp::PT>(a, st);
-  OI_IMAGE_PLANS(X)
-#undef X
+  rc = stage_urows(a, st);
   if (rc) return rc;
   if (a.mark) a.mark(a.mark_ctx, 5);
   return OI_OK;
@@ -1347,17 +1367,8 @@ int fp_interp(const FpArgs& a, int groups, hipStream_t st) {
 // The image from a band Ihat[img][q][2qr+1] (q in [0, qc]), without the
 // band kernel: the interpolation column and row transforms only.
 int fp_band_image(const FpArgs& a, hipStream_t st) {
-  int rc = OI_ERR_UNSUPPORTED;
-#define X(NN, PT) if (a.ny == NN) rc = fp::run_ucols<fp::PT>(a, st);
-  OI_IMAGE_PLANS(X)
-#undef X
-  if (rc) return rc == OI_ERR_UNSUPPORTED ? fail(rc, "fast path: unsupported ny") : rc;
-  rc = OI_ERR_UNSUPPORTED;
-#define X(NN, PT) if (a.nx == NN) rc = fp::run_urows<fp::PT>(a, st);
-  OI_IMAGE_PLANS(X)
-#undef X
-  if (rc) return rc == OI_ERR_UNSUPPORTED ? fail(rc, "fast path: unsupported nx") : rc;
-  return OI_OK;
+  int rc = stage_ucols(a, st);
+  return rc ? rc : stage_urows(a, st);
 }
 
 int fp_urows_sets(int ny, int nx, int batch) {
@@ -1465,18 +1476,10 @@ int fp_coherent_rows_fit(int L) {
 }
 
 int fp_spectrum(const FpArgs& a, hipStream_t st) {
-  int rc = OI_ERR_UNSUPPORTED;
-#define X(NN, PT) if (a.nx == NN) rc = fp::run_rows<fp::PT>(a, st);
-  OI_IMAGE_PLANS(X)
-#undef X
-  if (rc) return rc == OI_ERR_UNSUPPORTED ? fail(rc, "fast path: unsupported nx") : rc;
+  int rc = stage_rows(a, st);
+  if (rc) return rc;
   if (a.mark) a.mark(a.mark_ctx, 1);
-  rc = OI_ERR_UNSUPPORTED;
-#define X(NN, PT) if (a.ny == NN) rc = fp::run_cols<fp::PT>(a, st);
-  OI_IMAGE_PLANS(X)
-#undef X
-  if (rc) return rc == OI_ERR_UNSUPPORTED ? fail(rc, "fast path: unsupported ny") : rc;
-  return OI_OK;
+  return stage_cols(a, st);
 }
 
 static int fp_coherent(const FpArgs& a, const FpCoh& c, hipStream_t st) {

@@ -152,6 +152,17 @@ int oi_spectrum_window(oi_plan* plan, const void* field, int kind, int cin,
 int oi_coherent_image(oi_plan* plan, const void* spec, int batch,
                       const void* kern, int nkern, float* out, void* stream);
 
+/* Images of one spectrum under nsets kernel sets: out[s] is what
+ * oi_coherent_image gives for (spec, kern[s]), up to the summation order of the
+ * kernel groups, which is the plan's.  A one-pass plan (compile-time coarse grid
+ * of one workgroup) takes max_batch sets per launch chain, any other one set.
+ * The foci of CalculateAbbeImage (CalculateAerialImage.py:46-92) are such sets.
+ *   spec : c64 [nchan][wr][wc]
+ *   kern : c64 [nsets][nkern][wr][wc]
+ *   out  : float32 [nsets][ny][nx]                                            */
+int oi_coherent_sets(oi_plan* plan, const void* spec, int nsets, const void* kern,
+                     int nkern, float* out, void* stream);
+
 /* oi_spectrum_window followed by oi_coherent_image; spec lives in the plan.
  * Replaces CalculateAerialImage_SOCS (CalculateAerialImage_SOCS.py:3-11) for a
  * batch of masks.                                                            */

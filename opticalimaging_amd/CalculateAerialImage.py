@@ -5,8 +5,9 @@
 component e is one coherent kernel sqrt(n V_s / W) P_se(kappa) on the
 spectrum window (``oi_pupil_kernels``, float64, rho^2 <= 1 decided in
 float64); the image is the coherent sum over kernels and field channels
-(``oi_coherent_image``), evaluated on a coarse grid sized by one shifted
-pupil (2 floor(2 p) + 1) and Fourier-interpolated exactly to the image grid.
+(``oi_coherent_sets``, the foci in one launch chain), evaluated on a coarse
+grid sized by one shifted pupil (2 floor(2 p) + 1) and Fourier-interpolated
+exactly to the image grid.
 
 ``CalculateHopkinsImage``: per focus, TCC -> SOCS kernels -> SOCS image
 (CalculateAerialImage.py:105-130).
@@ -54,8 +55,18 @@ def abbe_images(field, source, scatter, projector, numerics, encoding=None) -> t
     k0r, wr, k0c, wc, br, bc = optics.abbe_window(src, py, px, ny, nx)
     tens, kind, cin, live = encoding if encoding is not None else engine.field_encoding(h)
     ncomp = 3 if vector else 1
+    foci = optics.focus_values(projector)
+    # One-pass coarse grids (2 band - 1 <= 128) image up to 16 foci per launch
+    # chain: 512^2, 196 points x 3 components, 5 foci: coherent sum 80 -> 47 us,
+    # band, columns and rows 90 -> 17 us.  Where 512 workgroups still have four
+    # kernels each, that many (two per CU) hide more latency than their partial
+    # sums cost: 47 us against 54 with 256.
+    need = 2 * max(br, bc) - 1
+    batch = max(1, min(len(foci), 16)) if need <= 128 and need < min(ny, nx) else 1
+    nk = ncomp * src.n
+    groups = -(-512 // batch) if batch > 1 and nk * batch >= 4 * 512 else 0
     plan = engine.PLANS.get(ny=ny, nx=nx, k0r=k0r, wr=wr, k0c=k0c, wc=wc, nchan=len(live),
-                            max_batch=1, band_r=br, band_c=bc, max_kernels=ncomp * src.n)
+                            max_batch=batch, max_groups=groups, band_r=br, band_c=bc, max_kernels=nk)
     lib = nat.load()
     spec = torch.empty((1, len(live), wr, wc), dtype=torch.complex64, device=dev)
     cptr, keep = nat.int_array(live)
@@ -63,18 +74,15 @@ def abbe_images(field, source, scatter, projector, numerics, encoding=None) -> t
                                      nat.stream()))
     del keep
     scale = src.kernel_scale(projector.IndexImage)
-    foci = optics.focus_values(projector)
     out = torch.empty((len(foci), ny, nx), dtype=torch.float32, device=dev)
     opt = optics.optics_record(source, projector, 0.0, py, px, vector)
     # every focus's kernels from one pass, in slices of at most 1 GiB
-    per_focus = ncomp * src.n * wr * wc * 8
+    per_focus = nk * wr * wc * 8
     step = max(1, min(len(foci), (1 << 30) // max(per_focus, 1)))
     for i0 in range(0, len(foci), step):
         G = optics.pupil_kernels_foci(src, opt, foci[i0:i0 + step], scale, k0r, wr, k0c, wc)
-        for k in range(G.shape[0]):
-            nat.check(lib.oi_coherent_image(plan.handle, nat.ptr(spec), 1, nat.ptr(G[k]),
-                                            G.shape[1] * G.shape[2], nat.ptr(out[i0 + k]),
-                                            nat.stream()))
+        nat.check(lib.oi_coherent_sets(plan.handle, nat.ptr(spec), G.shape[0], nat.ptr(G), nk,
+                                       nat.ptr(out[i0]), nat.stream()))
     return out
 
 

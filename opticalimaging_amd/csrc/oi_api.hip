@@ -507,11 +507,32 @@ static int spectrum_impl(oi_plan* p, const void* field, int kind, int cin, const
 }
 
 static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* kern, int nkern,
-                         float* out, const float* target, hipStream_t st, bool band_only = false);
+                         float* out, const float* target, hipStream_t st, bool band_only = false,
+                         bool sets = false);
 
 extern "C" int oi_coherent_image(oi_plan* p, const void* spec, int batch, const void* kern,
                                  int nkern, float* out, void* stream) {
   return coherent_impl(p, spec, batch, kern, nkern, out, nullptr, (hipStream_t)stream);
+}
+
+// One-pass plans take max_batch sets a launch chain: a chain of one image leaves
+// its three interpolation launches and the last kernels of the sum with most
+// of the chip idle.  Others take the sets one by one: their launches are larger,
+// and a two-pass plan would need the column fields of every set at once.
+extern "C" int oi_coherent_sets(oi_plan* p, const void* spec, int nsets, const void* kern,
+                                int nkern, float* out, void* stream) {
+  if (!p || !kern || !out) return fail(OI_ERR_INVALID, "coherent_sets: null argument");
+  if (nsets < 1) return fail(OI_ERR_INVALID, "coherent_sets: nsets must be >= 1");
+  const oi_geometry& g = p->g;
+  const int step = g.path == 1 ? g.max_batch : 1;
+  for (int s = 0; s < nsets; s += step) {
+    const int n = nsets - s < step ? nsets - s : step;
+    const int rc = coherent_impl(p, spec, n, static_cast<const float2*>(kern) + (size_t)s * nkern * g.wr * g.wc,
+                                 nkern, out + (size_t)s * g.ny * g.nx, nullptr, (hipStream_t)stream, false,
+                                 true);
+    if (rc) return rc;
+  }
+  return OI_OK;
 }
 
 // The residual form needs the compile-time-size image kernels (their row pass
@@ -523,8 +544,10 @@ static bool residual_fused(const oi_plan* p) {
 
 // target non-null: out = 2 (I - target), partial sums of (I - target)^2 in p->part.
 // band_only (plans with the residual pass): the band p->Ihat of the image, no image.
+// sets (one image, or a one-pass plan): the images share one spectrum and have
+// nkern kernels each.
 static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* kern, int nkern,
-                         float* out, const float* target, hipStream_t st, bool band_only) {
+                         float* out, const float* target, hipStream_t st, bool band_only, bool sets) {
   if (!p || !spec || !kern || (!out && !band_only))
     return fail(OI_ERR_INVALID, "coherent_image: null argument");
   if ((target || band_only) && !residual_fused(p))
@@ -573,6 +596,8 @@ static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* ke
     FpCoh c{};
     c.spec = static_cast<const float2*>(spec);
     c.kern = static_cast<const float2*>(kern);
+    c.spec_img = sets ? 0 : (size_t)g.nchan * g.wr * g.wc;
+    c.kern_img = sets ? (size_t)nkern * g.wr * g.wc : 0;
     c.nchan = g.nchan;
     c.nkern = nkern;
     c.k0r = g.k0r;

@@ -47,8 +47,9 @@ struct FpArgs {
 };
 
 struct FpCoh {
-  const float2* spec;
-  const float2* kern;
+  const float2* spec;   // image i's spectra start at spec + i spec_img, its kernels at
+  const float2* kern;   // kern + i kern_img (one-pass sums; 0: shared by the images)
+  size_t spec_img, kern_img;
   int nchan, nkern;
   int k0r, wr, k0c, wc;
   int groups;

@@ -407,6 +407,7 @@ __global__ __launch_bounds__(kBlock) void k_fp_coherent(FpCoh A) {
   float2* Bb = specL + wr * wc;
   float2* scr = Bb + M * wc;
   const int s = blockIdx.x, img = blockIdx.y, grp = blockIdx.z;
+  const float2* kern = A.kern + img * A.kern_img;
   const int tid = threadIdx.x;
 
   // row-stage geometry
@@ -429,12 +430,12 @@ __global__ __launch_bounds__(kBlock) void k_fp_coherent(FpCoh A) {
     for (int m = 0; m < VL; ++m) acc[q][m] = 0.f;
 
   for (int c = 0; c < A.nchan; ++c) {
-    const float2* sp = A.spec + ((size_t)img * A.nchan + c) * wr * wc;
+    const float2* sp = A.spec + img * A.spec_img + (size_t)c * wr * wc;
     __syncthreads();
     for (int e = tid; e < wr * wc; e += kBlock) specL[e] = sp[e];
     __syncthreads();
     for (int kk = grp; kk < A.nkern; kk += A.groups) {
-      const float2* kp = A.kern + (size_t)kk * wr * wc;
+      const float2* kp = kern + (size_t)kk * wr * wc;
       // column stage: column kc handled by group gm (round-robin); M-point
       // transform of the kr fold (kr mod M) twisted by exp(-2 pi i kr s / L)
       for (int c0 = 0; c0 < wc; c0 += GM) {
@@ -547,6 +548,7 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
   const int wr = A.wr, wc = A.wc;
   float2* specL = lds + L * S;
   const int img = blockIdx.x, grp = blockIdx.y;
+  const float2* kern = A.kern + img * A.kern_img;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int gw = lane / TL, t = lane - gw * TL;
   const int g = wave * GW + gw;
@@ -576,13 +578,13 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
   for (int m = 0; m < VL; ++m) acc[m] = 0.f;
 
   for (int c = 0; c < A.nchan; ++c) {
-    const float2* sp = A.spec + ((size_t)img * A.nchan + c) * wr * wc;
+    const float2* sp = A.spec + img * A.spec_img + (size_t)c * wr * wc;
     __syncthreads();
     for (int e = threadIdx.x; e < wr * wc; e += NT) specL[e] = sp[e];
     // this thread's kernel values of the first kernel
     float2 nxt[VL];
     {
-      const float2* kp = A.kern + (size_t)grp * wr * wc;
+      const float2* kp = kern + (size_t)grp * wr * wc;
 #pragma unroll
       for (int m = 0; m < VL; ++m) {
         int kr = kr0 + TL * m;
@@ -601,7 +603,7 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
       }
       // next kernel's values, in flight during this kernel's transforms
       const int kn = kk + A.groups;
-      const float2* kp = A.kern + (size_t)(kn < A.nkern ? kn : kk) * wr * wc;
+      const float2* kp = kern + (size_t)(kn < A.nkern ? kn : kk) * wr * wc;
 #pragma unroll
       for (int m = 0; m < VL; ++m) {
         int kr = kr0 + TL * m;

@@ -152,6 +152,20 @@ int oi_spectrum_window(oi_plan* plan, const void* field, int kind, int cin,
 int oi_coherent_image(oi_plan* plan, const void* spec, int batch,
                       const void* kern, int nkern, float* out, void* stream);
 
+/* PupilImage of Scatter.CalculateSpectrum (Scatter.py:25-35) from a windowed
+ * spectrum: out[i][j][c], c < cin, is Hk at row index i - oy and column index
+ * j - ox,
+ *   px py exp(-2 pi i (kr (ny/2)/ny + kc (nx/2)/nx)) spec[n](kr, kc)
+ * for c = chans[n], 0 for a channel that no n names, and NaN outside the unit
+ * circle (kr/py)^2 + (kc/px)^2 > 1, decided in float32 as the reference does.
+ * The window must hold [-oy, oy) x [-ox, ox).
+ *   spec  : c64 [nchan][wr][wc]
+ *   chans : host array [nchan], entries in [0, cin), nchan <= 3
+ *   out   : c64 [2 oy][2 ox][cin]                                             */
+int oi_pupil_crop(const void* spec, int nchan, int k0r, int wr, int k0c, int wc,
+                  const int* chans, int cin, int ny, int nx, double px, double py,
+                  int oy, int ox, void* out, void* stream);
+
 /* Images of one spectrum under nsets kernel sets: out[s] is what
  * oi_coherent_image gives for (spec, kern[s]), up to the summation order of the
  * kernel groups, which is the plan's.  A one-pass plan (compile-time coarse grid

@@ -46,6 +46,11 @@ def cartesian_to_polar(x, y):
 def abbe_images(field, source, scatter, projector, numerics, encoding=None) -> torch.Tensor:
     """Abbe intensities (nFocus, Ny, Nx) float32 on the device.  ``encoding``
     is engine.field_encoding(field) when the caller already has it."""
+    return _abbe_images(field, source, scatter, projector, numerics, encoding)[0]
+
+
+def _abbe_images(field, source, scatter, projector, numerics, encoding):
+    """abbe_images and the field's windowed spectrum as pupil_image takes it."""
     vector = optics.imaging_mode(numerics)
     dev = nat.device()
     h = torch.as_tensor(field)
@@ -68,7 +73,7 @@ def abbe_images(field, source, scatter, projector, numerics, encoding=None) -> t
     plan = engine.PLANS.get(ny=ny, nx=nx, k0r=k0r, wr=wr, k0c=k0c, wc=wc, nchan=len(live),
                             max_batch=batch, max_groups=groups, band_r=br, band_c=bc, max_kernels=nk)
     lib = nat.load()
-    spec = torch.empty((1, len(live), wr, wc), dtype=torch.complex64, device=dev)
+    spec = torch.empty((len(live), wr, wc), dtype=torch.complex64, device=dev)
     cptr, keep = nat.int_array(live)
     nat.check(lib.oi_spectrum_window(plan.handle, nat.ptr(tens), kind, cin, cptr, 1, nat.ptr(spec),
                                      nat.stream()))
@@ -83,7 +88,7 @@ def abbe_images(field, source, scatter, projector, numerics, encoding=None) -> t
         G = optics.pupil_kernels_foci(src, opt, foci[i0:i0 + step], scale, k0r, wr, k0c, wc)
         nat.check(lib.oi_coherent_sets(plan.handle, nat.ptr(spec), G.shape[0], nat.ptr(G), nk,
                                        nat.ptr(out[i0]), nat.stream()))
-    return out
+    return out, (spec, k0r, k0c)
 
 
 def _image_axes(scatter, nx, ny, projector):
@@ -100,9 +105,9 @@ def CalculateAbbeImage(source, scatter, projector, numerics):
     h = torch.as_tensor(scatter.ScatterField)
     ny, nx = int(h.shape[0]), int(h.shape[1])
     enc = engine.field_encoding(h)          # one device-to-host transfer per call
-    intensity = abbe_images(h, source, scatter, projector, numerics, encoding=enc)
+    intensity, spectrum = _abbe_images(h, source, scatter, projector, numerics, enc)
     px, py = _pitches(scatter, projector, source)
-    pupil = pupil_image(h, px, py, encoding=enc)
+    pupil = pupil_image(h, px, py, encoding=enc, spectrum=spectrum)
     d = _image_axes(scatter, nx, ny, projector)
     d.Intensity = intensity.to(h.device)
     return d, pupil.to(h.device)

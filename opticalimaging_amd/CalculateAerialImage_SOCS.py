@@ -31,6 +31,24 @@ def socs_field_image(field, ks: engine.KernelSet) -> torch.Tensor:
     return engine.socs_image(tens, ks, kind=kind, cin=cin, chans=live)[0]
 
 
+def _image_and_spectrum(enc, ks: engine.KernelSet):
+    """socs_field_image of an encoded field by its two calls, with the windowed
+    spectrum between them as pupil_image takes it."""
+    tens, kind, cin, live = enc
+    if kind == nat.OI_FIELD_REAL:
+        ks = ks.for_real_masks()
+    lib, plan = nat.load(), engine.plan_for(ks, len(live), 1)
+    spec = torch.empty((len(live), ks.wr, ks.wc), dtype=torch.complex64, device=tens.device)
+    out = torch.empty((ks.ny, ks.nx), dtype=torch.float32, device=tens.device)
+    cptr, keep = nat.int_array(live)
+    nat.check(lib.oi_spectrum_window(plan.handle, nat.ptr(tens), kind, cin, cptr, 1, nat.ptr(spec),
+                                     nat.stream()))
+    del keep
+    nat.check(lib.oi_coherent_image(plan.handle, nat.ptr(spec), 1, nat.ptr(ks.win), ks.K, nat.ptr(out),
+                                    nat.stream()))
+    return out, (spec, ks.k0r, ks.k0c)
+
+
 def CalculateAerialImage_SOCS(scatter, TCCMatrix_SOCS, source, projector):
     """Returns (intensity (Ny, Nx) float32, PupilImage), on the ScatterField's
     device."""
@@ -39,9 +57,10 @@ def CalculateAerialImage_SOCS(scatter, TCCMatrix_SOCS, source, projector):
     ks = kernel_set_of(TCCMatrix_SOCS)
     if tuple(h.shape[:2]) != (ks.ny, ks.nx):
         raise ValueError("ScatterField grid does not match the SOCS kernel grid")
-    intensity = socs_field_image(h, ks)
+    enc = engine.field_encoding(h)
+    intensity, spectrum = _image_and_spectrum(enc, ks)
     px, py = _pitches(scatter, projector, source)
-    pupil = pupil_image(h, px, py)
+    pupil = pupil_image(h, px, py, encoding=enc, spectrum=spectrum)
     return intensity.to(out_dev), pupil.to(out_dev)
 
 

@@ -2,9 +2,7 @@
 ``Scatter`` (Scatter.py:3-8).  ``CalculateSpectrum`` runs on the HIP device."""
 from __future__ import annotations
 
-import collections
 import ctypes
-import threading
 
 import torch
 
@@ -44,46 +42,16 @@ def full_spectrum(field: torch.Tensor, px: float, py: float) -> torch.Tensor:
     return hk
 
 
-# Per-grid constants of the windowed pupil image (the fftshift phase of the
-# crop and its unit-circle mask), kept on the device for the last few grids so
-# that a repeated call launches no table set-up and copies nothing to the
-# device.  The cached tensors are read, never written in place.
-_PUPIL_TABLES = collections.OrderedDict()
-_PUPIL_TABLES_SIZE = 16
-_PUPIL_LOCK = threading.Lock()
-
-
-def _pupil_tables(ny, nx, px, py, dev):
-    key = (ny, nx, float(px), float(py), dev.index)
-    with _PUPIL_LOCK:
-        hit = _PUPIL_TABLES.get(key)
-        if hit is not None:
-            _PUPIL_TABLES.move_to_end(key)
-            return hit
-    ox, oy = int(px) + 3, int(py) + 3
-    f, g = frequency_axes(nx, ny, px, py)
-    kr = torch.arange(-oy, oy, device=dev, dtype=torch.float64)
-    kc = torch.arange(-ox, ox, device=dev, dtype=torch.float64)
-    # exp(-2 pi i kappa (N//2)/N): the fftshift phase of Scatter.py:22
-    ph = torch.exp(-2j * torch.pi * (kr[:, None] * (ny // 2) / ny + kc[None, :] * (nx // 2) / nx))
-    gm, fm = torch.meshgrid(g[ny // 2 - oy: ny // 2 + oy].to(dev),
-                            f[nx // 2 - ox: nx // 2 + ox].to(dev), indexing="ij")
-    entry = (ph, (gm ** 2 + fm ** 2) > 1)
-    with _PUPIL_LOCK:
-        _PUPIL_TABLES[key] = entry
-        while len(_PUPIL_TABLES) > _PUPIL_TABLES_SIZE:
-            _PUPIL_TABLES.popitem(last=False)
-    return entry
-
-
 def pupil_image(field: torch.Tensor, px: float, py: float, hk: torch.Tensor | None = None,
-                encoding=None):
+                encoding=None, spectrum=None):
     """PupilImage of Scatter.CalculateSpectrum (Scatter.py:25-35): Hk with NaN
     outside the unit circle, cropped to +-(int(p)+3) samples about the centre.
 
-    When the crop lies inside the grid it is evaluated from the windowed
-    spectrum alone (a pruned transform); otherwise from the full spectrum with
-    the reference's slicing."""
+    When the crop lies inside the grid it is evaluated from a windowed spectrum
+    (a pruned transform): ``spectrum`` = (spec [C][wr][wc], k0r, k0c), the live
+    channels' window that the image was made from, where the crop lies inside
+    it, else one of the crop's own; otherwise from the full spectrum with the
+    reference's slicing."""
     dev = nat.device()
     h = torch.as_tensor(field).to(dev)
     ny, nx, cin = h.shape
@@ -92,20 +60,27 @@ def pupil_image(field: torch.Tensor, px: float, py: float, hk: torch.Tensor | No
     if inside and hk is None:
         enc = encoding if encoding is not None else engine.field_encoding(h)
         tens, kind, cin_, live = enc
-        plan = engine.PLANS.get(ny=ny, nx=nx, k0r=-oy, wr=2 * oy, k0c=-ox, wc=2 * ox,
-                                nchan=len(live), max_batch=1, max_kernels=1)
-        spec = torch.empty((1, len(live), 2 * oy, 2 * ox), dtype=torch.complex64, device=dev)
-        cptr, keep = nat.int_array(live)
-        nat.check(nat.load().oi_spectrum_window(plan.handle, nat.ptr(tens), kind, cin_, cptr, 1,
-                                                nat.ptr(spec), nat.stream()))
+        if spectrum is not None:
+            spec, k0r, k0c = spectrum
+            wr, wc = spec.shape[-2:]
+            if k0r > -oy or k0r + wr < oy or k0c > -ox or k0c + wc < ox:
+                spectrum = None
+        if spectrum is None:
+            k0r, wr, k0c, wc = -oy, 2 * oy, -ox, 2 * ox
+            plan = engine.PLANS.get(ny=ny, nx=nx, k0r=k0r, wr=wr, k0c=k0c, wc=wc, nchan=len(live),
+                                    max_batch=1, max_kernels=1)
+            spec = torch.empty((len(live), wr, wc), dtype=torch.complex64, device=dev)
+            cptr, keep = nat.int_array(live)
+            nat.check(nat.load().oi_spectrum_window(plan.handle, nat.ptr(tens), kind, cin_, cptr, 1,
+                                                    nat.ptr(spec), nat.stream()))
+            del keep
+        win = torch.empty((2 * oy, 2 * ox, cin), dtype=torch.complex64, device=dev)
+        cptr, keep = nat.int_array(enc.source_channels)
+        nat.check(nat.load().oi_pupil_crop(nat.ptr(spec), len(live), k0r, wr, k0c, wc, cptr, cin, ny,
+                                           nx, float(px), float(py), oy, ox, nat.ptr(win),
+                                           nat.stream()))
         del keep
-        # Hk = px py exp(-2 pi i kappa (N//2)/N) spec
-        ph, outside = _pupil_tables(ny, nx, px, py, dev)
-        win = torch.zeros((2 * oy, 2 * ox, cin), dtype=torch.complex64, device=dev)
-        vals = (spec[0].to(torch.complex128) * ph[None] * (px * py)).to(torch.complex64)
-        for i, c in enumerate(enc.source_channels):
-            win[:, :, c] = vals[i]
-        return win.masked_fill_(outside[..., None], float("nan"))   # no host round trip
+        return win
     f, g = frequency_axes(nx, ny, px, py)
     if hk is None:
         hk = full_spectrum(h, px, py)

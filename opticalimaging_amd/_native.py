@@ -84,6 +84,8 @@ SIGNATURES = {
                                     c_void_p, c_void_p]),
     "oi_pupil_kernels": (c_int, [ctypes.POINTER(Optics), c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
+    "oi_pupil_crop": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, P_int, c_int, c_int, c_int,
+                              c_double, c_double, c_int, c_int, c_void_p, c_void_p]),
     "oi_coherent_sets": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p]),
     "oi_pupil_kernels_foci": (c_int, [ctypes.POINTER(Optics), ctypes.POINTER(ctypes.c_double), c_int,
                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,

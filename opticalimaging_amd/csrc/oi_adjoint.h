@@ -29,7 +29,7 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
 
 // grad[b] = d/d mask[b] of sum_j gI[b][j] I[b][j], I the SOCS image of the real
 // masks whose windowed spectrum is spec (c64 [batch][wr][wc]).  bcols (or
-// null): the two-pass column buffer [batch][nkern][wc][lr] that the forward
+// null): the two-pass column buffer [batch][nkern][lr][wc] that the forward
 // pass of the same masks and kernels left (k_fp_bcols); when given on a
 // square register-size coarse grid, the adjoint reads its column stage from
 // there instead of recomputing it (same values).

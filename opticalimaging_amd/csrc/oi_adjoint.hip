@@ -169,18 +169,33 @@ __global__ __launch_bounds__(kThreads) void k_adj_cwin(const float2* __restrict_
 // the coarse grid without collisions (wr <= lr, wc <= lc).
 constexpr int kRegBlock = 256;
 
+// Column kernels: consecutive lanes hold consecutive window columns, so that
+// every load and store is a run of G columns (k_adj_cwin_reg for 16 images x 12
+// kernels at L = 256: 19.8 -> 17.0 us).  Row kernels: 64 / T rows per wavefront,
+// the exchange within the wave, no workgroup barrier (35.8 -> 26.2 us against a
+// pass that staged the rows of a column-major buffer through the LDS).
+template <class P>
+constexpr int cols_per_block() {
+  return kRegBlock / P::T;
+}
+template <class P>
+constexpr int rows_per_block() {
+  return (kRegBlock / 64) * (64 / P::T);
+}
+
 template <class P>
 __global__ __launch_bounds__(kRegBlock) void k_adj_cfield_reg(const float2* __restrict__ spec,
                                                               const float2* __restrict__ kern,
                                                               int nk, int k0r, int wr, int wc,
                                                               const float2* __restrict__ twt,
                                                               float2* __restrict__ Ec) {
-  constexpr int L = P::N, T = P::T, V = P::V, G = kRegBlock / T;
+  constexpr int L = P::N, T = P::T, V = P::V, G = cols_per_block<P>();
   extern __shared__ float2 lds[];
-  const int g = threadIdx.x / T, t = threadIdx.x - g * T;
+  const int g = threadIdx.x % G, tg = threadIdx.x / G;
   const int k = blockIdx.y, b = blockIdx.z;
   const int kc = blockIdx.x * G + g;
-  const bool on = g < G && kc < wc;
+  const bool on = tg < T && kc < wc;
+  const int t = tg < T ? tg : 0;
   const float2* sb = spec + (size_t)b * wr * wc + (on ? kc : 0);
   const float2* kb = kern ? kern + (size_t)k * wr * wc + (on ? kc : 0) : nullptr;
   float2 v[V];
@@ -196,34 +211,41 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cfield_reg(const float2* __re
     }
     v[m] = a;
   }
-  P::template run_live_tab<false>(v, lds + (g < G ? g : 0) * P::LDS, t, twt, g < G);
+  P::template run_live_tab<false>(v, lds + g * (P::LDS | 1), t, twt, on);
   if (!on) return;
   float2* out = Ec + ((size_t)b * nk + k) * L * wc + kc;
 #pragma unroll
   for (int m = 0; m < V; ++m) out[(size_t)(t + T * m) * wc] = v[m];
 }
 
+// Src: the column stage, Ec itself (in place) or the forward pass's two-pass
+// buffer (k_fp_bcols: the same values in the same layout).
 template <class P>
-__global__ __launch_bounds__(kRegBlock) void k_adj_rfield_reg(float2* __restrict__ Ec, int nk,
+__global__ __launch_bounds__(kRegBlock) void k_adj_rfield_reg(const float2* Src, float2* Ec, int nk,
                                                               int k0c, int wc, int lr,
                                                               const float2* __restrict__ twt,
                                                               const float* __restrict__ gamma_in,
                                                               float* __restrict__ gamma_out) {
-  constexpr int L = P::N, T = P::T, V = P::V, G = kRegBlock / T;
+  constexpr int L = P::N, T = P::T, V = P::V, GW = 64 / T;
   extern __shared__ float2 lds[];
-  const int g = threadIdx.x / T, t = threadIdx.x - g * T;
+  const int lane = threadIdx.x & 63, gw = lane / T;
+  const int t = gw < GW ? lane - gw * T : 0;
+  const int g = (threadIdx.x >> 6) * GW + (gw < GW ? gw : 0);
   const int k = blockIdx.y, b = blockIdx.z;
-  const int r = blockIdx.x * G + g;
-  const bool on = g < G && r < lr;
-  float2* scr = lds + (g < G ? g : 0) * P::LDS;
-  float2* row = Ec + (((size_t)b * nk + k) * lr + (on ? r : 0)) * wc;
+  const int r = blockIdx.x * rows_per_block<P>() + g;
+  const bool on = gw < GW && r < lr;
+  float2* scr = lds + g * P::LDS;
+  const size_t at = (((size_t)b * nk + k) * lr + (on ? r : 0)) * wc;
+  const float2* src = Src + at;
+  const int c0 = pmod(t - k0c, L);                    // T m < L: kc = c0 + T m, less L once
   float2 v[V];
 #pragma unroll
   for (int m = 0; m < V; ++m) {
-    const int kc = pmod(t + T * m - k0c, L);
-    v[m] = (on && kc < wc) ? row[kc] : make_float2(0.f, 0.f);
+    int kc = c0 + T * m;
+    kc = kc >= L ? kc - L : kc;
+    v[m] = (on && kc < wc) ? src[kc] : make_float2(0.f, 0.f);
   }
-  P::template run_live_tab<false>(v, scr, t, twt, g < G);
+  P::template run_live_tab_wave<false>(v, scr, t, twt, on);
   if (!gamma_in) {
     if (on) {
       float* go = gamma_out + ((size_t)b * lr + r) * L;
@@ -238,66 +260,13 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_rfield_reg(float2* __restrict
     const float gm = on ? gi[t + T * m] : 0.f;
     v[m] = make_float2(gm * v[m].x, -gm * v[m].y);
   }
-  P::template run_live_tab<false>(v, scr, t, twt, g < G);
+  P::template run_live_tab_wave<false>(v, scr, t, twt, on);
   if (!on) return;
+  float2* row = Ec + at;
 #pragma unroll
   for (int m = 0; m < V; ++m) {
-    const int kc = pmod(t + T * m - k0c, L);
-    if (kc < wc) row[kc] = v[m];
-  }
-}
-
-// k_adj_rfield_reg (with gamma) taking the column stage from the forward
-// pass's two-pass buffer Bc[b][k][kc][t] (k_fp_bcols: the same values as
-// k_adj_cfield_reg's Ec, column-major) instead of recomputing it.  A block
-// stages rows r0 .. r0 + G - 1 of every window column through LDS (one
-// contiguous run of G values per column), runs the row stage and writes the
-// result to Ec[b][k][r][kc] as k_adj_rfield_reg does.  The staging tile and
-// the transform scratch share the LDS (the larger of the two).
-template <class P>
-__global__ __launch_bounds__(kRegBlock) void k_adj_rfield_bcols(const float2* __restrict__ Bc,
-                                                                float2* __restrict__ Ec, int nk,
-                                                                int k0c, int wc, int lr,
-                                                                const float2* __restrict__ twt,
-                                                                const float* __restrict__ gamma_in) {
-  constexpr int L = P::N, T = P::T, V = P::V, G = kRegBlock / T;
-  constexpr int TS = G + 1;
-  extern __shared__ float2 lds[];
-  float2* tile = lds;                              // [wc][TS], then the scratch over it
-  float2* scr = lds;
-  const int g = threadIdx.x / T, t = threadIdx.x - g * T;
-  const int gg = g < G ? g : 0;
-  const int k = blockIdx.y, b = blockIdx.z;
-  const int r0 = blockIdx.x * G;
-  const int r = r0 + gg;
-  const bool on = g < G && r < lr;
-  const float2* src = Bc + ((size_t)b * nk + k) * wc * lr + r0;
-  for (int e = threadIdx.x; e < wc * G; e += kRegBlock) {
-    const int kc = e / G, rr = e - kc * G;
-    tile[kc * TS + rr] = r0 + rr < lr ? src[(size_t)kc * lr + rr] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();
-  float2 v[V];
-#pragma unroll
-  for (int m = 0; m < V; ++m) {
-    const int kc = pmod(t + T * m - k0c, L);
-    v[m] = (on && kc < wc) ? tile[kc * TS + gg] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();                                 // the tile is read: the scratch reuses it
-  float2* sg = scr + (size_t)gg * P::LDS;
-  P::template run_live_tab<false>(v, sg, t, twt, g < G);
-  const float* gi = gamma_in + ((size_t)b * lr + (on ? r : 0)) * L;
-#pragma unroll
-  for (int m = 0; m < V; ++m) {
-    const float gm = on ? gi[t + T * m] : 0.f;
-    v[m] = make_float2(gm * v[m].x, -gm * v[m].y);
-  }
-  P::template run_live_tab<false>(v, sg, t, twt, g < G);
-  if (!on) return;
-  float2* row = Ec + (((size_t)b * nk + k) * lr + r) * wc;
-#pragma unroll
-  for (int m = 0; m < V; ++m) {
-    const int kc = pmod(t + T * m - k0c, L);
+    int kc = c0 + T * m;
+    kc = kc >= L ? kc - L : kc;
     if (kc < wc) row[kc] = v[m];
   }
 }
@@ -308,7 +277,7 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cwin_reg(const float2* __rest
                                                             int k0r, int wr, int wc,
                                                             const float2* __restrict__ twt,
                                                             float2* __restrict__ Ak, int batch) {
-  constexpr int L = P::N, T = P::T, V = P::V, G = kRegBlock / T;
+  constexpr int L = P::N, T = P::T, V = P::V, G = cols_per_block<P>();
   extern __shared__ float2 lds[];
   // items (column block, kernel, image), column blocks fastest, in XCD order:
   // a row of Pc is split over the column blocks of one (image, kernel), and
@@ -317,14 +286,15 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cwin_reg(const float2* __rest
   int w;
   if (!xcd_item(blockIdx.x, nxb * nk * batch, w)) return;   // uniform over the block
   const int xb = w % nxb, k = (w / nxb) % nk, b = w / (nxb * nk);
-  const int g = threadIdx.x / T, t = threadIdx.x - g * T;
+  const int g = threadIdx.x % G, tg = threadIdx.x / G;
   const int kc = xb * G + g;
-  const bool on = g < G && kc < wc;
+  const bool on = tg < T && kc < wc;
+  const int t = tg < T ? tg : 0;
   const float2* pb = Pc + ((size_t)b * nk + k) * L * wc + (on ? kc : 0);
   float2 v[V];
 #pragma unroll
   for (int m = 0; m < V; ++m) v[m] = on ? pb[(size_t)(t + T * m) * wc] : make_float2(0.f, 0.f);
-  P::template run_live_tab<false>(v, lds + (g < G ? g : 0) * P::LDS, t, twt, g < G);
+  P::template run_live_tab<false>(v, lds + g * (P::LDS | 1), t, twt, on);
   if (!on) return;
   const float2* kb = kern + (size_t)k * wr * wc + kc;
   float2* out = Ak + ((size_t)b * nk + k) * wr * wc + kc;
@@ -350,8 +320,12 @@ static bool adj_reg_size(int L) {
 }
 
 template <class P>
-static size_t adj_reg_lds() {
-  return (size_t)(kRegBlock / P::T) * P::LDS * sizeof(float2);
+static size_t adj_cols_lds() {
+  return (size_t)cols_per_block<P>() * (P::LDS | 1) * sizeof(float2);
+}
+template <class P>
+static size_t adj_rows_lds() {
+  return (size_t)rows_per_block<P>() * P::LDS * sizeof(float2);
 }
 
 // Column stage (kern == nullptr: gamma's spectrum) with register transforms.
@@ -360,11 +334,11 @@ static int adj_cfield_reg(int L, dim3 grid_y_z, const float2* spec, const float2
 #define X(NN, A, B)                                                                            \
   if (L == NN) {                                                                               \
     using P = reg::GFFT<NN, A, B>;                                                             \
-    constexpr int G = kRegBlock / P::T;                                                        \
-    int rc = allow_lds_adj(k_adj_cfield_reg<P>, adj_reg_lds<P>());                             \
+    constexpr int G = cols_per_block<P>();                                                     \
+    int rc = allow_lds_adj(k_adj_cfield_reg<P>, adj_cols_lds<P>());                             \
     if (rc) return rc;                                                                         \
     dim3 grid((wc + G - 1) / G, grid_y_z.y, grid_y_z.z);                                       \
-    hipLaunchKernelGGL(k_adj_cfield_reg<P>, grid, dim3(kRegBlock), adj_reg_lds<P>(), st, spec, \
+    hipLaunchKernelGGL(k_adj_cfield_reg<P>, grid, dim3(kRegBlock), adj_cols_lds<P>(), st, spec, \
                        kern, nk, k0r, wr, wc, twt, Ec);                                        \
     OI_LAUNCH_CHECK("adj_cfield_reg");                                                         \
     return OI_OK;                                                                              \
@@ -374,18 +348,18 @@ static int adj_cfield_reg(int L, dim3 grid_y_z, const float2* spec, const float2
   return fail(OI_ERR_UNSUPPORTED, "adjoint: no register transform for this coarse size");
 }
 
-static int adj_rfield_reg(int L, dim3 grid_y_z, float2* Ec, int nk, int k0c, int wc, int lr,
-                          const float2* twt, const float* gamma_in, float* gamma_out,
-                          hipStream_t st) {
+static int adj_rfield_reg(int L, dim3 grid_y_z, const float2* src, float2* Ec, int nk, int k0c,
+                          int wc, int lr, const float2* twt, const float* gamma_in,
+                          float* gamma_out, hipStream_t st) {
 #define X(NN, A, B)                                                                            \
   if (L == NN) {                                                                               \
     using P = reg::GFFT<NN, A, B>;                                                             \
-    constexpr int G = kRegBlock / P::T;                                                        \
-    int rc = allow_lds_adj(k_adj_rfield_reg<P>, adj_reg_lds<P>());                             \
+    constexpr int RB = rows_per_block<P>();                                                    \
+    int rc = allow_lds_adj(k_adj_rfield_reg<P>, adj_rows_lds<P>());                            \
     if (rc) return rc;                                                                         \
-    dim3 grid((lr + G - 1) / G, grid_y_z.y, grid_y_z.z);                                       \
-    hipLaunchKernelGGL(k_adj_rfield_reg<P>, grid, dim3(kRegBlock), adj_reg_lds<P>(), st, Ec,   \
-                       nk, k0c, wc, lr, twt, gamma_in, gamma_out);                             \
+    dim3 grid((lr + RB - 1) / RB, grid_y_z.y, grid_y_z.z);                                     \
+    hipLaunchKernelGGL(k_adj_rfield_reg<P>, grid, dim3(kRegBlock), adj_rows_lds<P>(), st, src, \
+                       Ec, nk, k0c, wc, lr, twt, gamma_in, gamma_out);                         \
     OI_LAUNCH_CHECK("adj_rfield_reg");                                                         \
     return OI_OK;                                                                              \
   }
@@ -394,48 +368,17 @@ static int adj_rfield_reg(int L, dim3 grid_y_z, float2* Ec, int nk, int k0c, int
   return fail(OI_ERR_UNSUPPORTED, "adjoint: no register transform for this coarse size");
 }
 
-// Sizes of the forward's two-pass column buffer.
-#define OI_ADJ_BCOLS_PLANS(X) X(144, 12, 12) X(256, 16, 16) X(450, 15, 30) X(512, 16, 32)
-
-static bool adj_bcols_size(int L) {
-#define X(NN, A, B) if (L == NN) return true;
-  OI_ADJ_BCOLS_PLANS(X)
-#undef X
-  return false;
-}
-
-static int adj_rfield_bcols(int L, dim3 grid_y_z, const float2* Bc, float2* Ec, int nk, int k0c,
-                            int wc, int lr, const float2* twt, const float* gamma_in, hipStream_t st) {
-#define X(NN, A, B)                                                                            \
-  if (L == NN) {                                                                               \
-    using P = reg::GFFT<NN, A, B>;                                                             \
-    constexpr int G = kRegBlock / P::T;                                                        \
-    const size_t tile = (size_t)wc * (G + 1), scr = (size_t)G * P::LDS;                        \
-    const size_t lds = (tile > scr ? tile : scr) * sizeof(float2);                             \
-    int rc = allow_lds_adj(k_adj_rfield_bcols<P>, lds);                                        \
-    if (rc) return rc;                                                                         \
-    dim3 grid((lr + G - 1) / G, grid_y_z.y, grid_y_z.z);                                       \
-    hipLaunchKernelGGL(k_adj_rfield_bcols<P>, grid, dim3(kRegBlock), lds, st, Bc, Ec, nk, k0c, \
-                       wc, lr, twt, gamma_in);                                                 \
-    OI_LAUNCH_CHECK("adj_rfield_bcols");                                                       \
-    return OI_OK;                                                                              \
-  }
-  OI_ADJ_BCOLS_PLANS(X)
-#undef X
-  return fail(OI_ERR_UNSUPPORTED, "adjoint: no two-pass column buffer for this coarse size");
-}
-
 static int adj_cwin_reg(int L, dim3 grid_y_z, const float2* Pc, const float2* kern, int nk,
                         int k0r, int wr, int wc, const float2* twt, float2* Ak, hipStream_t st) {
 #define X(NN, A, B)                                                                            \
   if (L == NN) {                                                                               \
     using P = reg::GFFT<NN, A, B>;                                                             \
-    constexpr int G = kRegBlock / P::T;                                                        \
-    int rc = allow_lds_adj(k_adj_cwin_reg<P>, adj_reg_lds<P>());                               \
+    constexpr int G = cols_per_block<P>();                                                     \
+    int rc = allow_lds_adj(k_adj_cwin_reg<P>, adj_cols_lds<P>());                               \
     if (rc) return rc;                                                                         \
     const int items = ((wc + G - 1) / G) * (int)grid_y_z.y * (int)grid_y_z.z;                  \
     hipLaunchKernelGGL(k_adj_cwin_reg<P>, dim3(xcd_grid(items)), dim3(kRegBlock),              \
-                       adj_reg_lds<P>(), st, Pc, kern, nk, k0r, wr, wc, twt, Ak,               \
+                       adj_cols_lds<P>(), st, Pc, kern, nk, k0r, wr, wc, twt, Ak,               \
                        (int)grid_y_z.z);                                                       \
     OI_LAUNCH_CHECK("adj_cwin_reg");                                                           \
     return OI_OK;                                                                              \
@@ -686,7 +629,7 @@ int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int ba
       if ((rc = adj_cfield_reg(g.lr, dim3(1, 1, batch), specg, nullptr, 1, -g.qr, wgr, wgc,
                                g.flr.tw, Ecg, st)))
         return rc;
-      if ((rc = adj_rfield_reg(g.lc, dim3(1, 1, batch), Ecg, 1, -g.qc, wgc, g.lr, g.flc.tw,
+      if ((rc = adj_rfield_reg(g.lc, dim3(1, 1, batch), Ecg, Ecg, 1, -g.qc, wgc, g.lr, g.flc.tw,
                                nullptr, gamma, st)))
         return rc;
     } else {
@@ -702,20 +645,17 @@ int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int ba
   }
   const float* gam = g.direct ? gI : gamma;
 
-  if (reg && bcols && !g.direct && g.lr == g.lc && adj_bcols_size(g.lr)) {
-    // the column stage is the forward pass's column buffer
-    if ((rc = adj_rfield_bcols(g.lc, dim3(1, nkern, batch), bcols, Ec, nkern, g.k0c, g.wc, g.lr,
-                               g.flc.tw, gam, st)))
-      return rc;
-    if ((rc = adj_cwin_reg(g.lr, dim3(1, nkern, batch), Ec, kern, nkern, g.k0r, g.wr, g.wc,
-                           g.flr.tw, Ak, st)))
-      return rc;
-  } else if (reg) {
-    if ((rc = adj_cfield_reg(g.lr, dim3(1, nkern, batch), spec, kern, nkern, g.k0r, g.wr, g.wc,
-                             g.flr.tw, Ec, st)))
-      return rc;
-    if ((rc = adj_rfield_reg(g.lc, dim3(1, nkern, batch), Ec, nkern, g.k0c, g.wc, g.lr, g.flc.tw,
-                             gam, nullptr, st)))
+  if (reg) {
+    // the column stage is the forward pass's column buffer where it left one
+    const float2* src = g.lr == g.lc ? bcols : nullptr;
+    if (!src) {
+      if ((rc = adj_cfield_reg(g.lr, dim3(1, nkern, batch), spec, kern, nkern, g.k0r, g.wr, g.wc,
+                               g.flr.tw, Ec, st)))
+        return rc;
+      src = Ec;
+    }
+    if ((rc = adj_rfield_reg(g.lc, dim3(1, nkern, batch), src, Ec, nkern, g.k0c, g.wc, g.lr,
+                             g.flc.tw, gam, nullptr, st)))
       return rc;
     if ((rc = adj_cwin_reg(g.lr, dim3(1, nkern, batch), Ec, kern, nkern, g.k0r, g.wr, g.wc,
                            g.flr.tw, Ak, st)))

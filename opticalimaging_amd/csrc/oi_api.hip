@@ -212,7 +212,7 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
     const int L = need > 144 ? fp_two_pass_choose(need)
                              : (L1 > 0 && !fp_one_pass_ok(L1) && fp_two_pass_size_ok(L1) ? L1 : 0);
     if (L > 0 && L < g.ny && L < g.nx && g.wr <= L && g.wc <= L &&
-        fp_two_pass_lds(L, g.wc) <= kLdsLimit) {
+        fp_two_pass_lds(L) <= kLdsLimit) {
       g.path = 2;
       g.lr = g.lc = lr = lc = L;
       if (g.max_groups <= 0) {

@@ -108,7 +108,7 @@ int ilt_target_const(const float* target, size_t npix, const float2* tband, size
 // batch * nkern * nchan * wc * L c64; R in [img][group][q][t].
 bool fp_two_pass_size_ok(int l);
 int fp_two_pass_choose(int need);
-size_t fp_two_pass_lds(int L, int wc);
+size_t fp_two_pass_lds(int L);
 int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st);
 
 }  // namespace oi

@@ -644,10 +644,16 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
 // ------------------------------------------------ two-pass coherent sum
 // For coarse grids too large for one workgroup (L = 256, 512).  Pass 1
 // transforms every window column of every (kernel, channel) into
-// B[img][kc][c][t] (column-major, t the coarse row); pass 2 gives each block G
-// coarse rows, loops over all (kernel, channel) pairs reading its rows of B
-// through an LDS tile, and accumulates |E|^2 in registers; its epilogue takes
-// the row DFT (+ sign) to R.  Stage twiddles are read from the table at use.
+// B[img][kc][t][c] (row-major, t the coarse row); pass 2 gives each wavefront
+// 64 / T coarse rows, loops over all (kernel, channel) pairs reading its rows
+// of B, and accumulates |E|^2 in registers; its epilogue takes the row DFT
+// (+ sign) to R.
+//
+// Pass 1: consecutive lanes hold consecutive window columns, so that a load of
+// the kernel, the spectrum or a store to B is a run of G columns (128 bytes at
+// G = 16) and not four of each of sixteen rows.  Bound by the stores of B: 16
+// images x 12 kernels x 105 columns of 256 in 20 us (41 MB; with the exchange
+// inside one wave instead, four columns each, 25 us).
 template <class PL>
 __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ spec,
                                                      const float2* __restrict__ kern, int nk,
@@ -656,11 +662,12 @@ __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ 
                                                      float2* __restrict__ B) {
   constexpr int L = PL::N, TL = PL::T, VL = PL::V, G = groups_per_block<PL>();
   extern __shared__ float2 lds[];
-  const int g = threadIdx.x / TL, t = threadIdx.x - g * TL;
+  const int g = threadIdx.x % G, tg = threadIdx.x / G;
   const int c = blockIdx.x * G + g;
   const int kc = blockIdx.y, img = blockIdx.z;        // kc = k * nchan + channel
   const int k = kc / nchan, ch = kc - k * nchan;
-  const bool live = g < G && c < wc;
+  const bool live = tg < TL && c < wc;
+  const int t = tg < TL ? tg : 0;
   const float2* kp = kern + (size_t)k * wr * wc;
   const float2* sp = spec + ((size_t)img * nchan + ch) * wr * wc;
   const int kr0 = pmod(t - k0r, L);
@@ -672,81 +679,93 @@ __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ 
     // rounded product: the adjoint's k_adj_cfield_reg forms the same values
     v[m] = (live && kr < wr) ? reg::mul_rn(kp[kr * wc + c], sp[kr * wc + c]) : make_float2(0.f, 0.f);
   }
-  PL::template run_live_tab<false>(v, lds + g * PL::LDS, t, twt, live);
+  PL::template run_live_tab<false>(v, lds + g * (PL::LDS | 1), t, twt, live);
   if (!live) return;
-  float2* dst = B + (((size_t)img * nk * nchan + kc) * wc + c) * L;
+  float2* dst = B + ((size_t)img * nk * nchan + kc) * L * wc + c;
 #pragma unroll
-  for (int m = 0; m < VL; ++m) dst[t + TL * m] = v[m];
+  for (int m = 0; m < VL; ++m) dst[(size_t)(t + TL * m) * wc] = v[m];
 }
 
-// Blocks (row group, img, grp) sum the (kernel, channel) pairs kc = grp,
-// grp + groups, ... into their own partial R[img][grp].
-// Four waves per SIMD (at most 128 registers) up to coarse 256: four
-// workgroups then share a CU, as their 34 KB of LDS allow (ILT step 0.355 ->
-// 0.348 ms).  From 450 on the LDS (about 70 KB) holds two workgroups per CU
-// whatever the registers, and the 30- and 32-value transforms would spill
-// under 128: two waves per SIMD (up to 256 registers).
+template <class PL>
+constexpr size_t bcols_lds() {
+  return (size_t)groups_per_block<PL>() * (PL::LDS | 1) * sizeof(float2);
+}
+
+// Coarse rows per workgroup of the row pass: whole transform groups per wave.
+template <class PL>
+constexpr int brows_rows() {
+  return (kBlock / 64) * (64 / PL::T);
+}
+
+// Waves per SIMD that the registers are sized for: up to 256 three (at most 168
+// registers hold a row, its sums and its twiddles; under the 128 of four waves
+// they spill), above that two.
 template <class PL>
 constexpr int brows_min_blocks() {
-  return PL::N > 256 ? 2 : 4;
+  return PL::N > 256 ? 2 : 3;
 }
 
+// Items (row group, image, kernel group); an item sums the (kernel, channel)
+// pairs kc = grp, grp + groups, ... into its own partial R[img][grp].
+// A wave is on its own: it loads its rows of B straight into registers (a row
+// is contiguous) and exchanges inside its own part of the LDS, so the loop has
+// no workgroup barrier, where staging a column-major B through an LDS tile took
+// six a kernel and left the waves waiting for each other.  Row pass of 16 images
+// x 12 kernels at L = 256: 30 -> 21 us, 24 x 12: 45 -> 26, 4 x 12 at L = 450:
+// 56 -> 32.  Loading the next kernel's row ahead needs 32 more registers and
+// gives up a wave per SIMD for it: 21, 32 and 49 us.
 template <class PL>
 __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(const float2* __restrict__ B, int nkc, int k0c,
                                                      int wc, int qc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ R, int batch,
                                                      int groups) {
-  constexpr int L = PL::N, TL = PL::T, VL = PL::V, G = groups_per_block<PL>();
-  constexpr int TS = G + 1;                // tile row stride (bank spread)
+  constexpr int L = PL::N, TL = PL::T, VL = PL::V, GW = 64 / TL, RB = brows_rows<PL>();
   static_assert(VL <= 32, "row mask holds VL bits");
   extern __shared__ float2 lds[];
-  // items (row group, image, kernel group), row groups fastest, in XCD order:
-  // a column of B is split over the row groups of one (image, kernel group),
-  // and where 8 G bytes do not divide the line, the lines at the edges are
-  // read by two of them
-  constexpr int NXR = (L + G - 1) / G;
+  // row groups fastest, in XCD order: neighbouring rows share the lines at
+  // their ends
+  constexpr int NXR = (L + RB - 1) / RB;
   int w;
   if (!xcd_item(blockIdx.x, NXR * batch * groups, w)) return;   // uniform over the block
   const int xr = w % NXR, img = (w / NXR) % batch, grp = w / (NXR * batch);
-  float2* tile = lds;                      // [wc][TS]
-  float2* scr = lds;                       // transform scratch, over the tile once it is read
-  const int g = threadIdx.x / TL, t = threadIdx.x - g * TL;
-  const int r0 = xr * G;
-  const int row = r0 + g;
-  const bool live = g < G && row < L;
+  const int lane = threadIdx.x & 63, gw = lane / TL;
+  const int t = gw < GW ? lane - gw * TL : 0;
+  const int g = (threadIdx.x >> 6) * GW + (gw < GW ? gw : 0);
+  const int row = xr * RB + g;
+  const bool live = gw < GW && row < L;
+  float2* scr = lds + g * PL::LDS;
+  const int c0 = pmod(t - k0c, L);                    // TL m < L: c = c0 + TL m, less L once
   unsigned rmask = 0;
-  int cidx[VL];
 #pragma unroll
   for (int m = 0; m < VL; ++m) {
-    const int cc = pmod(t + TL * m - k0c, L);
-    cidx[m] = cc < wc ? cc : 0;
+    int cc = c0 + TL * m;
+    cc = cc >= L ? cc - L : cc;
     if (live && cc < wc) rmask |= 1u << m;
   }
+  typename PL::Tw tw;
+  PL::load_tw(tw, t, twt);
   float acc[VL];
 #pragma unroll
   for (int m = 0; m < VL; ++m) acc[m] = 0.f;
+  const float2* src = B + ((size_t)img * nkc + grp) * L * wc + (size_t)(live ? row : 0) * wc;
+  const size_t step = (size_t)groups * L * wc;
+  float2 v[VL];
   for (int kc = grp; kc < nkc; kc += groups) {
-    const float2* src = B + ((size_t)img * nkc + kc) * wc * L + r0;
-    __syncthreads();
-    for (int e = threadIdx.x; e < wc * G; e += kBlock) {
-      const int cc = e / G, r = e - cc * G;
-      tile[cc * TS + r] = (r0 + r < L) ? src[(size_t)cc * L + r] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    float2 v[VL];
 #pragma unroll
-    for (int m = 0; m < VL; ++m)
-      v[m] = ((rmask >> m) & 1u) ? tile[cidx[m] * TS + (g < G ? g : 0)] : make_float2(0.f, 0.f);
-    __syncthreads();                       // every row is read: the scratch reuses the tile
-    PL::template run_live_tab<false>(v, scr + g * PL::LDS, t, twt, g < G);
+    for (int m = 0; m < VL; ++m) {
+      int cc = c0 + TL * m;
+      cc = cc >= L ? cc - L : cc;
+      v[m] = ((rmask >> m) & 1u) ? src[cc] : make_float2(0.f, 0.f);
+    }
+    src += step;
+    PL::template run_live_wave<false>(v, scr, t, tw, live);
 #pragma unroll
     for (int m = 0; m < VL; ++m) acc[m] += v[m].x * v[m].x + v[m].y * v[m].y;
   }
-  float2 v[VL];
 #pragma unroll
   for (int m = 0; m < VL; ++m) v[m] = make_float2(acc[m], 0.f);
-  PL::template run_live_tab<true>(v, scr + g * PL::LDS, t, twt, g < G);
+  PL::template run_live_wave<true>(v, scr, t, tw, live);
   if (!live) return;
   const int nq = qc + 1;
 #pragma unroll
@@ -1249,27 +1268,24 @@ static int run_band(const FpArgs& a, int groups, hipStream_t st) {
 #define OI_TWO_PASS_PLANS(X) X(144, 12, 12) X(256, 16, 16) X(450, 15, 30) X(512, 16, 32)
 
 template <class PL>
-static size_t two_pass_rows_lds(int wc) {
-  // the row tile and the transform scratch share the LDS (k_fp_brows)
-  const size_t tile = (size_t)wc * (groups_per_block<PL>() + 1);
-  const size_t scr = (size_t)scratch_groups<PL>() * PL::LDS;
-  return (tile > scr ? tile : scr) * sizeof(float2);
+static size_t two_pass_rows_lds() {
+  return (size_t)brows_rows<PL>() * PL::LDS * sizeof(float2);
 }
 
 template <class PL>
 static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st) {
-  constexpr int G = groups_per_block<PL>();
-  const size_t lds1 = rows_lds<PL>();
+  constexpr int G = groups_per_block<PL>(), RB = brows_rows<PL>();
+  const size_t lds1 = bcols_lds<PL>();
   int rc = allow(k_fp_bcols<PL>, lds1);
   if (rc) return rc;
   dim3 g1((a.wc + G - 1) / G, c.nkern * c.nchan, a.batch);
   hipLaunchKernelGGL(k_fp_bcols<PL>, g1, dim3(kBlock), lds1, st, c.spec, c.kern, c.nkern, c.nchan,
                      a.k0r, a.wr, a.wc, a.tw_l, B);
   OI_LAUNCH_CHECK("fp_bcols");
-  const size_t lds2 = two_pass_rows_lds<PL>(a.wc);
+  const size_t lds2 = two_pass_rows_lds<PL>();
   rc = allow(k_fp_brows<PL>, lds2);
   if (rc) return rc;
-  const int items = ((PL::N + G - 1) / G) * a.batch * c.groups;
+  const int items = ((PL::N + RB - 1) / RB) * a.batch * c.groups;
   hipLaunchKernelGGL(k_fp_brows<PL>, dim3(xcd_grid(items)), dim3(kBlock), lds2, st, B,
                      c.nkern * c.nchan, a.k0c, a.wc, a.qc, a.tw_l, c.R, a.batch,
                      c.groups);
@@ -1295,8 +1311,13 @@ int fp_two_pass_choose(int need) {
   return best;
 }
 
-size_t fp_two_pass_lds(int L, int wc) {
-#define X(NN, A, B) if (L == NN) return fp::two_pass_rows_lds<reg::GFFT<NN, A, B>>(wc);
+size_t fp_two_pass_lds(int L) {
+#define X(NN, A, B)                                                                       \
+  if (L == NN) {                                                                          \
+    using P = reg::GFFT<NN, A, B>;                                                        \
+    const size_t cols = fp::bcols_lds<P>(), rows = fp::two_pass_rows_lds<P>();            \
+    return cols > rows ? cols : rows;                                                     \
+  }
   OI_TWO_PASS_PLANS(X)
 #undef X
   return (size_t)-1;

@@ -337,6 +337,12 @@ struct GFFT {
     run_gen<INV, true>(v, [lds](int i) -> float2& { return lds[xi(i)]; }, t, RegTw{tw}, live);
   }
 
+  template <bool INV>
+  __device__ __forceinline__ static void run_live_tab_wave(float2 (&v)[V], float2* lds, int t,
+                                                           const float2* table, bool live) {
+    run_gen<INV, true>(v, [lds](int i) -> float2& { return lds[xi(i)]; }, t, TabTw{table}, live);
+  }
+
   template <bool INV, bool WAVE = false, class Addr, class TW>
   __device__ __forceinline__ static void run_gen(float2 (&v)[V], Addr at, int t, const TW& tw,
                                                  bool live) {

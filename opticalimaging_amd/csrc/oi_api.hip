@@ -109,7 +109,8 @@ struct oi_plan {
   float* Ic = nullptr;
   float2* Ihat = nullptr;
   float* part = nullptr;    // residual sums of the image-row pass, [B][ny]
-  float2* Bbuf = nullptr;   // two-pass column fields of max_batch x max_kernels kernels
+  float2* Bbuf = nullptr;   // two-pass column fields of max_kernels kernels of
+  int bimg = 0;             // this many images (path 2: max_batch)
   float* dft = nullptr;     // product tables of the image lengths (dft_bytes)
   DftTable tab_x, tab_y;
   size_t bytes = 0;
@@ -254,13 +255,36 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
   return OI_OK;
 }
 
+// Column fields of one image in the two-pass coherent sum.
+static size_t column_bytes(const oi_geometry& g) {
+  return (size_t)g.max_kernels * g.nchan * g.wc * (size_t)g.lr * sizeof(float2);
+}
+
+// Images whose column fields a plan holds.  The two-pass path keeps its batch's
+// (the adjoint reads them again).  On the one-pass path, coarse grids of 100 and
+// 128 are summed in two passes too, in chunks of images: 8 fields x 3 channels x
+// 24 kernels at 128 take 64 us in the one-pass kernel, whose rows wait for its
+// columns behind workgroup barriers, and 16 us in two passes.  A chunk is
+// bounded (512 MiB), and kernel sets of which one image passes 128 MiB stay with
+// the one-pass kernel.
+constexpr size_t kColumnsImage = (size_t)128 << 20, kColumnsPlan = (size_t)512 << 20;
+
+static size_t column_images(const oi_geometry& g, size_t B) {
+  if (g.path == 2) return B;
+  if (g.path != 1 || !fp_split_size_ok(g.lr) || g.wr > g.lr || g.wc > g.lr) return 0;
+  const size_t one = column_bytes(g);
+  if (one > kColumnsImage) return 0;
+  return B * one <= kColumnsPlan ? B : kColumnsPlan / one;
+}
+
 // Device scratch of a plan for max_batch images: byte size of each buffer.
 struct ScratchLayout {
   size_t T, spec, R, U, Ic, Ihat, part, Bbuf;
   size_t total() const { return T + spec + R + U + Ic + Ihat + part + Bbuf; }
 };
 
-static ScratchLayout scratch_layout(const oi_geometry& g, size_t B) {
+// columns: with the column fields that a one-pass plan can do without.
+static ScratchLayout scratch_layout(const oi_geometry& g, size_t B, bool columns = true) {
   const size_t C = (size_t)g.nchan, G = (size_t)g.max_groups;
   const size_t lr = (size_t)g.lr, lc = (size_t)g.lc;
   ScratchLayout s;
@@ -271,7 +295,7 @@ static ScratchLayout scratch_layout(const oi_geometry& g, size_t B) {
   s.Ic = (g.direct && G > 1) ? B * G * lr * lc * sizeof(float) : 0;
   s.Ihat = g.path ? B * (size_t)(g.qc + 1) * (2 * g.qr + 1) * sizeof(float2) : 0;
   s.part = g.path ? B * (size_t)g.ny * sizeof(float) : 0;
-  s.Bbuf = g.path == 2 ? B * (size_t)g.max_kernels * C * g.wc * lr * sizeof(float2) : 0;
+  s.Bbuf = (columns || g.path == 2) ? column_images(g, B) * column_bytes(g) : 0;
   return s;
 }
 
@@ -322,6 +346,7 @@ extern "C" int oi_plan_create(oi_geometry* geo, oi_plan** out) {
   p->flc = d[3];
   p->frows = d[4];
   const ScratchLayout sl = scratch_layout(g, (size_t)g.max_batch);
+  p->bimg = (int)column_images(g, (size_t)g.max_batch);
   struct Want {
     void** ptr;
     size_t bytes;
@@ -515,16 +540,15 @@ extern "C" int oi_coherent_image(oi_plan* p, const void* spec, int batch, const 
   return coherent_impl(p, spec, batch, kern, nkern, out, nullptr, (hipStream_t)stream);
 }
 
-// One-pass plans take max_batch sets a launch chain: a chain of one image leaves
-// its three interpolation launches and the last kernels of the sum with most
-// of the chip idle.  Others take the sets one by one: their launches are larger,
-// and a two-pass plan would need the column fields of every set at once.
+// Plans of compile-time sizes take max_batch sets a launch chain: a chain of one
+// image leaves its three interpolation launches and the last kernels of the sum
+// with most of the chip idle.  The generic kernels take the sets one by one.
 extern "C" int oi_coherent_sets(oi_plan* p, const void* spec, int nsets, const void* kern,
                                 int nkern, float* out, void* stream) {
   if (!p || !kern || !out) return fail(OI_ERR_INVALID, "coherent_sets: null argument");
   if (nsets < 1) return fail(OI_ERR_INVALID, "coherent_sets: nsets must be >= 1");
   const oi_geometry& g = p->g;
-  const int step = g.path == 1 ? g.max_batch : 1;
+  const int step = g.path ? g.max_batch : 1;
   for (int s = 0; s < nsets; s += step) {
     const int n = nsets - s < step ? nsets - s : step;
     const int rc = coherent_impl(p, spec, n, static_cast<const float2*>(kern) + (size_t)s * nkern * g.wr * g.wc,
@@ -544,8 +568,8 @@ static bool residual_fused(const oi_plan* p) {
 
 // target non-null: out = 2 (I - target), partial sums of (I - target)^2 in p->part.
 // band_only (plans with the residual pass): the band p->Ihat of the image, no image.
-// sets (one image, or a one-pass plan): the images share one spectrum and have
-// nkern kernels each.
+// sets (one image, or a plan of compile-time sizes): the images share one
+// spectrum and have nkern kernels each.
 static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* kern, int nkern,
                          float* out, const float* target, hipStream_t st, bool band_only, bool sets) {
   if (!p || !spec || !kern || (!out && !band_only))
@@ -560,34 +584,6 @@ static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* ke
   const oi_geometry& g = p->g;
   const int phases = g.lr / g.rows;
   int groups = g.max_groups < nkern ? g.max_groups : nkern;
-  if (g.path == 2) {
-    FpArgs a = fast_args(p, batch, st);
-    a.out = out;
-    a.target = target;
-    a.part = p->part;
-    FpCoh c{};
-    c.spec = static_cast<const float2*>(spec);
-    c.kern = static_cast<const float2*>(kern);
-    c.nchan = g.nchan;
-    c.nkern = nkern;
-    c.k0r = g.k0r;
-    c.wr = g.wr;
-    c.k0c = g.k0c;
-    c.wc = g.wc;
-    const int nkc = nkern * g.nchan;
-    c.groups = groups < nkc ? groups : nkc;
-    c.qc = g.qc;
-    c.tw_l = p->flr.tw;
-    c.tw_m = p->flr.tw;
-    c.R = p->R;
-    int rc = fp_two_pass(a, c, p->Bbuf, st);
-    if (rc) return rc;
-    if (band_only) return fp_band(a, c.groups, st);
-    mark(p, 3, st);
-    rc = fp_interp(a, c.groups, st);
-    mark_done(p);
-    return rc;
-  }
   if (g.path) {
     FpArgs a = fast_args(p, batch, st);
     a.out = out;
@@ -609,8 +605,23 @@ static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* ke
     c.tw_l = p->flr.tw;
     c.tw_m = p->flr.tw;
     c.R = p->R;
-    if (band_only) return fp_image_band(a, c, st);
-    int rc = fp_image(a, c, st);
+    int rc;
+    if (p->Bbuf) {
+      for (int i = 0; i < batch; i += p->bimg) {
+        FpArgs ai = a;
+        FpCoh ci = c;
+        ai.batch = batch - i < p->bimg ? batch - i : p->bimg;
+        ci.spec += i * c.spec_img;
+        ci.kern += i * c.kern_img;
+        ci.R += (size_t)i * c.groups * (g.qc + 1) * g.lr;
+        if ((rc = fp_two_pass(ai, ci, p->Bbuf, st))) return rc;
+      }
+    } else if ((rc = fp_coherent(a, c, st))) {
+      return rc;
+    }
+    if (band_only) return fp_band(a, c.groups, st);
+    mark(p, 3, st);
+    rc = fp_interp(a, c.groups, st);
     mark_done(p);
     return rc;
   }
@@ -782,6 +793,12 @@ static AdjGeom adj_geom(const oi_plan* p) {
   return a;
 }
 
+// The column fields that the forward pass of `batch` images left in the plan,
+// null where it made none or had to take the images in chunks.
+static const float2* columns_of(const oi_plan* p, int batch) {
+  return batch <= p->bimg ? p->Bbuf : nullptr;
+}
+
 extern "C" int oi_socs_residual_adjoint(oi_plan* p, const float* mask, int batch, const void* kern,
                                         int nkern, const float* target, float* resid2, float* loss,
                                         void* work, float* grad_mask, void* stream) {
@@ -790,7 +807,7 @@ extern "C" int oi_socs_residual_adjoint(oi_plan* p, const float* mask, int batch
   if (rc) return rc;
   // the residual pass left this batch's mask spectrum in p->spec and, on the
   // two-pass path, its kernels' column stage in p->Bbuf
-  const float2* bcols = p->g.path == 2 ? p->Bbuf : nullptr;
+  const float2* bcols = columns_of(p, batch);
   return launch_adjoint(adj_geom(p), resid2, p->spec, batch, static_cast<const float2*>(kern), nkern,
                         work, grad_mask, (hipStream_t)stream, bcols);
 }
@@ -864,7 +881,7 @@ static int band_step_impl(oi_plan* p, const float* field, bool logits, int batch
   if (rc) return rc;
   if (loss && (rc = ilt_sum(p->part, batch * ilt_band_blocks(p->g.qr, p->g.qc), loss, st)))
     return rc;
-  const float2* bcols = p->g.path == 2 ? p->Bbuf : nullptr;
+  const float2* bcols = columns_of(p, batch);
   return launch_adjoint(ag, nullptr, p->spec, batch, static_cast<const float2*>(kern), nkern, work,
                         grad, st, bcols, logits ? field : nullptr, logits ? p->part : nullptr);
 }
@@ -997,11 +1014,11 @@ static size_t aligned_total(const ScratchLayout& s) {
 
 // Scratch of one image with its tables, at most (twiddle tables counted once
 // per transform length, shared or not).
-static size_t noalloc_bytes(const oi_geometry& g) {
+static size_t noalloc_bytes(const oi_geometry& g, bool columns) {
   const size_t tw = align_up(2 * (size_t)g.nx * sizeof(float2)) + align_up(2 * (size_t)g.ny * sizeof(float2)) +
                     align_up(2 * (size_t)g.lr * sizeof(float2)) + align_up(2 * (size_t)g.lc * sizeof(float2)) +
                     align_up(2 * (size_t)g.rows * sizeof(float2));
-  return tw + align_up(dft_bytes(g, false) + dft_bytes(g, true)) + aligned_total(scratch_layout(g, 1));
+  return tw + align_up(dft_bytes(g, false) + dft_bytes(g, true)) + aligned_total(scratch_layout(g, 1, columns));
 }
 
 extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, int kind, int cin,
@@ -1021,7 +1038,8 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   // the tables and buffers of image lengths without a register transform may
   // not fit beside one image: those sizes then take the generic kernels, whose
   // scratch is smaller
-  if (noalloc_bytes(g) > kNoAllocScratch && (rc = plan_geometry(in, g, true))) return rc;
+  if (noalloc_bytes(g, false) > kNoAllocScratch && (rc = plan_geometry(in, g, true))) return rc;
+  const bool columns = noalloc_bytes(g, true) <= kNoAllocScratch;
   // twiddle tables first, one per distinct length
   const int sizes[5] = {g.nx, g.ny, g.lr, g.lc, g.rows};
   FftDesc d[5];
@@ -1038,7 +1056,7 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   }
   const size_t dft_off = used;
   used += align_up(dft_bytes(g, false) + dft_bytes(g, true));
-  const size_t per_image = aligned_total(scratch_layout(g, 1));
+  const size_t per_image = aligned_total(scratch_layout(g, 1, columns));
   if (used + per_image > kNoAllocScratch)
     return fail(OI_ERR_INVALID, "socs_image_noalloc: one image needs " +
                                     std::to_string(used + per_image) + " bytes of scratch, beyond the " +
@@ -1073,7 +1091,8 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   pl.frows = d[4];
   pl.dft = reinterpret_cast<float*>(base + dft_off);
   if ((rc = dft_build(&pl, st))) return rc;
-  const ScratchLayout sl = scratch_layout(pl.g, (size_t)chunk);
+  const ScratchLayout sl = scratch_layout(pl.g, (size_t)chunk, columns);
+  pl.bimg = sl.Bbuf ? (int)column_images(pl.g, (size_t)chunk) : 0;
   unsigned char* cur = base + used;
   auto carve = [&cur](size_t bytes) -> unsigned char* {
     unsigned char* p = bytes ? cur : nullptr;

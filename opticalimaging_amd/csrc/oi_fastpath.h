@@ -48,7 +48,7 @@ struct FpArgs {
 
 struct FpCoh {
   const float2* spec;   // image i's spectra start at spec + i spec_img, its kernels at
-  const float2* kern;   // kern + i kern_img (one-pass sums; 0: shared by the images)
+  const float2* kern;   // kern + i kern_img (0: shared by the images)
   size_t spec_img, kern_img;
   int nchan, nkern;
   int k0r, wr, k0c, wc;
@@ -72,10 +72,8 @@ size_t fp_coherent_lds(int L, int wr, int wc);
 int fp_coherent_rows_fit(int L);
 bool fp_one_pass_ok(int L);             // the one-pass coherent kernel serves L
 int fp_spectrum(const FpArgs& a, hipStream_t st);  // marks stage 1 between its launches
-int fp_image(const FpArgs& a, const FpCoh& c, hipStream_t st);  // marks stages 3, 4, 5
+int fp_coherent(const FpArgs& a, const FpCoh& c, hipStream_t st);   // the one-pass coherent sum to R
 int fp_interp(const FpArgs& a, int groups, hipStream_t st);      // marks stages 4, 5
-// the one-pass coherent sum and the band Ihat of the image, without the image
-int fp_image_band(const FpArgs& a, const FpCoh& c, hipStream_t st);
 // the band Ihat from partial sums R (the first kernel of fp_interp)
 int fp_band(const FpArgs& a, int groups, hipStream_t st);
 // interpolation column and row transforms of a band already in a.Ihat
@@ -104,9 +102,12 @@ int ilt_update_theta(float* theta, const float* gt, float lr, int batch, size_t 
 size_t ilt_target_const_scratch(int batch);
 int ilt_target_const(const float* target, size_t npix, const float2* tband, size_t nband,
                      int batch, void* scratch, float* tconst, hipStream_t st);
-// Two-pass coherent sum for coarse grids L in {256, 512}: B holds
-// batch * nkern * nchan * wc * L c64; R in [img][group][q][t].
+// Two-pass coherent sum: B holds batch * nkern * nchan * wc * L c64; R in
+// [img][group][q][t].  fp_two_pass_size_ok: the two-pass path's coarse grids;
+// fp_split_size_ok: grids of the one-pass path that it serves better where a
+// plan holds B.
 bool fp_two_pass_size_ok(int l);
+bool fp_split_size_ok(int l);
 int fp_two_pass_choose(int need);
 size_t fp_two_pass_lds(int L);
 int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st);

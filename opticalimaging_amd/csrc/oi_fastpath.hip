@@ -656,7 +656,8 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
 // inside one wave instead, four columns each, 25 us).
 template <class PL>
 __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ spec,
-                                                     const float2* __restrict__ kern, int nk,
+                                                     const float2* __restrict__ kern,
+                                                     size_t spec_img, size_t kern_img, int nk,
                                                      int nchan, int k0r, int wr, int wc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ B) {
@@ -668,8 +669,8 @@ __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ 
   const int k = kc / nchan, ch = kc - k * nchan;
   const bool live = tg < TL && c < wc;
   const int t = tg < TL ? tg : 0;
-  const float2* kp = kern + (size_t)k * wr * wc;
-  const float2* sp = spec + ((size_t)img * nchan + ch) * wr * wc;
+  const float2* kp = kern + img * kern_img + (size_t)k * wr * wc;
+  const float2* sp = spec + img * spec_img + (size_t)ch * wr * wc;
   const int kr0 = pmod(t - k0r, L);
   float2 v[VL];
 #pragma unroll
@@ -1264,8 +1265,11 @@ static int run_band(const FpArgs& a, int groups, hipStream_t st) {
   return OI_OK;
 }
 
-// Large coarse grids of the two-pass coherent sum.
+// Coarse grids of the two-pass coherent sum: those of the two-pass path, and
+// those of the one-pass path whose tile no workgroup holds with one wave per
+// transform group (OI_COARSE_PLANS without a thread count).
 #define OI_TWO_PASS_PLANS(X) X(144, 12, 12) X(256, 16, 16) X(450, 15, 30) X(512, 16, 32)
+#define OI_SPLIT_PLANS(X) X(100, 10, 10) X(128, 8, 16)
 
 template <class PL>
 static size_t two_pass_rows_lds() {
@@ -1279,8 +1283,8 @@ static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t 
   int rc = allow(k_fp_bcols<PL>, lds1);
   if (rc) return rc;
   dim3 g1((a.wc + G - 1) / G, c.nkern * c.nchan, a.batch);
-  hipLaunchKernelGGL(k_fp_bcols<PL>, g1, dim3(kBlock), lds1, st, c.spec, c.kern, c.nkern, c.nchan,
-                     a.k0r, a.wr, a.wc, a.tw_l, B);
+  hipLaunchKernelGGL(k_fp_bcols<PL>, g1, dim3(kBlock), lds1, st, c.spec, c.kern, c.spec_img,
+                     c.kern_img, c.nkern, c.nchan, a.k0r, a.wr, a.wc, a.tw_l, B);
   OI_LAUNCH_CHECK("fp_bcols");
   const size_t lds2 = two_pass_rows_lds<PL>();
   rc = allow(k_fp_brows<PL>, lds2);
@@ -1311,6 +1315,13 @@ int fp_two_pass_choose(int need) {
   return best;
 }
 
+bool fp_split_size_ok(int l) {
+#define X(NN, A, B) if (l == NN) return true;
+  OI_SPLIT_PLANS(X)
+#undef X
+  return false;
+}
+
 size_t fp_two_pass_lds(int L) {
 #define X(NN, A, B)                                                                       \
   if (L == NN) {                                                                          \
@@ -1327,6 +1338,7 @@ int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st) {
   int rc = OI_ERR_UNSUPPORTED;
 #define X(NN, A, B_) if (a.L == NN) rc = fp::run_two_pass<reg::GFFT<NN, A, B_>>(a, c, B, st);
   OI_TWO_PASS_PLANS(X)
+  OI_SPLIT_PLANS(X)
 #undef X
   if (rc == OI_ERR_UNSUPPORTED) return fail(rc, "two-pass path: unsupported coarse size");
   return rc;
@@ -1505,26 +1517,13 @@ int fp_spectrum(const FpArgs& a, hipStream_t st) {
   return stage_cols(a, st);
 }
 
-static int fp_coherent(const FpArgs& a, const FpCoh& c, hipStream_t st) {
+int fp_coherent(const FpArgs& a, const FpCoh& c, hipStream_t st) {
   int rc = OI_ERR_UNSUPPORTED;
 #define X(NN, A, B, NT) if (a.L == NN) rc = fp::run_coherent<reg::GFFT<NN, A, B>, NT>(a, c, st);
   OI_COARSE_PLANS(X)
 #undef X
   if (rc) return rc == OI_ERR_UNSUPPORTED ? fail(rc, "fast path: unsupported coarse size") : rc;
   return OI_OK;
-}
-
-int fp_image(const FpArgs& a, const FpCoh& c, hipStream_t st) {
-  int rc = fp_coherent(a, c, st);
-  if (rc) return rc;
-  if (a.mark) a.mark(a.mark_ctx, 3);
-  return fp_interp(a, c.groups, st);
-}
-
-int fp_image_band(const FpArgs& a, const FpCoh& c, hipStream_t st) {
-  int rc = fp_coherent(a, c, st);
-  if (rc) return rc;
-  return fp_band(a, c.groups, st);
 }
 
 }  // namespace oi

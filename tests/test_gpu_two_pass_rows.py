@@ -42,3 +42,51 @@ def test_image_and_gradient(gpu, ny, nx, rows, cols, K, batch, coarse):
         assert np.max(np.abs(img[b] - ref)) <= IMAGE_TOL * ref.max()
         ref = _gradient(full, h[b], g[b])
         assert np.max(np.abs(grad[b] - ref)) <= GRAD_TOL * np.abs(ref).max()
+
+
+# the one-pass path's grids of 100 and 128, summed in two passes: window, channels, kernels, batch
+SPLIT = [
+    (128, 192, (-24, 48), (-25, 50), 1, 7, 3, 100),
+    (192, 128, (-2, 4), (-20, 45), 3, 1, 1, 100),
+    (256, 256, (-31, 64), (-28, 57), 3, 24, 2, 128),
+    (160, 512, (-30, 61), (-40, 52), 2, 3, 4, 128),
+]
+
+
+@pytest.mark.parametrize("ny,nx,rows,cols,nchan,K,batch,coarse", SPLIT)
+def test_split_sum_of_fields(gpu, ny, nx, rows, cols, nchan, K, batch, coarse):
+    from opticalimaging_amd import _native as nat
+    ks, full = _kernels(ny, nx, rows, cols, K, ny + K)
+    plan = engine.plan_for(ks, nchan, batch)
+    assert plan.info()["path"] < 2 and plan.info()["lr"] == coarse
+    rng = np.random.default_rng(nx)
+    f = (rng.standard_normal((batch, ny, nx, 3)) + 1j * rng.standard_normal((batch, ny, nx, 3))).astype(np.complex64)
+    chans = [2, 0, 1][:nchan]
+    img = engine.socs_image(torch.as_tensor(f).cuda(), ks, kind=nat.OI_FIELD_C64_CHLAST, cin=3,
+                            chans=chans).cpu().numpy()
+    for b in range(batch):
+        ref = sum(_image(full, f[b, :, :, c]) for c in chans)
+        assert np.max(np.abs(img[b] - ref)) <= IMAGE_TOL * ref.max()
+    if nchan == 1:
+        h, g = rng.random((2, batch, ny, nx)).astype(np.float32)
+        out = engine.socs_adjoint(torch.as_tensor(h).cuda(), torch.as_tensor(g).cuda(), ks,
+                                  pack_real=False).cpu().numpy()
+        for b in range(batch):
+            ref = _gradient(full, h[b], g[b])
+            assert np.max(np.abs(out[b] - ref)) <= GRAD_TOL * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("K,batch", [(1700, 6), (2300, 2)])
+def test_split_sum_beyond_its_bounds(gpu, K, batch):
+    """Column fields of 104 MB an image (chunks of five images) and of 141 MB
+    (the one-pass kernel) against one kernel set split over two calls: the same
+    squares in another order, K 2^-24 of the peak."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    win = torch.randn((K, 60, 60), dtype=torch.complex64, device="cuda", generator=g)
+    m = torch.rand((batch, 192, 160), device="cuda", generator=g)
+    def image(w):
+        ks = engine.KernelSet(w.contiguous(), -30, -30, 192, 160)
+        return engine.socs_image(m, ks, pack_real=False)
+    out = image(win)
+    ref = image(win[:K // 2]) + image(win[K // 2:])
+    assert (out - ref).abs().max() <= K * 2.0 ** -24 * ref.max()

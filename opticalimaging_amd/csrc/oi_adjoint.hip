@@ -202,14 +202,13 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cfield_reg(const float2* __re
 #pragma unroll
   for (int m = 0; m < V; ++m) {
     const int ir = pmod(t + T * m - k0r, L);
-    float2 a = make_float2(0.f, 0.f);
-    if (on && ir < wr) {
-      a = sb[(size_t)ir * wc];
-      // kernel x spectrum as the forward's k_fp_bcols forms it, so that Ec
-      // holds the same bits as its column buffer
-      if (kb) a = reg::mul_rn(kb[(size_t)ir * wc], a);
-    }
-    v[m] = a;
+    // every load at a valid address, as in the forward's k_fp_bcols; kernel x
+    // spectrum as it forms it, so that Ec holds the same bits as its buffer
+    const bool in = on && ir < wr;
+    const size_t at = in ? (size_t)ir * wc : 0;
+    float2 a = sb[at];
+    if (kb) a = reg::mul_rn(kb[at], a);
+    v[m] = in ? a : make_float2(0.f, 0.f);
   }
   P::template run_live_tab<false>(v, lds + g * (P::LDS | 1), t, twt, on);
   if (!on) return;
@@ -225,14 +224,18 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_rfield_reg(const float2* Src,
                                                               int k0c, int wc, int lr,
                                                               const float2* __restrict__ twt,
                                                               const float* __restrict__ gamma_in,
-                                                              float* __restrict__ gamma_out) {
-  constexpr int L = P::N, T = P::T, V = P::V, GW = 64 / T;
+                                                              float* __restrict__ gamma_out,
+                                                              int batch) {
+  constexpr int L = P::N, T = P::T, V = P::V, GW = 64 / T, RB = rows_per_block<P>();
   extern __shared__ float2 lds[];
+  const int nxr = (lr + RB - 1) / RB;
+  int w;
+  if (!xcd_item(blockIdx.x, nxr * nk * batch, w)) return;   // uniform over the block
   const int lane = threadIdx.x & 63, gw = lane / T;
   const int t = gw < GW ? lane - gw * T : 0;
   const int g = (threadIdx.x >> 6) * GW + (gw < GW ? gw : 0);
-  const int k = blockIdx.y, b = blockIdx.z;
-  const int r = blockIdx.x * rows_per_block<P>() + g;
+  const int k = (w / nxr) % nk, b = w / (nxr * nk);
+  const int r = w % nxr * RB + g;
   const bool on = gw < GW && r < lr;
   float2* scr = lds + g * P::LDS;
   const size_t at = (((size_t)b * nk + k) * lr + (on ? r : 0)) * wc;
@@ -243,7 +246,9 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_rfield_reg(const float2* Src,
   for (int m = 0; m < V; ++m) {
     int kc = c0 + T * m;
     kc = kc >= L ? kc - L : kc;
-    v[m] = (on && kc < wc) ? src[kc] : make_float2(0.f, 0.f);
+    const bool in = on && kc < wc;
+    const float2 a = src[in ? kc : 0];
+    v[m] = in ? a : make_float2(0.f, 0.f);
   }
   P::template run_live_tab_wave<false>(v, scr, t, twt, on);
   if (!gamma_in) {
@@ -257,7 +262,7 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_rfield_reg(const float2* Src,
   const float* gi = gamma_in + ((size_t)b * lr + (on ? r : 0)) * L;
 #pragma unroll
   for (int m = 0; m < V; ++m) {
-    const float gm = on ? gi[t + T * m] : 0.f;
+    const float gm = gi[t + T * m];   // row 0 for a lane without one
     v[m] = make_float2(gm * v[m].x, -gm * v[m].y);
   }
   P::template run_live_tab_wave<false>(v, scr, t, twt, on);
@@ -293,7 +298,7 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cwin_reg(const float2* __rest
   const float2* pb = Pc + ((size_t)b * nk + k) * L * wc + (on ? kc : 0);
   float2 v[V];
 #pragma unroll
-  for (int m = 0; m < V; ++m) v[m] = on ? pb[(size_t)(t + T * m) * wc] : make_float2(0.f, 0.f);
+  for (int m = 0; m < V; ++m) v[m] = pb[(size_t)(t + T * m) * wc];   // column 0 for a lane without one
   P::template run_live_tab<false>(v, lds + g * (P::LDS | 1), t, twt, on);
   if (!on) return;
   const float2* kb = kern + (size_t)k * wr * wc + kc;
@@ -357,9 +362,10 @@ static int adj_rfield_reg(int L, dim3 grid_y_z, const float2* src, float2* Ec, i
     constexpr int RB = rows_per_block<P>();                                                    \
     int rc = allow_lds_adj(k_adj_rfield_reg<P>, adj_rows_lds<P>());                            \
     if (rc) return rc;                                                                         \
-    dim3 grid((lr + RB - 1) / RB, grid_y_z.y, grid_y_z.z);                                     \
-    hipLaunchKernelGGL(k_adj_rfield_reg<P>, grid, dim3(kRegBlock), adj_rows_lds<P>(), st, src, \
-                       Ec, nk, k0c, wc, lr, twt, gamma_in, gamma_out);                         \
+    const int items = ((lr + RB - 1) / RB) * (int)grid_y_z.y * (int)grid_y_z.z;                \
+    hipLaunchKernelGGL(k_adj_rfield_reg<P>, dim3(xcd_grid(items)), dim3(kRegBlock),            \
+                       adj_rows_lds<P>(), st, src, Ec, nk, k0c, wc, lr, twt, gamma_in,         \
+                       gamma_out, (int)grid_y_z.z);                                            \
     OI_LAUNCH_CHECK("adj_rfield_reg");                                                         \
     return OI_OK;                                                                              \
   }

@@ -651,21 +651,27 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
 //
 // Pass 1: consecutive lanes hold consecutive window columns, so that a load of
 // the kernel, the spectrum or a store to B is a run of G columns (128 bytes at
-// G = 16) and not four of each of sixteen rows.  Bound by the stores of B: 16
-// images x 12 kernels x 105 columns of 256 in 20 us (41 MB; with the exchange
-// inside one wave instead, four columns each, 25 us).
+// G = 16) and not four of each of sixteen rows, and the column blocks of one
+// kernel and image run on one XCD, which then holds the lines that two of them
+// share.  Bound by the stores of B and by arithmetic: 16 images x 12 kernels x
+// 107 columns of 256 in 17 us (42 MB; 20 with the blocks over all XCDs, 25 with
+// the exchange inside one wave, four columns each), 4 x 12 x 214 of 450 in 20
+// (27 with its loads under the window's condition).
 template <class PL>
 __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ spec,
                                                      const float2* __restrict__ kern,
                                                      size_t spec_img, size_t kern_img, int nk,
                                                      int nchan, int k0r, int wr, int wc,
                                                      const float2* __restrict__ twt,
-                                                     float2* __restrict__ B) {
+                                                     float2* __restrict__ B, int batch) {
   constexpr int L = PL::N, TL = PL::T, VL = PL::V, G = groups_per_block<PL>();
   extern __shared__ float2 lds[];
+  const int nxb = (wc + G - 1) / G, nkc = nk * nchan;
+  int w;
+  if (!xcd_item(blockIdx.x, nxb * nkc * batch, w)) return;   // uniform over the block
   const int g = threadIdx.x % G, tg = threadIdx.x / G;
-  const int c = blockIdx.x * G + g;
-  const int kc = blockIdx.y, img = blockIdx.z;        // kc = k * nchan + channel
+  const int c = w % nxb * G + g;
+  const int kc = (w / nxb) % nkc, img = w / (nxb * nkc);   // kc = k * nchan + channel
   const int k = kc / nchan, ch = kc - k * nchan;
   const bool live = tg < TL && c < wc;
   const int t = tg < TL ? tg : 0;
@@ -677,12 +683,17 @@ __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ 
   for (int m = 0; m < VL; ++m) {
     int kr = kr0 + TL * m;
     kr = kr >= L ? kr - L : kr;
-    // rounded product: the adjoint's k_adj_cfield_reg forms the same values
-    v[m] = (live && kr < wr) ? reg::mul_rn(kp[kr * wc + c], sp[kr * wc + c]) : make_float2(0.f, 0.f);
+    // every load at a valid address, what lies outside the window dropped
+    // after it: loads under a condition are waited for one by one.
+    // Rounded product: the adjoint's k_adj_cfield_reg forms the same values
+    const bool in = live && kr < wr;
+    const int at = in ? kr * wc + c : 0;
+    const float2 a = reg::mul_rn(kp[at], sp[at]);
+    v[m] = in ? a : make_float2(0.f, 0.f);
   }
   PL::template run_live_tab<false>(v, lds + g * (PL::LDS | 1), t, twt, live);
   if (!live) return;
-  float2* dst = B + ((size_t)img * nk * nchan + kc) * L * wc + c;
+  float2* dst = B + ((size_t)img * nkc + kc) * L * wc + c;
 #pragma unroll
   for (int m = 0; m < VL; ++m) dst[(size_t)(t + TL * m) * wc] = v[m];
 }
@@ -707,7 +718,8 @@ constexpr int brows_min_blocks() {
 }
 
 // Items (row group, image, kernel group); an item sums the (kernel, channel)
-// pairs kc = grp, grp + groups, ... into its own partial R[img][grp].
+// pairs kc = grp, grp + groups, ... into its own partial R[img][grp].  Images
+// slowest, as pass 1 writes them: an XCD reads what it wrote.
 // A wave is on its own: it loads its rows of B straight into registers (a row
 // is contiguous) and exchanges inside its own part of the LDS, so the loop has
 // no workgroup barrier, where staging a column-major B through an LDS tile took
@@ -729,7 +741,7 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
   constexpr int NXR = (L + RB - 1) / RB;
   int w;
   if (!xcd_item(blockIdx.x, NXR * batch * groups, w)) return;   // uniform over the block
-  const int xr = w % NXR, img = (w / NXR) % batch, grp = w / (NXR * batch);
+  const int xr = w % NXR, grp = (w / NXR) % groups, img = w / (NXR * groups);
   const int lane = threadIdx.x & 63, gw = lane / TL;
   const int t = gw < GW ? lane - gw * TL : 0;
   const int g = (threadIdx.x >> 6) * GW + (gw < GW ? gw : 0);
@@ -757,7 +769,9 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
     for (int m = 0; m < VL; ++m) {
       int cc = c0 + TL * m;
       cc = cc >= L ? cc - L : cc;
-      v[m] = ((rmask >> m) & 1u) ? src[cc] : make_float2(0.f, 0.f);
+      const bool in = (rmask >> m) & 1u;
+      const float2 a = src[in ? cc : 0];
+      v[m] = in ? a : make_float2(0.f, 0.f);
     }
     src += step;
     PL::template run_live_wave<false>(v, scr, t, tw, live);
@@ -1282,9 +1296,9 @@ static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t 
   const size_t lds1 = bcols_lds<PL>();
   int rc = allow(k_fp_bcols<PL>, lds1);
   if (rc) return rc;
-  dim3 g1((a.wc + G - 1) / G, c.nkern * c.nchan, a.batch);
-  hipLaunchKernelGGL(k_fp_bcols<PL>, g1, dim3(kBlock), lds1, st, c.spec, c.kern, c.spec_img,
-                     c.kern_img, c.nkern, c.nchan, a.k0r, a.wr, a.wc, a.tw_l, B);
+  const int cols = ((a.wc + G - 1) / G) * c.nkern * c.nchan * a.batch;
+  hipLaunchKernelGGL(k_fp_bcols<PL>, dim3(xcd_grid(cols)), dim3(kBlock), lds1, st, c.spec, c.kern,
+                     c.spec_img, c.kern_img, c.nkern, c.nchan, a.k0r, a.wr, a.wc, a.tw_l, B, a.batch);
   OI_LAUNCH_CHECK("fp_bcols");
   const size_t lds2 = two_pass_rows_lds<PL>();
   rc = allow(k_fp_brows<PL>, lds2);

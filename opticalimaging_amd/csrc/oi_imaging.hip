@@ -575,9 +575,14 @@ extern "C" int oi_kernel_dense(const void* win, int nk, int k0r, int wr, int k0c
 }
 
 // ------------------------------------------------------------ coded masks --
+// Bound by the stores: consecutive lanes write consecutive 16 bytes, and a
+// thread has the loads of kDecode such pieces in flight before its first store.
+// (Sixteen or thirty-two pixels in a row per thread, each store of a wave spread
+// over 4 or 8 KB: bits of 16.8 million pixels took 23 us, 12 so.)
 // Masks sent as one byte per pixel: out[i] = levels[codes[i]] (codes past the
-// table give 0).  Sixteen codes per thread and iteration (one 16-byte load,
-// four 16-byte stores); the table sits in LDS.
+// table give 0); the table sits in LDS.
+constexpr int kDecode = 8;   // float4 per thread
+
 namespace {
 struct Levels {
   float v[256];
@@ -588,46 +593,61 @@ __global__ __launch_bounds__(256) void k_decode_u8(const uint8_t* __restrict__ c
   __shared__ float lut[256];
   lut[threadIdx.x] = (int)threadIdx.x < nl ? lv.v[threadIdx.x] : 0.f;
   __syncthreads();
-  const size_t n16 = n / 16;
-  const uint4* c16 = reinterpret_cast<const uint4*>(codes);
+  const size_t n4 = n / 4;
+  const uint32_t* c4 = reinterpret_cast<const uint32_t*>(codes);
   float4* o4 = reinterpret_cast<float4*>(out);
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) {
-    const uint4 c = c16[i];
-    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+  const size_t first = (size_t)blockIdx.x * (kDecode * 256) + threadIdx.x;
+  uint32_t w[kDecode];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      o4[4 * i + q] = make_float4(lut[w[q] & 0xff], lut[(w[q] >> 8) & 0xff], lut[(w[q] >> 16) & 0xff],
-                                  lut[w[q] >> 24]);
+  for (int k = 0; k < kDecode; ++k) {
+    const size_t i = first + k * 256;
+    w[k] = i < n4 ? c4[i] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kDecode; ++k) {
+    const size_t i = first + k * 256;
+    if (i < n4)
+      o4[i] = make_float4(lut[w[k] & 0xff], lut[(w[k] >> 8) & 0xff], lut[(w[k] >> 16) & 0xff],
+                          lut[w[k] >> 24]);
   }
   if (blockIdx.x == 0) {
-    for (size_t i = n16 * 16 + threadIdx.x; i < n; i += blockDim.x) out[i] = lut[codes[i]];
+    for (size_t i = n4 * 4 + threadIdx.x; i < n; i += blockDim.x) out[i] = lut[codes[i]];
   }
 }
 
-// One bit per pixel: each thread expands 4 bytes (32 pixels, bit 7 of a byte
-// first) into eight 16-byte stores.
+// One bit per pixel, bit 7 of a byte first: eight lanes expand one 4-byte word.
 __global__ __launch_bounds__(256) void k_decode_bits(const uint8_t* __restrict__ bits, size_t n,
                                                      float v0, float v1, float* __restrict__ out) {
-  const size_t n32 = n / 32;
+  const size_t n32 = n / 32, n4 = n32 * 8;
   const uint32_t* b4 = reinterpret_cast<const uint32_t*>(bits);
   float4* o4 = reinterpret_cast<float4*>(out);
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n32; i += stride) {
-    const uint32_t w = b4[i];
+  const size_t first = (size_t)blockIdx.x * (kDecode * 256) + threadIdx.x;
+  // the word's byte (little-endian: byte order kept) and its half, the same for
+  // every piece of a thread
+  const int shift = 8 * ((threadIdx.x >> 1) & 3) + 4 * (1 - (threadIdx.x & 1));
+  uint32_t w[kDecode];
 #pragma unroll
-    for (int byte = 0; byte < 4; ++byte) {
-      const uint32_t c = (w >> (8 * byte)) & 0xffu;     // little-endian words: byte order kept
-      o4[8 * i + 2 * byte] = make_float4((c & 0x80u) ? v1 : v0, (c & 0x40u) ? v1 : v0,
-                                         (c & 0x20u) ? v1 : v0, (c & 0x10u) ? v1 : v0);
-      o4[8 * i + 2 * byte + 1] = make_float4((c & 0x08u) ? v1 : v0, (c & 0x04u) ? v1 : v0,
-                                             (c & 0x02u) ? v1 : v0, (c & 0x01u) ? v1 : v0);
-    }
+  for (int k = 0; k < kDecode; ++k) {
+    const size_t i = first + k * 256;
+    w[k] = i < n4 ? b4[i >> 3] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kDecode; ++k) {
+    const size_t i = first + k * 256;
+    const uint32_t c = w[k] >> shift;
+    if (i < n4)
+      o4[i] = make_float4((c & 8u) ? v1 : v0, (c & 4u) ? v1 : v0, (c & 2u) ? v1 : v0, (c & 1u) ? v1 : v0);
   }
   if (blockIdx.x == 0) {
     for (size_t i = n32 * 32 + threadIdx.x; i < n; i += blockDim.x)
       out[i] = ((bits[i >> 3] >> (7 - (i & 7))) & 1u) ? v1 : v0;
   }
+}
+
+// Workgroups for count pixels, 0 past the grid's limit.
+unsigned decode_blocks(size_t count) {
+  const size_t per = 4 * kDecode * 256, blocks = (count + per - 1) / per;
+  return blocks > 0x7fffffffu ? 0 : (unsigned)blocks;
 }
 }  // namespace
 
@@ -637,11 +657,9 @@ extern "C" int oi_mask_decode_bits(const void* bits, size_t count, const float* 
   if ((reinterpret_cast<uintptr_t>(bits) & 3) || (reinterpret_cast<uintptr_t>(out) & 15))
     return fail(OI_ERR_INVALID, "mask_decode_bits: bits must be 4-byte and out 16-byte aligned");
   if (count == 0) return OI_OK;
-  const size_t n32 = count / 32;
-  size_t blocks = (n32 + 255) / 256;
-  if (blocks < 1) blocks = 1;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(k_decode_bits, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
+  const unsigned blocks = decode_blocks(count);
+  if (!blocks) return fail(OI_ERR_INVALID, "mask_decode_bits: too many pixels");
+  hipLaunchKernelGGL(k_decode_bits, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
                      static_cast<const uint8_t*>(bits), count, levels[0], levels[1], out);
   OI_LAUNCH_CHECK("mask_decode_bits");
   return OI_OK;
@@ -656,11 +674,9 @@ extern "C" int oi_mask_decode_u8(const void* codes, size_t count, const float* l
   if (count == 0) return OI_OK;
   Levels lv;
   for (int i = 0; i < 256; ++i) lv.v[i] = i < nlevels ? levels[i] : 0.f;
-  const size_t n16 = count / 16;
-  size_t blocks = (n16 + 255) / 256;
-  if (blocks < 1) blocks = 1;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(k_decode_u8, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
+  const unsigned blocks = decode_blocks(count);
+  if (!blocks) return fail(OI_ERR_INVALID, "mask_decode_u8: too many pixels");
+  hipLaunchKernelGGL(k_decode_u8, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
                      static_cast<const uint8_t*>(codes), count, lv, nlevels, out);
   OI_LAUNCH_CHECK("mask_decode_u8");
   return OI_OK;

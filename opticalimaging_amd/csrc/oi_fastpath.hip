@@ -292,23 +292,25 @@ template <class P>
 __global__ __launch_bounds__(kBlock) void k_fp_rows_c64(const float2* __restrict__ field, int cin,
                                                         Chans ch, int nchan, int ny, int k0c,
                                                         int wc, const float2* __restrict__ twt,
-                                                        float2* __restrict__ T) {
+                                                        float2* __restrict__ T, int batch) {
   constexpr int N = P::N, TT = P::T, V = P::V, G = groups_per_block<P>();
   extern __shared__ float2 lds[];
+  // channels fastest, in XCD order: the channels of a pixel share its lines
+  const int nrb = (ny + G - 1) / G;
+  int w;
+  if (!xcd_item(blockIdx.x, nrb * nchan * batch, w)) return;   // uniform over the block
+  const int ci = w % nchan, xb = (w / nchan) % nrb, img = w / (nchan * nrb);
   const int g = threadIdx.x / TT, t = threadIdx.x - g * TT;
   const bool live = g < G;
   const int gg = live ? g : 0;
   float2* scr = lds + g * P::LDS;
-  const int bc = blockIdx.y;
-  const int img = bc / nchan, ci = bc - img * nchan;
   const int chan = ch.c[ci];
-  const int r = blockIdx.x * G + gg;
+  const int r = xb * G + gg;
+  // row 0 for a group without one: its values are not stored
+  const float2* src = field + ((size_t)img * ny + (r < ny ? r : 0)) * N * cin + chan;
   float2 v[V];
 #pragma unroll
-  for (int m = 0; m < V; ++m) {
-    const int x = t + TT * m;
-    v[m] = (live && r < ny) ? field[(((size_t)img * ny + r) * N + x) * cin + chan] : make_float2(0.f, 0.f);
-  }
+  for (int m = 0; m < V; ++m) v[m] = src[(size_t)(t + TT * m) * cin];
   P::template run_live_tab<true>(v, scr, t, twt, true);
   if (live) {
 #pragma unroll
@@ -320,8 +322,8 @@ __global__ __launch_bounds__(kBlock) void k_fp_rows_c64(const float2* __restrict
   if (live && r < ny)
     for (int j = t; j < wc; j += TT) tile[j * TS + gg] = scr[pad(pmod(k0c + j, N))];
   __syncthreads();
-  const int rb = blockIdx.x * G;
-  float2* Tb = T + (size_t)bc * wc * ny;
+  const int rb = xb * G;
+  float2* Tb = T + ((size_t)img * nchan + ci) * wc * ny;
   for (int e = threadIdx.x; e < wc * G; e += kBlock) {
     const int j = e / G, rr = e - j * G;
     if (rb + rr < ny) Tb[(size_t)j * ny + rb + rr] = tile[j * TS + rr];
@@ -1141,12 +1143,15 @@ static int run_rows(const FpArgs& a, hipStream_t st) {
                        static_cast<const float*>(a.field), a.ny, a.k0c, a.wc, a.tw_x, a.T,
                        (int)(a.kind == kFieldLogits));
   } else {
-    int rc = allow(k_fp_rows_c64<P>, lds);
+    // its tile is [wc][G + 1]: at 512 points and windows up to 90 columns two
+    // workgroups share a CU instead of one
+    const size_t lds_c = rows_lds<P>() + (size_t)a.wc * (G + 1) * sizeof(float2);
+    int rc = allow(k_fp_rows_c64<P>, lds_c);
     if (rc) return rc;
-    dim3 grid((a.ny + G - 1) / G, a.batch * a.nchan);
-    hipLaunchKernelGGL(k_fp_rows_c64<P>, grid, dim3(kBlock), lds, st,
+    const int items = (a.ny + G - 1) / G * a.nchan * a.batch;
+    hipLaunchKernelGGL(k_fp_rows_c64<P>, dim3(xcd_grid(items)), dim3(kBlock), lds_c, st,
                        static_cast<const float2*>(a.field), a.cin, a.chans, a.nchan, a.ny, a.k0c,
-                       a.wc, a.tw_x, a.T);
+                       a.wc, a.tw_x, a.T, a.batch);
   }
   OI_LAUNCH_CHECK("fp_rows");
   return OI_OK;

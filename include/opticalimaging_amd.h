@@ -152,6 +152,33 @@ int oi_spectrum_window(oi_plan* plan, const void* field, int kind, int cin,
 int oi_coherent_image(oi_plan* plan, const void* spec, int batch,
                       const void* kern, int nkern, float* out, void* stream);
 
+/* Weighted kernels of the Abbe image as a function of its source weights:
+ * K[z][s][e] = G[z][s][e] sqrt(index_image V_s / sum V), G the unit-weight
+ * shifted pupils (CalculateAerialImage.py:46-92 applies the same weights).
+ *   G, K : c64 [nfoci][nsrc][ncomp][wr][wc];  V : float64 [nsrc]              */
+int oi_source_kernels(const void* G, const double* V, int nfoci, int nsrc, int ncomp,
+                      int wr, int wc, double index_image, void* K, void* stream);
+
+/* Kt[y][t] = (1/n) sum_{|q| <= band} cos(2 pi q (t/lr - y/n)): the resampling of
+ * oi_source_gradient along one axis (n, lr <= 2^24, band <= 4096).
+ *   Kt : float64 [n][lr]                                                      */
+int oi_source_resampling(int n, int lr, int band, double* Kt, void* stream);
+
+/* Gradient of a loss with respect to the source weights of the Abbe image
+ * I = (n / W) sum_s V_s J_s at one focus, from the image cotangent g:
+ *   out[s] (add: +=) (n / W) (ny nx / (lr lc)) sum_t J[s][t] gamma[t] - <g, I> / W,
+ *   gamma[tr][tc] = sum_{y,x} Ktr[y][tr] Ktc[x][tc] g[y][x],
+ * with W = sum V.  Ktr (Ktc) null: that axis is not resampled, lr = ny (lc = nx).
+ * No counterpart in the reference (it would differentiate its image loop).
+ *   grad_image, image : float32 [ny][nx];  Ktr, Ktc : float64 [ny][lr], [nx][lc]
+ *   J : float32 [nsrc][lr][lc];  V, out : float64 [nsrc]
+ *   work : oi_source_gradient_work_bytes(nx, lr, lc) bytes of device memory   */
+size_t oi_source_gradient_work_bytes(int nx, int lr, int lc);
+int oi_source_gradient(const float* grad_image, const float* image, int ny, int nx,
+                       const double* Ktr, int lr, const double* Ktc, int lc, const float* J,
+                       int nsrc, const double* V, double index_image, int add, void* work,
+                       double* out, void* stream);
+
 /* PupilImage of Scatter.CalculateSpectrum (Scatter.py:25-35) from a windowed
  * spectrum: out[i][j][c], c < cin, is Hk at row index i - oy and column index
  * j - ox,

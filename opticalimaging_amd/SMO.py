@@ -20,8 +20,8 @@ exactly.  All J_s^L come from one oi_coherent_image call on a direct L x L
 plan with the roles of spectrum and kernels exchanged: the unit-weight
 shifted pupils of the points are the "spectra" of a batch of Nsrc images with
 one channel per polarisation component, and the field's windowed spectrum
-(one kernel per field channel) is the "kernel set".  gamma comes from a
-float64 FFT of g on the device.
+(one kernel per field channel) is the "kernel set".  gamma and the sums against
+it are float64 products and reductions on the device (oi_source_gradient).
 
 ``AbbeSourceImage`` wraps this as a torch.autograd.Function of V;
 ``abbe_source_problem`` sets up a fixed field and optics.  The reference has
@@ -29,8 +29,6 @@ no source gradient (it would differentiate its complex64 loop with torch
 autograd); the float64 gradient of the oracle's I(V) pins this one.
 """
 from __future__ import annotations
-
-import math
 
 import torch
 
@@ -52,6 +50,16 @@ def _smooth_at_least(n: int) -> int:
         if k == 1 and m % 2 == 0:
             return m
         m += 1
+
+
+def _resampling(n: int, L: int, B: int, dev) -> torch.Tensor | None:
+    """Kt[y][t] = (1/n) sum_{|q| <= B} cos(2 pi q (t/L - y/n)): the band |q| <= B
+    of n samples on L points, or None where the axis keeps its points."""
+    if n == L:
+        return None
+    Kt = torch.empty((n, L), dtype=torch.float64, device=dev)
+    nat.check(nat.load().oi_source_resampling(n, L, B, nat.ptr(Kt), nat.stream()))
+    return Kt
 
 
 class AbbeSourceProblem:
@@ -84,13 +92,15 @@ class AbbeSourceProblem:
         nat.check(lib.oi_spectrum_window(self.plan.handle, nat.ptr(tens), kind, cin, cptr, 1,
                                          nat.ptr(self.spec), nat.stream()))
         del keep
-        # unit-weight shifted pupils per focus, c64 [ncomp][nsrc][wr][wc]
+        # unit-weight shifted pupils per focus, c64 [nsrc][ncomp][wr][wc]: a
+        # point's components together, as point_intensities takes them
         ones = torch.ones(nsrc, dtype=torch.float64, device=self.dev)
         self.foci = optics.focus_values(projector)
         self.G = []
         for z in self.foci:
             opt = optics.optics_record(source, projector, z, py, px, self.vector)
-            self.G.append(optics.pupil_kernels(self.src, opt, ones, k0r, wr, k0c, wc))
+            G = optics.pupil_kernels(self.src, opt, ones, k0r, wr, k0c, wc)
+            self.G.append(G.permute(1, 0, 2, 3).contiguous())
         # coarse grid of the per-point intensities: holds the window and
         # twice a pupil's band
         need = max(2 * max(br, bc) - 1, 2 * max(-k0r, k0r + wr - 1, -k0c, k0c + wc - 1) + 2)
@@ -101,6 +111,8 @@ class AbbeSourceProblem:
                                  band_r=wr, band_c=wc, lr=self.Lr, lc=self.Lc, max_kernels=self.C)
         if not self.cplan.geo.direct:
             raise RuntimeError("per-point intensity plan is not direct")
+        self.Kr = _resampling(self.ny, self.Lr, br - 1, self.dev)
+        self.Kc = _resampling(self.nx, self.Lc, bc - 1, self.dev)
 
     @property
     def nsrc(self) -> int:
@@ -108,54 +120,49 @@ class AbbeSourceProblem:
 
     def image(self, V: torch.Tensor) -> torch.Tensor:
         """Abbe intensities (nFocus, ny, nx) float32 for weights V (nsrc,)."""
-        V = V.detach().to(self.dev, torch.float64)
-        scale = torch.sqrt(self.n_index * V / V.sum()).to(torch.float32)
+        V = self._weights(V)
         lib = nat.load()
         out = torch.empty((len(self.foci), self.ny, self.nx), dtype=torch.float32, device=self.dev)
         for i, G in enumerate(self.G):
-            K = (G * scale[None, :, None, None]).contiguous()
+            K = torch.empty_like(G)
+            nat.check(lib.oi_source_kernels(nat.ptr(G), nat.ptr(V), 1, self.nsrc, self.ncomp,
+                                            G.shape[2], G.shape[3], self.n_index, nat.ptr(K),
+                                            nat.stream()))
             nat.check(lib.oi_coherent_image(self.plan.handle, nat.ptr(self.spec), 1, nat.ptr(K),
                                             K.shape[0] * K.shape[1], nat.ptr(out[i]), nat.stream()))
         return out
 
+    def _weights(self, V: torch.Tensor) -> torch.Tensor:
+        V = V.detach().to(self.dev, torch.float64).contiguous()
+        if V.shape != (self.nsrc,):
+            raise ValueError(f"V must hold {self.nsrc} source weights")
+        return V
+
     def point_intensities(self, focus_index: int) -> torch.Tensor:
         """J_s on the coarse Lr x Lc grid, float32 (nsrc, Lr, Lc)."""
-        G = self.G[focus_index]
-        pupils = G.permute(1, 0, 2, 3).contiguous()          # [nsrc][ncomp][wr][wc]
-        kern = self.spec[0].contiguous()                      # [C][wr][wc]
         out = torch.empty((self.nsrc, self.Lr, self.Lc), dtype=torch.float32, device=self.dev)
-        nat.check(nat.load().oi_coherent_image(self.cplan.handle, nat.ptr(pupils), self.nsrc,
-                                               nat.ptr(kern), self.C, nat.ptr(out), nat.stream()))
+        nat.check(nat.load().oi_coherent_image(self.cplan.handle, nat.ptr(self.G[focus_index]),
+                                               self.nsrc, nat.ptr(self.spec), self.C, nat.ptr(out),
+                                               nat.stream()))
         return out
-
-    def _gamma(self, g: torch.Tensor) -> torch.Tensor:
-        """Band |q| <= band - 1 of g (ny, nx) resampled to the Lr x Lc grid."""
-        ny, nx, Lr, Lc = self.ny, self.nx, self.Lr, self.Lc
-        if (Lr, Lc) == (ny, nx):
-            return g.to(torch.float64)
-        gh = torch.fft.fft2(g.to(torch.float64)) / (ny * nx)
-        Br, Bc = self.band[0] - 1, self.band[1] - 1
-        qr = torch.arange(-Br, Br + 1, device=self.dev)
-        qc = torch.arange(-Bc, Bc + 1, device=self.dev)
-        sub = gh[qr.remainder(ny)][:, qc.remainder(nx)]
-        gl = torch.zeros((Lr, Lc), dtype=torch.complex128, device=self.dev)
-        gl[qr.remainder(Lr)[:, None], qc.remainder(Lc)[None, :]] = sub
-        return (torch.fft.ifft2(gl) * (Lr * Lc)).real
 
     def source_gradient(self, V: torch.Tensor, grad_image: torch.Tensor) -> torch.Tensor:
         """dL/dV (float64, nsrc) for image cotangents grad_image (nFocus, ny, nx)."""
-        V = V.detach().to(self.dev, torch.float64)
-        W = float(V.sum())
-        g = grad_image.detach().to(self.dev, torch.float32)
+        V = self._weights(V)
+        g = grad_image.detach().to(self.dev, torch.float32).contiguous()
+        if g.shape != (len(self.foci), self.ny, self.nx):
+            raise ValueError("grad_image must have the image's shape")
         img = self.image(V)
-        scale = (self.ny * self.nx) / (self.Lr * self.Lc)
-        out = torch.zeros(self.nsrc, dtype=torch.float64, device=self.dev)
+        lib = nat.load()
+        out = torch.empty(self.nsrc, dtype=torch.float64, device=self.dev)
+        work = torch.empty(int(lib.oi_source_gradient_work_bytes(self.nx, self.Lr, self.Lc)),
+                           dtype=torch.uint8, device=self.dev)
         for i in range(len(self.foci)):
-            gam = self._gamma(g[i])
-            J = self.point_intensities(i).to(torch.float64)
-            gJ = scale * (J.reshape(self.nsrc, -1) @ gam.reshape(-1))
-            gI = float((g[i].double() * img[i].double()).sum())
-            out += self.n_index / W * gJ - gI / W
+            J = self.point_intensities(i)
+            nat.check(lib.oi_source_gradient(nat.ptr(g[i]), nat.ptr(img[i]), self.ny, self.nx,
+                                             nat.ptr(self.Kr), self.Lr, nat.ptr(self.Kc), self.Lc,
+                                             nat.ptr(J), self.nsrc, nat.ptr(V), self.n_index,
+                                             int(i > 0), nat.ptr(work), nat.ptr(out), nat.stream()))
         return out
 
 

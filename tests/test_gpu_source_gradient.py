@@ -1,0 +1,68 @@
+"""oi_source_kernels and oi_source_gradient against the same sums in torch
+float64 on the CPU: part-filled tiles of 64 columns and 8 outputs, axes that are
+resampled and axes that keep their points, accumulation over foci.  float64 sums
+in another order: 1e-12 of the sum of magnitudes."""
+import math
+
+import pytest
+import torch
+
+from opticalimaging_amd import _native as nat
+from opticalimaging_amd.SMO import _resampling
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(128, 128, 20, 20, 9, 120), (64, 65, 64, 9, 4, 3), (65, 64, 7, 64, 3, 257), (40, 72, 40, 72, 1, 5),
+         (256, 130, 33, 47, 16, 1), (1, 200, 1, 8, 3, 2)]
+
+
+@pytest.mark.parametrize("ny,nx,lr,lc,B,nsrc", CASES)
+def test_gradient(gpu, ny, nx, lr, lc, B, nsrc):
+    lib, gen = nat.load(), torch.Generator().manual_seed(ny + nx)
+    g, img = (torch.randn((2, ny, nx), generator=gen) for _ in range(2))
+    J = torch.rand((2, nsrc, lr, lc), generator=gen)
+    V = torch.rand(nsrc, dtype=torch.float64, generator=gen) + 0.1
+    Kr, Kc = _resampling(ny, lr, min(B, lr // 2), "cuda"), _resampling(nx, lc, min(B, lc // 2), "cuda")
+    ref, size = torch.zeros(nsrc, dtype=torch.float64), 0.0
+    for i in range(2):
+        gam = g[i].double()
+        gam = gam if Kr is None else Kr.cpu().T @ gam
+        gam = gam if Kc is None else gam @ Kc.cpu()
+        s = (ny * nx) / (lr * lc)
+        ref += 1.44 / V.sum() * s * (J[i].double() * gam).sum((1, 2)) - (g[i].double() * img[i].double()).sum() / V.sum()
+        size = max(size, float((J[i].double() * gam.abs()).sum((1, 2)).max()) * s + float((g[i] * img[i]).abs().sum()))
+    dev = [None if t is None else t.cuda() for t in (g, img, J, V, Kr, Kc)]
+    g, img, J, Vd, Kr, Kc = dev
+    out = torch.full((nsrc,), float("nan"), dtype=torch.float64, device="cuda")
+    work = torch.empty(int(lib.oi_source_gradient_work_bytes(nx, lr, lc)), dtype=torch.uint8, device="cuda")
+    for i in range(2):
+        nat.check(lib.oi_source_gradient(nat.ptr(g[i]), nat.ptr(img[i]), ny, nx, nat.ptr(Kr), lr, nat.ptr(Kc),
+                                         lc, nat.ptr(J[i]), nsrc, nat.ptr(Vd), 1.44, i, nat.ptr(work),
+                                         nat.ptr(out), nat.stream()))
+    assert (out.cpu() - ref).abs().max() <= 1e-12 * 2 * size / float(V.sum())
+
+
+@pytest.mark.parametrize("ny,L,B", [(128, 20, 9), (96, 25, 12), (81, 80, 30), (1024, 250, 124)])
+def test_resampling_table(gpu, ny, L, B):
+    """Band-limited samples of n points go to L points exactly (n 1e-15 each)."""
+    Kt = _resampling(ny, L, B, torch.device("cuda")).cpu()
+    y, t = torch.arange(ny).double() / ny, torch.arange(L).double() / L
+    for q in (0, 1, B - 1, B):
+        f = lambda x: torch.cos(2 * math.pi * q * x + 0.3)  # noqa: E731
+        assert (Kt.T @ f(y) - f(t)).abs().max() < 1e-15 * 4 * ny
+    q = min(B + 1, (ny - 1) // 2)
+    if q > B:
+        assert (Kt.T @ torch.cos(2 * math.pi * q * y)).abs().max() < 1e-15 * 4 * ny
+
+
+@pytest.mark.parametrize("nsrc,ncomp,wr,wc", [(1, 1, 3, 5), (120, 1, 22, 22), (196, 3, 35, 33)])
+def test_kernels(gpu, nsrc, ncomp, wr, wc):
+    gen = torch.Generator().manual_seed(nsrc)
+    G = torch.randn((2, nsrc, ncomp, wr, wc), dtype=torch.complex64, generator=gen)
+    V = torch.rand(nsrc, dtype=torch.float64, generator=gen)
+    Gd, Vd = G.cuda(), V.cuda()
+    K = torch.empty_like(Gd)
+    nat.check(nat.load().oi_source_kernels(nat.ptr(Gd), nat.ptr(Vd), 2, nsrc, ncomp, wr, wc, 1.44, nat.ptr(K),
+                                           nat.stream()))
+    ref = G * torch.sqrt(1.44 * V / V.sum()).to(torch.float32)[None, :, None, None, None]
+    assert ((K.cpu() - ref).abs() <= 2.0 ** -22 * ref.abs()).all()     # two float32 roundings each

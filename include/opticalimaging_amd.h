@@ -153,11 +153,12 @@ int oi_coherent_image(oi_plan* plan, const void* spec, int batch,
                       const void* kern, int nkern, float* out, void* stream);
 
 /* Weighted kernels of the Abbe image as a function of its source weights:
- * K[z][s][e] = G[z][s][e] sqrt(index_image V_s / sum V), G the unit-weight
- * shifted pupils (CalculateAerialImage.py:46-92 applies the same weights).
- *   G, K : c64 [nfoci][nsrc][ncomp][wr][wc];  V : float64 [nsrc]              */
-int oi_source_kernels(const void* G, const double* V, int nfoci, int nsrc, int ncomp,
-                      int wr, int wc, double index_image, void* K, void* stream);
+ * K[e][s] = G[s][e] sqrt(index_image V_s / sum V), G the unit-weight shifted
+ * pupils (CalculateAerialImage.py:46-92 applies the same weights).
+ *   G : c64 [nsrc][ncomp][wr][wc];  K : c64 [ncomp][nsrc][wr][wc]
+ *   V : float64 [nsrc]                                                        */
+int oi_source_kernels(const void* G, const double* V, int nsrc, int ncomp, int wr, int wc,
+                      double index_image, void* K, void* stream);
 
 /* Kt[y][t] = (1/n) sum_{|q| <= band} cos(2 pi q (t/lr - y/n)): the resampling of
  * oi_source_gradient along one axis (n, lr <= 2^24, band <= 4096).

@@ -52,6 +52,19 @@ def _smooth_at_least(n: int) -> int:
         m += 1
 
 
+# image lengths with register transforms (csrc/oi_fastpath.hip)
+_REGISTER_LENGTHS = {128, 256, 512, 1024, 2048}
+
+
+def _coarse(need: int, n: int) -> int:
+    """The library's coarse size for a band: the smallest 2,3,5-smooth multiple
+    of 8 that is >= need, n when that reaches n."""
+    m = _smooth_at_least(max(need, 8))
+    while m % 8 and m < n:
+        m = _smooth_at_least(m + 1)
+    return min(m, n)
+
+
 def _resampling(n: int, L: int, B: int, dev) -> torch.Tensor | None:
     """Kt[y][t] = (1/n) sum_{|q| <= B} cos(2 pi q (t/L - y/n)): the band |q| <= B
     of n samples on L points, or None where the axis keeps its points."""
@@ -84,8 +97,14 @@ class AbbeSourceProblem:
         tens, kind, cin, live = engine.field_encoding(h)
         self.C = len(live)
         nsrc = self.src.n
+        # The float64 gradient takes <g, I> from this float32 image: image lengths
+        # without register transforms keep the general kernels (a coarse grid of
+        # the caller's choice) and with them the rounding of that term.
+        lr = lc = 0
+        if not {self.ny, self.nx} <= _REGISTER_LENGTHS:
+            lr, lc = _coarse(2 * br - 1, self.ny), _coarse(2 * bc - 1, self.nx)
         self.plan = engine.Plan(self.ny, self.nx, k0r, wr, k0c, wc, nchan=self.C, max_batch=1,
-                                band_r=br, band_c=bc, max_kernels=self.ncomp * nsrc)
+                                band_r=br, band_c=bc, lr=lr, lc=lc, max_kernels=self.ncomp * nsrc)
         lib = nat.load()
         self.spec = torch.empty((1, self.C, wr, wc), dtype=torch.complex64, device=self.dev)
         cptr, keep = nat.int_array(live)
@@ -124,8 +143,8 @@ class AbbeSourceProblem:
         lib = nat.load()
         out = torch.empty((len(self.foci), self.ny, self.nx), dtype=torch.float32, device=self.dev)
         for i, G in enumerate(self.G):
-            K = torch.empty_like(G)
-            nat.check(lib.oi_source_kernels(nat.ptr(G), nat.ptr(V), 1, self.nsrc, self.ncomp,
+            K = torch.empty_like(G)                           # [ncomp][nsrc][wr][wc]
+            nat.check(lib.oi_source_kernels(nat.ptr(G), nat.ptr(V), self.nsrc, self.ncomp,
                                             G.shape[2], G.shape[3], self.n_index, nat.ptr(K),
                                             nat.stream()))
             nat.check(lib.oi_coherent_image(self.plan.handle, nat.ptr(self.spec), 1, nat.ptr(K),

@@ -84,8 +84,8 @@ SIGNATURES = {
                                     c_void_p, c_void_p]),
     "oi_pupil_kernels": (c_int, [ctypes.POINTER(Optics), c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
-    "oi_source_kernels": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_double,
-                                  c_void_p, c_void_p]),
+    "oi_source_kernels": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_double, c_void_p,
+                                  c_void_p]),
     "oi_source_resampling": (c_int, [c_int, c_int, c_int, c_void_p, c_void_p]),
     "oi_source_gradient_work_bytes": (c_size_t, [c_int, c_int, c_int]),
     "oi_source_gradient": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int,

@@ -40,17 +40,19 @@ __device__ __forceinline__ double weight_sum(const double* __restrict__ V, int n
   return block_sum(w, red);
 }
 
-// K[s][e][i] = G[s][e][i] sqrt(n V_s / W); one source point per blockIdx.y
+// K[e][s][i] = G[s][e][i] sqrt(n V_s / W); point s = blockIdx.y, component e =
+// blockIdx.z.
 __global__ __launch_bounds__(kT) void k_smo_kernels(const float2* __restrict__ G,
                                                     const double* __restrict__ V, int nsrc,
-                                                    size_t per, double n, float2* __restrict__ K) {
+                                                    int per, double n, float2* __restrict__ K) {
   __shared__ double red[kT / 64];
   const double W = weight_sum(V, nsrc, red);
+  const int e = blockIdx.z, ncomp = gridDim.z;
   for (int s = blockIdx.y; s < nsrc; s += gridDim.y) {
     const float c = (float)sqrt(n * V[s] / W);
-    const float2* src = G + ((size_t)blockIdx.z * nsrc + s) * per;
-    float2* dst = K + ((size_t)blockIdx.z * nsrc + s) * per;
-    for (size_t i = (size_t)blockIdx.x * kT + threadIdx.x; i < per; i += (size_t)gridDim.x * kT) {
+    const float2* src = G + ((size_t)s * ncomp + e) * per;
+    float2* dst = K + ((size_t)e * nsrc + s) * per;
+    for (int i = blockIdx.x * kT + threadIdx.x; i < per; i += gridDim.x * kT) {
       const float2 v = src[i];
       dst[i] = make_float2(v.x * c, v.y * c);
     }
@@ -167,13 +169,13 @@ extern "C" int oi_source_resampling(int n, int lr, int band, double* Kt, void* s
   return OI_OK;
 }
 
-extern "C" int oi_source_kernels(const void* G, const double* V, int nfoci, int nsrc, int ncomp,
-                                 int wr, int wc, double index_image, void* K, void* stream) {
-  if (!G || !V || !K || nfoci < 1 || nfoci > 65535 || nsrc < 1 || ncomp < 1 || wr < 1 || wc < 1)
+extern "C" int oi_source_kernels(const void* G, const double* V, int nsrc, int ncomp, int wr, int wc,
+                                 double index_image, void* K, void* stream) {
+  if (!G || !V || !K || nsrc < 1 || ncomp < 1 || ncomp > 65535 || wr < 1 || wc < 1 ||
+      (size_t)wr * wc > 0x40000000u)
     return fail(OI_ERR_INVALID, "source_kernels: bad arguments");
-  const size_t per = (size_t)ncomp * wr * wc;
-  const size_t bx = (per + 4 * kT - 1) / (4 * kT);
-  const dim3 grid((unsigned)(bx < 1024 ? bx : 1024), (unsigned)(nsrc < 65535 ? nsrc : 65535), nfoci);
+  const int per = wr * wc, bx = (per + 4 * kT - 1) / (4 * kT);
+  const dim3 grid(bx < 1024 ? bx : 1024, nsrc < 65535 ? nsrc : 65535, ncomp);
   hipLaunchKernelGGL(k_smo_kernels, grid, dim3(kT), 0, (hipStream_t)stream,
                      static_cast<const float2*>(G), V, nsrc, per, index_image, static_cast<float2*>(K));
   OI_LAUNCH_CHECK("source_kernels");

@@ -58,11 +58,11 @@ def test_resampling_table(gpu, ny, L, B):
 @pytest.mark.parametrize("nsrc,ncomp,wr,wc", [(1, 1, 3, 5), (120, 1, 22, 22), (196, 3, 35, 33)])
 def test_kernels(gpu, nsrc, ncomp, wr, wc):
     gen = torch.Generator().manual_seed(nsrc)
-    G = torch.randn((2, nsrc, ncomp, wr, wc), dtype=torch.complex64, generator=gen)
+    G = torch.randn((nsrc, ncomp, wr, wc), dtype=torch.complex64, generator=gen)
     V = torch.rand(nsrc, dtype=torch.float64, generator=gen)
     Gd, Vd = G.cuda(), V.cuda()
-    K = torch.empty_like(Gd)
-    nat.check(nat.load().oi_source_kernels(nat.ptr(Gd), nat.ptr(Vd), 2, nsrc, ncomp, wr, wc, 1.44, nat.ptr(K),
+    K = torch.empty((ncomp, nsrc, wr, wc), dtype=torch.complex64, device="cuda")
+    nat.check(nat.load().oi_source_kernels(nat.ptr(Gd), nat.ptr(Vd), nsrc, ncomp, wr, wc, 1.44, nat.ptr(K),
                                            nat.stream()))
-    ref = G * torch.sqrt(1.44 * V / V.sum()).to(torch.float32)[None, :, None, None, None]
+    ref = (G * torch.sqrt(1.44 * V / V.sum()).to(torch.float32)[:, None, None, None]).transpose(0, 1)
     assert ((K.cpu() - ref).abs() <= 2.0 ** -22 * ref.abs()).all()     # two float32 roundings each

@@ -314,8 +314,9 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cwin_reg(const float2* __rest
 // dividing the larger), as the fast imaging path's coarse grids.
 #define OI_ADJ_PLANS(X)                                                                        \
   X(16, 4, 4) X(25, 5, 5) X(32, 4, 8) X(36, 6, 6) X(48, 4, 12) X(64, 8, 8) X(75, 5, 15)       \
-  X(81, 9, 9) X(100, 10, 10) X(128, 8, 16) X(144, 12, 12) X(256, 16, 16) X(450, 15, 30)     \
-  X(512, 16, 32)
+  X(81, 9, 9) X(100, 10, 10) X(128, 8, 16) X(144, 12, 12) X(200, 10, 20) X(256, 16, 16)     \
+  X(324, 18, 18) X(400, 20, 20) X(450, 15, 30) X(512, 16, 32) X(576, 24, 24) X(900, 30, 30)   \
+  X(1024, 32, 32)
 
 static bool adj_reg_size(int L) {
 #define X(NN, A, B) if (L == NN) return true;

@@ -1,5 +1,6 @@
 // C ABI: error state, twiddle tables, imaging plans and the imaging entry
 // points (spectrum window, coherent image, SOCS image, full spectrum).
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -147,10 +148,17 @@ static bool image_lengths_tabled(const oi_geometry& g) {
   return fp_image_size_ok(g.ny) && fp_image_size_ok(g.nx);
 }
 
+// Two-pass coarse grids up to this one keep the column fields of the whole batch
+// in the plan; larger ones those of a chunk of images (kColumnsPlan), and none
+// where one image's pass kTwoPassImage (4 GiB): such kernel sets stay with the
+// generic kernels, which need no such buffer.
+constexpr int kTwoPassBatch = 512;
+constexpr size_t kTwoPassImage = (size_t)4 << 30;
+
 // Validates a geometry and fills the library-chosen fields (coarse grid,
 // path, rows, kernel groups, band half-widths); allocates nothing.  generic:
 // image lengths without register transforms take the generic kernels
-// throughout (no product tables).
+// throughout (no product tables), and so do coarse grids past kTwoPassBatch.
 static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = false) {
   g = in;
   if (g.ny <= 0 || g.nx <= 0 || g.wr <= 0 || g.wc <= 0 || g.nchan <= 0 || g.nchan > 3 ||
@@ -210,10 +218,11 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
     // coarse grids past one workgroup's reach, and those the one-pass kernel
     // does not serve when the two-pass table has them (144)
     const int L1 = fp_coarse_choose(need);
-    const int L = need > 144 ? fp_two_pass_choose(need)
+    const int L = need > 144 ? fp_two_pass_choose(need, generic ? kTwoPassBatch : INT_MAX)
                              : (L1 > 0 && !fp_one_pass_ok(L1) && fp_two_pass_size_ok(L1) ? L1 : 0);
     if (L > 0 && L < g.ny && L < g.nx && g.wr <= L && g.wc <= L &&
-        fp_two_pass_lds(L) <= kLdsLimit) {
+        fp_two_pass_lds(L) <= kLdsLimit &&
+        (L <= kTwoPassBatch || (size_t)g.max_kernels * g.nchan * g.wc * L * sizeof(float2) <= kTwoPassImage)) {
       g.path = 2;
       g.lr = g.lc = lr = lc = L;
       if (g.max_groups <= 0) {
@@ -261,7 +270,7 @@ static size_t column_bytes(const oi_geometry& g) {
 }
 
 // Images whose column fields a plan holds.  The two-pass path keeps its batch's
-// (the adjoint reads them again).  On the one-pass path, coarse grids of 100 and
+// up to kTwoPassBatch (the adjoint reads them again).  On the one-pass path, coarse grids of 100 and
 // 128 are summed in two passes too, in chunks of images: 8 fields x 3 channels x
 // 24 kernels at 128 take 64 us in the one-pass kernel, whose rows wait for its
 // columns behind workgroup barriers, and 16 us in two passes.  A chunk is
@@ -270,7 +279,11 @@ static size_t column_bytes(const oi_geometry& g) {
 constexpr size_t kColumnsImage = (size_t)128 << 20, kColumnsPlan = (size_t)512 << 20;
 
 static size_t column_images(const oi_geometry& g, size_t B) {
-  if (g.path == 2) return B;
+  if (g.path == 2 && g.lr <= kTwoPassBatch) return B;
+  if (g.path == 2) {
+    const size_t fit = kColumnsPlan / column_bytes(g);
+    return fit < 1 ? 1 : (fit < B ? fit : B);
+  }
   if (g.path != 1 || !fp_split_size_ok(g.lr) || g.wr > g.lr || g.wc > g.lr) return 0;
   const size_t one = column_bytes(g);
   if (one > kColumnsImage) return 0;
@@ -563,7 +576,7 @@ extern "C" int oi_coherent_sets(oi_plan* p, const void* spec, int nsets, const v
 // writes 2 (I - target) and its partial sums).
 static bool residual_fused(const oi_plan* p) {
   const oi_geometry& g = p->g;
-  return g.path && image_lengths_tabled(g) && fp_urows_blocks(g.ny, g.nx, 1) <= g.ny;
+  return g.path && g.lr <= kTwoPassBatch && image_lengths_tabled(g) && fp_urows_blocks(g.ny, g.nx, 1) <= g.ny;
 }
 
 // target non-null: out = 2 (I - target), partial sums of (I - target)^2 in p->part.

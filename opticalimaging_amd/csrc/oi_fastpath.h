@@ -108,7 +108,7 @@ int ilt_target_const(const float* target, size_t npix, const float2* tband, size
 // plan holds B.
 bool fp_two_pass_size_ok(int l);
 bool fp_split_size_ok(int l);
-int fp_two_pass_choose(int need);
+int fp_two_pass_choose(int need, int most);   // smallest table size in [need, most], 0 if none
 size_t fp_two_pass_lds(int L);
 int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st);
 

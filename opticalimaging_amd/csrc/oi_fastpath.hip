@@ -1287,7 +1287,12 @@ static int run_band(const FpArgs& a, int groups, hipStream_t st) {
 // Coarse grids of the two-pass coherent sum: those of the two-pass path, and
 // those of the one-pass path whose tile no workgroup holds with one wave per
 // transform group (OI_COARSE_PLANS without a thread count).
-#define OI_TWO_PASS_PLANS(X) X(144, 12, 12) X(256, 16, 16) X(450, 15, 30) X(512, 16, 32)
+// The smallest one that holds the band serves: the work goes with L^2 log L, so
+// a grid of 256 for a band of 190 costs 1.7 times the one of 200, and bands past
+// 512 went to kernels of any length at 20 times the price.
+#define OI_TWO_PASS_PLANS(X)                                                      \
+  X(144, 12, 12) X(200, 10, 20) X(256, 16, 16) X(324, 18, 18) X(400, 20, 20)      \
+  X(450, 15, 30) X(512, 16, 32) X(576, 24, 24) X(900, 30, 30) X(1024, 32, 32)
 #define OI_SPLIT_PLANS(X) X(100, 10, 10) X(128, 8, 16)
 
 template <class PL>
@@ -1326,9 +1331,9 @@ bool fp_two_pass_size_ok(int l) {
   return false;
 }
 
-int fp_two_pass_choose(int need) {
+int fp_two_pass_choose(int need, int most) {
   int best = 0;
-#define X(NN, A, B) if (NN >= need && (best == 0 || NN < best)) best = NN;
+#define X(NN, A, B) if (NN >= need && NN <= most && (best == 0 || NN < best)) best = NN;
   OI_TWO_PASS_PLANS(X)
 #undef X
   return best;

@@ -1,6 +1,5 @@
 """The two-pass coherent sum and its adjoint on the row-major column fields, at
-every coarse size of the table (144, 256, 450, 512: groups of 12, 15 and 16
-lanes), windows of few and many columns, odd and even, on and off the centre,
+every coarse size of the table (144 to 1024: groups of 10 to 32 lanes), windows of few and many columns, odd and even, on and off the centre,
 single kernels and several groups of them, against float64 transforms.
 
 Tolerances as for the other image transforms of these lengths: 6e-6 of the peak
@@ -20,9 +19,14 @@ SIZES = [
     (320, 256, (-30, 71), (-3, 5), 1, 1, 144),       # five columns: one part-filled block
     (512, 512, (-55, 111), (-55, 111), 12, 3, 256),
     (288, 512, (-64, 128), (-40, 65), 2, 1, 256),    # the widest window of 256
-    (640, 512, (-60, 131), (-9, 17), 5, 1, 450),
+    (256, 320, (-50, 100), (-36, 73), 4, 2, 200),
+    (640, 512, (-60, 131), (-9, 17), 5, 1, 324),
+    (512, 640, (-100, 200), (-81, 163), 2, 2, 400),
     (512, 640, (-112, 225), (-107, 215), 3, 2, 450),
     (576, 576, (-128, 256), (-120, 231), 2, 1, 512),
+    (1024, 640, (-140, 288), (-144, 270), 2, 3, 576),
+    (1024, 960, (-200, 401), (-30, 61), 2, 1, 900),
+    (1080, 2048, (-250, 500), (-256, 512), 1, 2, 1024),
 ]
 
 

@@ -155,6 +155,32 @@ static bool image_lengths_tabled(const oi_geometry& g) {
 constexpr int kTwoPassBatch = 512;
 constexpr size_t kTwoPassImage = (size_t)4 << 30;
 
+// Column fields of one image in the two-pass coherent sum.
+static size_t column_bytes(const oi_geometry& g) {
+  return (size_t)g.max_kernels * g.nchan * g.wc * (size_t)g.lr * sizeof(float2);
+}
+
+// Images whose column fields a plan holds.  The two-pass path keeps its batch's
+// up to kTwoPassBatch (the adjoint reads them again).  On the one-pass path, coarse grids of 100 and
+// 128 are summed in two passes too, in chunks of images: 8 fields x 3 channels x
+// 24 kernels at 128 take 64 us in the one-pass kernel, whose rows wait for its
+// columns behind workgroup barriers, and 16 us in two passes.  A chunk is
+// bounded (512 MiB), and kernel sets of which one image passes 128 MiB stay with
+// the one-pass kernel.
+constexpr size_t kColumnsImage = (size_t)128 << 20, kColumnsPlan = (size_t)512 << 20;
+
+static size_t column_images(const oi_geometry& g, size_t B) {
+  if (g.path == 2 && g.lr <= kTwoPassBatch) return B;
+  if (g.path == 2) {
+    const size_t fit = kColumnsPlan / column_bytes(g);
+    return fit < 1 ? 1 : (fit < B ? fit : B);
+  }
+  if (g.path != 1 || !fp_split_size_ok(g.lr) || g.wr > g.lr || g.wc > g.lr) return 0;
+  const size_t one = column_bytes(g);
+  if (one > kColumnsImage) return 0;
+  return B * one <= kColumnsPlan ? B : kColumnsPlan / one;
+}
+
 // Validates a geometry and fills the library-chosen fields (coarse grid,
 // path, rows, kernel groups, band half-widths); allocates nothing.  generic:
 // image lengths without register transforms take the generic kernels
@@ -225,13 +251,8 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
         (L <= kTwoPassBatch || (size_t)g.max_kernels * g.nchan * g.wc * L * sizeof(float2) <= kTwoPassImage)) {
       g.path = 2;
       g.lr = g.lc = lr = lc = L;
-      if (g.max_groups <= 0) {
-        // kernel groups of the row pass: about 1024 blocks (16 coarse rows
-        // each) over the batch, at most 8 partial sums per image
-        const int blocks = (L / 16) * g.max_batch;
-        int gr = (1024 + blocks - 1) / blocks;
-        g.max_groups = gr < 1 ? 1 : (gr > 8 ? 8 : gr);
-      }
+      if (g.max_groups <= 0)
+        g.max_groups = fp_two_pass_groups(L, g.max_batch, g.max_kernels * g.nchan);
     }
   }
   // Coarse rows per workgroup: largest of 16, 8, 4, 2, 1 dividing lr whose
@@ -249,6 +270,8 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
   g.rows = rows;  // the compile-time path keeps every coarse row in one block
   // Kernel groups: fixed per plan so an image's summation order never depends
   // on the batch it is computed in.  0 = enough groups for ~512 workgroups.
+  if (g.max_groups <= 0 && g.path == 1 && column_images(g, g.max_batch))
+    g.max_groups = fp_two_pass_groups(g.lr, (int)column_images(g, g.max_batch), g.max_kernels * g.nchan);
   if (g.max_groups <= 0) {
     // about one workgroup per CU for the compile-time-size kernels (one
     // large block per CU; more partial sums cost more than they hide), about
@@ -262,32 +285,6 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
     g.max_groups = gr < 1 ? 1 : (gr > cap ? cap : gr);
   }
   return OI_OK;
-}
-
-// Column fields of one image in the two-pass coherent sum.
-static size_t column_bytes(const oi_geometry& g) {
-  return (size_t)g.max_kernels * g.nchan * g.wc * (size_t)g.lr * sizeof(float2);
-}
-
-// Images whose column fields a plan holds.  The two-pass path keeps its batch's
-// up to kTwoPassBatch (the adjoint reads them again).  On the one-pass path, coarse grids of 100 and
-// 128 are summed in two passes too, in chunks of images: 8 fields x 3 channels x
-// 24 kernels at 128 take 64 us in the one-pass kernel, whose rows wait for its
-// columns behind workgroup barriers, and 16 us in two passes.  A chunk is
-// bounded (512 MiB), and kernel sets of which one image passes 128 MiB stay with
-// the one-pass kernel.
-constexpr size_t kColumnsImage = (size_t)128 << 20, kColumnsPlan = (size_t)512 << 20;
-
-static size_t column_images(const oi_geometry& g, size_t B) {
-  if (g.path == 2 && g.lr <= kTwoPassBatch) return B;
-  if (g.path == 2) {
-    const size_t fit = kColumnsPlan / column_bytes(g);
-    return fit < 1 ? 1 : (fit < B ? fit : B);
-  }
-  if (g.path != 1 || !fp_split_size_ok(g.lr) || g.wr > g.lr || g.wc > g.lr) return 0;
-  const size_t one = column_bytes(g);
-  if (one > kColumnsImage) return 0;
-  return B * one <= kColumnsPlan ? B : kColumnsPlan / one;
 }
 
 // Device scratch of a plan for max_batch images: byte size of each buffer.

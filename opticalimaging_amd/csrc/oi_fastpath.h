@@ -110,6 +110,9 @@ bool fp_two_pass_size_ok(int l);
 bool fp_split_size_ok(int l);
 int fp_two_pass_choose(int need, int most);   // smallest table size in [need, most], 0 if none
 size_t fp_two_pass_lds(int L);
+constexpr int kTwoPassGroups = 64;
+// kernel groups (partial sums per image) of its row pass, at most kTwoPassGroups
+int fp_two_pass_groups(int L, int batch, int nkc);
 int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st);
 
 }  // namespace oi

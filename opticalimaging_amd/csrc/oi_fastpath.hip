@@ -727,7 +727,8 @@ constexpr int brows_min_blocks() {
 // no workgroup barrier, where staging a column-major B through an LDS tile took
 // six a kernel and left the waves waiting for each other.  Row pass of 16 images
 // x 12 kernels at L = 256: 30 -> 21 us, 24 x 12: 45 -> 26, 4 x 12 at L = 450:
-// 56 -> 32.  Loading the next kernel's row ahead needs 32 more registers and
+// 56 -> 32; with the groups that brows_groups chooses 18, 21 (at L = 200) and 22.
+// Loading the next kernel's row ahead needs 32 more registers and
 // gives up a wave per SIMD for it: 21, 32 and 49 us.
 template <class PL>
 __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(const float2* __restrict__ B, int nkc, int k0c,
@@ -1287,9 +1288,10 @@ static int run_band(const FpArgs& a, int groups, hipStream_t st) {
 // Coarse grids of the two-pass coherent sum: those of the two-pass path, and
 // those of the one-pass path whose tile no workgroup holds with one wave per
 // transform group (OI_COARSE_PLANS without a thread count).
-// The smallest one that holds the band serves: the work goes with L^2 log L, so
-// a grid of 256 for a band of 190 costs 1.7 times the one of 200, and bands past
-// 512 went to kernels of any length at 20 times the price.
+// The smallest one that holds the band serves: for bands of 173 orders (24 images
+// x 12 kernels) the row pass takes 21 us at 200 and 26 at 256, and a 2048^2 field
+// of 3 channels x 30 kernels with a band of 537 takes 0.17 ms at 576 where the
+// kernels for any length took 3.4.
 #define OI_TWO_PASS_PLANS(X)                                                      \
   X(144, 12, 12) X(200, 10, 20) X(256, 16, 16) X(324, 18, 18) X(400, 20, 20)      \
   X(450, 15, 30) X(512, 16, 32) X(576, 24, 24) X(900, 30, 30) X(1024, 32, 32)
@@ -1337,6 +1339,36 @@ int fp_two_pass_choose(int need, int most) {
   OI_TWO_PASS_PLANS(X)
 #undef X
   return best;
+}
+
+// An item of the row pass sums its kernels in one go, so a grid of one workgroup
+// more than the chip holds takes twice as long: the groups are chosen for the
+// fewest kernel turns, rounds x (kernels per group + 1.5 for the prologue and
+// the row DFT), and a little for each group's partial sum, which the band pass
+// reads again (about half a turn for 256 row groups).
+template <class PL>
+static int brows_groups(int batch, int nkc) {
+  const int per = (PL::N + fp::brows_rows<PL>() - 1) / fp::brows_rows<PL>() * batch;
+  const int slots = 256 * fp::brows_min_blocks<PL>();
+  int best = 1;
+  float least = 0.f;
+  for (int g = 1; g <= nkc && g <= kTwoPassGroups; ++g) {
+    const int rounds = (int)(((long long)per * g + slots - 1) / slots);
+    const float cost = rounds * ((nkc + g - 1) / g + 1.5f) + 0.5f * g * per / 256.f;
+    if (g == 1 || cost < least) {
+      least = cost;
+      best = g;
+    }
+  }
+  return best;
+}
+
+int fp_two_pass_groups(int L, int batch, int nkc) {
+#define X(NN, A, B) if (L == NN) return brows_groups<reg::GFFT<NN, A, B>>(batch, nkc);
+  OI_TWO_PASS_PLANS(X)
+  OI_SPLIT_PLANS(X)
+#undef X
+  return 1;
 }
 
 bool fp_split_size_ok(int l) {

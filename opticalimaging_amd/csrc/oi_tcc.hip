@@ -31,45 +31,54 @@ __device__ __forceinline__ unsigned short bf16_bits(float x) {
 }
 __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as_float((unsigned int)h << 16); }
 
-// Operand preparation.  mode 0: bf16 hi/lo planes [4][M][Kp] = Xh, Xl, Zh, Zl;
-// mode 1: fp32 planes [2][M][Kp] = X, Z; mode 2: fp64 planes [2][M][Kp].
-__global__ void k_tcc_prep(const float2* __restrict__ G, const float* __restrict__ w, int M, int nsrc,
-                           int ncomp, int Kp, int mode, void* __restrict__ work) {
+// Operand preparation.  MODE 0: bf16 hi/lo planes [4][M][Kp] = Xh, Xl, Zh, Zl;
+// MODE 1: fp32 planes [2][M][Kp] = X, Z; MODE 2: fp64 planes [2][M][Kp].  Row rr
+// of G takes columns 2 rr and 2 rr + 1 of a plane, (re, im) of X and (-im, re) of
+// Z, so that one store writes both.
+// G is read along m and the planes are written along k: a workgroup takes 64 m x
+// 32 rows through the LDS.  (One plane entry per thread, lanes along k, read a
+// line of G per lane: 20 us at M = 10201, 120 rows, 11.5 so.)
+template <int MODE>
+__global__ __launch_bounds__(256) void k_tcc_prep(const float2* __restrict__ G,
+                                                  const float* __restrict__ w, int M, int nsrc,
+                                                  int ncomp, int Kp, void* __restrict__ work) {
+  __shared__ float2 tile[32][65];
   const int r = ncomp * nsrc;
-  const size_t total = (size_t)M * Kp;
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-       e += (size_t)gridDim.x * blockDim.x) {
-    const int m = (int)(e / Kp), k = (int)(e - (size_t)m * Kp);
-    float xv = 0.f, zv = 0.f;
-    if (k < 2 * r) {
-      const int rr = k < r ? k : k - r;
-      const int s = rr % nsrc;
-      const float2 a = G[(size_t)rr * M + m];
-      const float sw = sqrtf(w[s]);
-      const float re = a.x * sw, im = a.y * sw;
-      if (k < r) {
-        xv = re;
-        zv = -im;
-      } else {
-        xv = im;
-        zv = re;
-      }
-    }
-    if (mode == 0) {
-      unsigned short* P = static_cast<unsigned short*>(work);
-      const unsigned short xh = bf16_bits(xv), zh = bf16_bits(zv);
-      P[e] = xh;
-      P[total + e] = bf16_bits(xv - bf16_value(xh));
-      P[2 * total + e] = zh;
-      P[3 * total + e] = bf16_bits(zv - bf16_value(zh));
-    } else if (mode == 1) {
-      float* P = static_cast<float*>(work);
-      P[e] = xv;
-      P[total + e] = zv;
+  const int m0 = blockIdx.x * 64, r0 = blockIdx.y * 32;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int rr = (threadIdx.x >> 6) + 4 * i, m = threadIdx.x & 63;
+    const bool in = r0 + rr < r && m0 + m < M;
+    const size_t row = in ? r0 + rr : 0;
+    const float2 a = G[row * M + (in ? m0 + m : 0)];
+    const float sw = in ? sqrtf(w[row % nsrc]) : 0.f;
+    tile[rr][m] = in ? make_float2(a.x * sw, a.y * sw) : make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+  const size_t half = (size_t)M * Kp / 2;   // pairs of a plane (Kp is even)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int m = (threadIdx.x >> 5) + 8 * i, rr = threadIdx.x & 31;
+    if (m0 + m >= M || r0 + rr >= Kp / 2) continue;
+    const float2 v = tile[rr][m];
+    const size_t e = (size_t)(m0 + m) * (Kp / 2) + r0 + rr;
+    if constexpr (MODE == 0) {
+      unsigned int* P = static_cast<unsigned int*>(work);
+      const unsigned int rh = bf16_bits(v.x), ih = bf16_bits(v.y), nh = bf16_bits(-v.y);
+      const unsigned int rl = bf16_bits(v.x - bf16_value(rh)), il = bf16_bits(v.y - bf16_value(ih));
+      const unsigned int nl = bf16_bits(-v.y - bf16_value(nh));
+      P[e] = rh | ih << 16;
+      P[half + e] = rl | il << 16;
+      P[2 * half + e] = nh | rh << 16;
+      P[3 * half + e] = nl | rl << 16;
+    } else if constexpr (MODE == 1) {
+      float2* P = static_cast<float2*>(work);
+      P[e] = v;
+      P[half + e] = make_float2(-v.y, v.x);
     } else {
-      double* P = static_cast<double*>(work);
-      P[e] = (double)xv;
-      P[total + e] = (double)zv;
+      double2* P = static_cast<double2*>(work);
+      P[e] = make_double2(v.x, v.y);
+      P[half + e] = make_double2(-v.y, v.x);
     }
   }
 }
@@ -559,10 +568,9 @@ extern "C" int oi_tcc_build(const void* G, const float* w, int M, int nsrc, int 
   hipStream_t st = (hipStream_t)stream;
   const int Kp = (int)kp_for(nsrc, ncomp, precision);
   const int mode = precision == OI_TCC_SPLIT_BF16 ? 0 : (precision == OI_TCC_FP32 ? 1 : 2);
-  size_t tot = (size_t)M * Kp;
-  int blocks = (int)((tot + 255) / 256 > 16384 ? 16384 : (tot + 255) / 256);
-  hipLaunchKernelGGL(k_tcc_prep, dim3(blocks), dim3(256), 0, st, static_cast<const float2*>(G), w, M,
-                     nsrc, ncomp, Kp, mode, work);
+  const dim3 prep((M + 63) / 64, (Kp / 2 + 31) / 32);
+  hipLaunchKernelGGL(mode == 0 ? k_tcc_prep<0> : (mode == 1 ? k_tcc_prep<1> : k_tcc_prep<2>), prep,
+                     dim3(256), 0, st, static_cast<const float2*>(G), w, M, nsrc, ncomp, Kp, work);
   OI_LAUNCH_CHECK("tcc_prep");
   const int nt = (M + kTile - 1) / kTile;
   const int pairs = nt * (nt + 1) / 2;

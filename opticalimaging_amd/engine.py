@@ -328,7 +328,7 @@ class _PlanCache:
         self.lock = threading.Lock()
 
     def get(self, **kw) -> Plan:
-        owner = (threading.get_ident(), torch.cuda.current_stream().cuda_stream)
+        owner = (threading.get_ident(), nat.stream_handle())
         key = (owner, tuple(sorted(kw.items())))
         with self.lock:
             p = self.plans.get(key)

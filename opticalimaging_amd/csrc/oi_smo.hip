@@ -8,7 +8,8 @@
 // All sums in float64.  At the small grids where this is called most the
 // launches are the cost: four here, where the same steps as separate transforms,
 // gathers, scalings and reductions were about sixty with two host waits.
-// 128^2, 120 points, image and gradient: 525 -> 184 us.
+// 128^2, 120 points, image and gradient: 525 -> 184 us (155 with
+// cheaper launches from Python).
 #include "oi_internal.h"
 
 namespace oi {

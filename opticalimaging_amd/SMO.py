@@ -166,10 +166,11 @@ class AbbeSourceProblem:
         return out
 
     def source_gradient(self, V: torch.Tensor, grad_image: torch.Tensor) -> torch.Tensor:
-        """dL/dV (float64, nsrc) for image cotangents grad_image (nFocus, ny, nx)."""
+        """dL/dV (float64, nsrc) for image cotangents grad_image (nFocus, ny, nx);
+        those past the problem's foci are not read."""
         V = self._weights(V)
         g = grad_image.detach().to(self.dev, torch.float32).contiguous()
-        if g.shape != (len(self.foci), self.ny, self.nx):
+        if g.dim() != 3 or len(g) < len(self.foci) or g.shape[1:] != (self.ny, self.nx):
             raise ValueError("grad_image must have the image's shape")
         img = self.image(V)
         lib = nat.load()

@@ -28,3 +28,12 @@ def test_no_focus_gives_zeros(gpu):
     del used
     image.sum().backward()
     assert torch.equal(V.grad, torch.zeros_like(V))
+
+
+def test_cotangents_of_more_foci(gpu):
+    prob = _problem([0.0, 40.0])
+    g = torch.randn((3, 64, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    assert torch.equal(prob.source_gradient(prob.V0, g), prob.source_gradient(prob.V0, g[:2]))
+    for bad in (g[:1], g[:2, :63], g[:2].reshape(2, -1)):
+        with pytest.raises(ValueError):
+            prob.source_gradient(prob.V0, bad)

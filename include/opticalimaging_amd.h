@@ -216,13 +216,17 @@ int oi_socs_image(oi_plan* plan, const void* field, int kind, int cin,
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It takes
  * the geometry inputs of oi_plan_create instead of a plan (max_batch and
- * max_kernels are ignored: kernel groups are chosen as for a plan of
- * `batch` images, so each image is summed as oi_socs_image sums it with such
- * a plan) and calls no hipMalloc, hipFree or other allocating routine.
+ * max_kernels are ignored: kernel groups are chosen as for a plan of `batch`
+ * images and `nkern` kernels, so each image is summed as oi_socs_image sums it
+ * with such a plan) and calls no hipMalloc, hipFree or other allocating routine.
  * Twiddle tables and scratch live in one static device array of
  * OI_NOALLOC_SCRATCH_BYTES per GPU, held from module load until the process
- * ends; the batch runs in passes of as many images as fit.  A geometry whose
- * single image needs more than that fails with OI_ERR_INVALID.  Every call
+ * ends; the batch runs in passes of as many images as fit, and where not one
+ * fits, its kernel groups in passes of as many as fit.  Where one group, or the
+ * tables of an image length without a compile-time transform, do not fit
+ * either, the image takes whatever form needs the least scratch (the same
+ * squares, to float32 rounding); one that does not fit so fails with
+ * OI_ERR_INVALID.  Every call
  * on one GPU shares the array: calls that overlap on one GPU (several
  * streams or host threads) race and give undefined images.  Enqueued on
  * `stream`; no synchronisation.                                              */

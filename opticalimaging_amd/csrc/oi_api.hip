@@ -111,7 +111,8 @@ struct oi_plan {
   float2* Ihat = nullptr;
   float* part = nullptr;    // residual sums of the image-row pass, [B][ny]
   float2* Bbuf = nullptr;   // two-pass column fields of max_kernels kernels of
-  int bimg = 0;             // this many images (path 2: max_batch)
+  int bimg = 0;             // this many images (path 2: max_batch), or of
+  int bgroups = 0;          // this many of one image's kernel groups (0: of all)
   float* dft = nullptr;     // product tables of the image lengths (dft_bytes)
   DftTable tab_x, tab_y;
   size_t bytes = 0;
@@ -155,9 +156,17 @@ static bool image_lengths_tabled(const oi_geometry& g) {
 constexpr int kTwoPassBatch = 512;
 constexpr size_t kTwoPassImage = (size_t)4 << 30;
 
-// Column fields of one image in the two-pass coherent sum.
+// Column fields of one image in the two-pass coherent sum: all of them, or those
+// of `groups` of its kernel groups.
+static int sum_groups(const oi_geometry& g) { return g.max_groups < g.max_kernels ? g.max_groups : g.max_kernels; }
+
 static size_t column_bytes(const oi_geometry& g) {
   return (size_t)g.max_kernels * g.nchan * g.wc * (size_t)g.lr * sizeof(float2);
+}
+
+static size_t column_bytes(const oi_geometry& g, int groups) {
+  return (size_t)fp_two_pass_slots(g.max_kernels * g.nchan, sum_groups(g), groups) * g.wc * (size_t)g.lr *
+         sizeof(float2);
 }
 
 // Images whose column fields a plan holds.  The two-pass path keeps its batch's
@@ -182,9 +191,11 @@ static size_t column_images(const oi_geometry& g, size_t B) {
 }
 
 // Validates a geometry and fills the library-chosen fields (coarse grid,
-// path, rows, kernel groups, band half-widths); allocates nothing.  generic:
-// image lengths without register transforms take the generic kernels
-// throughout (no product tables), and so do coarse grids past kTwoPassBatch.
+// path, rows, kernel groups, band half-widths); allocates nothing.  generic (the
+// form with the least scratch): image lengths without register transforms take
+// the generic kernels throughout (no product tables), and so do coarse grids
+// past kTwoPassBatch; a two-pass sum has the groups for which one image's partial
+// sums and one group's column fields are fewest.
 static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = false) {
   g = in;
   if (g.ny <= 0 || g.nx <= 0 || g.wr <= 0 || g.wc <= 0 || g.nchan <= 0 || g.nchan > 3 ||
@@ -253,6 +264,16 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
       g.lr = g.lc = lr = lc = L;
       if (g.max_groups <= 0)
         g.max_groups = fp_two_pass_groups(L, g.max_batch, g.max_kernels * g.nchan);
+      if (generic && in.max_groups <= 0) {
+        size_t least = 0;
+        for (int n = 1; n <= g.max_kernels && n <= kTwoPassGroups; ++n) {
+          const size_t nkc = (size_t)g.max_kernels * g.nchan;
+          const size_t rows = (size_t)n * (g.qc + 1) + (nkc + n - 1) / n * g.wc;
+          if (n > 1 && rows >= least) continue;
+          least = rows;
+          g.max_groups = n;
+        }
+      }
     }
   }
   // Coarse rows per workgroup: largest of 16, 8, 4, 2, 1 dividing lr whose
@@ -293,8 +314,9 @@ struct ScratchLayout {
   size_t total() const { return T + spec + R + U + Ic + Ihat + part + Bbuf; }
 };
 
-// columns: with the column fields that a one-pass plan can do without.
-static ScratchLayout scratch_layout(const oi_geometry& g, size_t B, bool columns = true) {
+// groups: the kernel groups whose column fields are kept (less than all: of one
+// image; 0: none, which a one-pass plan can do without).
+static ScratchLayout scratch_layout(const oi_geometry& g, size_t B, int groups = INT_MAX) {
   const size_t C = (size_t)g.nchan, G = (size_t)g.max_groups;
   const size_t lr = (size_t)g.lr, lc = (size_t)g.lc;
   ScratchLayout s;
@@ -305,7 +327,7 @@ static ScratchLayout scratch_layout(const oi_geometry& g, size_t B, bool columns
   s.Ic = (g.direct && G > 1) ? B * G * lr * lc * sizeof(float) : 0;
   s.Ihat = g.path ? B * (size_t)(g.qc + 1) * (2 * g.qr + 1) * sizeof(float2) : 0;
   s.part = g.path ? B * (size_t)g.ny * sizeof(float) : 0;
-  s.Bbuf = (columns || g.path == 2) ? column_images(g, B) * column_bytes(g) : 0;
+  s.Bbuf = column_images(g, B) * (groups < sum_groups(g) ? column_bytes(g, groups) : column_bytes(g));
   return s;
 }
 
@@ -610,7 +632,7 @@ static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* ke
     c.wr = g.wr;
     c.k0c = g.k0c;
     c.wc = g.wc;
-    c.groups = groups;
+    c.groups = c.count = groups;
     c.qc = g.qc;
     c.tw_l = p->flr.tw;
     c.tw_m = p->flr.tw;
@@ -624,7 +646,11 @@ static int coherent_impl(oi_plan* p, const void* spec, int batch, const void* ke
         ci.spec += i * c.spec_img;
         ci.kern += i * c.kern_img;
         ci.R += (size_t)i * c.groups * (g.qc + 1) * g.lr;
-        if ((rc = fp_two_pass(ai, ci, p->Bbuf, st))) return rc;
+        const int step = p->bgroups > 0 && p->bgroups < groups ? p->bgroups : groups;
+        for (ci.first = 0; ci.first < groups; ci.first += step) {
+          ci.count = groups - ci.first < step ? groups - ci.first : step;
+          if ((rc = fp_two_pass(ai, ci, p->Bbuf, st))) return rc;
+        }
       }
     } else if ((rc = fp_coherent(a, c, st))) {
       return rc;
@@ -1022,13 +1048,24 @@ static size_t aligned_total(const ScratchLayout& s) {
          align_up(s.Ihat) + align_up(s.part) + align_up(s.Bbuf);
 }
 
-// Scratch of one image with its tables, at most (twiddle tables counted once
-// per transform length, shared or not).
-static size_t noalloc_bytes(const oi_geometry& g, bool columns) {
+// Scratch of one image with its tables and the column fields of `groups` kernel
+// groups, at most (twiddle tables counted once per transform length, shared or
+// not).
+static size_t noalloc_bytes(const oi_geometry& g, int groups) {
   const size_t tw = align_up(2 * (size_t)g.nx * sizeof(float2)) + align_up(2 * (size_t)g.ny * sizeof(float2)) +
                     align_up(2 * (size_t)g.lr * sizeof(float2)) + align_up(2 * (size_t)g.lc * sizeof(float2)) +
                     align_up(2 * (size_t)g.rows * sizeof(float2));
-  return tw + align_up(dft_bytes(g, false) + dft_bytes(g, true)) + aligned_total(scratch_layout(g, 1, columns));
+  return tw + align_up(dft_bytes(g, false) + dft_bytes(g, true)) + aligned_total(scratch_layout(g, 1, groups));
+}
+
+// Kernel groups whose column fields the scratch holds beside one image: all of
+// them, fewer, or none (one-pass sum).  fits: whether the image fits with them.
+static int noalloc_groups(const oi_geometry& g, bool& fits) {
+  int groups = column_images(g, 1) ? sum_groups(g) : 0;
+  while (groups > 1 && noalloc_bytes(g, groups) > kNoAllocScratch) --groups;
+  if (g.path == 1 && noalloc_bytes(g, groups) > kNoAllocScratch) groups = 0;
+  fits = noalloc_bytes(g, groups) <= kNoAllocScratch;
+  return groups;
 }
 
 extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, int kind, int cin,
@@ -1038,18 +1075,24 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   if (batch < 1) return fail(OI_ERR_INVALID, "socs_image_noalloc: batch must be >= 1");
   if (nkern < 1) return fail(OI_ERR_INVALID, "socs_image_noalloc: nkern must be >= 1");
   // Kernel groups are chosen as for a plan of `batch` images and `nkern`
-  // kernels, so each image is summed exactly as oi_socs_image sums it there.
+  // kernels, and where the column fields of all do not fit, they go through the
+  // scratch a few groups at a time: each image is summed exactly as oi_socs_image
+  // sums it there.
   oi_geometry in = *geo;
   in.max_batch = batch;
   in.max_kernels = nkern;
   oi_geometry g;
   int rc = plan_geometry(in, g);
   if (rc) return rc;
-  // the tables and buffers of image lengths without a register transform may
-  // not fit beside one image: those sizes then take the generic kernels, whose
-  // scratch is smaller
-  if (noalloc_bytes(g, false) > kNoAllocScratch && (rc = plan_geometry(in, g, true))) return rc;
-  const bool columns = noalloc_bytes(g, true) <= kNoAllocScratch;
+  // Close to the limit one image may not fit with the tables of lengths without
+  // a register transform, its partial sums and the column fields of one group:
+  // it then takes the form with the least scratch, which sums in another order.
+  bool fits = false;
+  int cgroups = noalloc_groups(g, fits);
+  if (!fits) {
+    if ((rc = plan_geometry(in, g, true))) return rc;
+    cgroups = noalloc_groups(g, fits);
+  }
   // twiddle tables first, one per distinct length
   const int sizes[5] = {g.nx, g.ny, g.lr, g.lc, g.rows};
   FftDesc d[5];
@@ -1066,7 +1109,7 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   }
   const size_t dft_off = used;
   used += align_up(dft_bytes(g, false) + dft_bytes(g, true));
-  const size_t per_image = aligned_total(scratch_layout(g, 1, columns));
+  const size_t per_image = aligned_total(scratch_layout(g, 1, cgroups));
   if (used + per_image > kNoAllocScratch)
     return fail(OI_ERR_INVALID, "socs_image_noalloc: one image needs " +
                                     std::to_string(used + per_image) + " bytes of scratch, beyond the " +
@@ -1074,7 +1117,8 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   // images per pass: align_up(c x) <= c align_up(x), so c images fit in c
   // one-image layouts
   const size_t fit = (kNoAllocScratch - used) / per_image;
-  const int chunk = fit < (size_t)batch ? (int)fit : batch;
+  const bool part = cgroups > 0 && cgroups < sum_groups(g);
+  const int chunk = part ? 1 : (fit < (size_t)batch ? (int)fit : batch);
   unsigned char* base = nullptr;
   rc = scratch_of_current_device(&base);
   if (rc) return rc;
@@ -1101,8 +1145,9 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   pl.frows = d[4];
   pl.dft = reinterpret_cast<float*>(base + dft_off);
   if ((rc = dft_build(&pl, st))) return rc;
-  const ScratchLayout sl = scratch_layout(pl.g, (size_t)chunk, columns);
+  const ScratchLayout sl = scratch_layout(pl.g, (size_t)chunk, cgroups);
   pl.bimg = sl.Bbuf ? (int)column_images(pl.g, (size_t)chunk) : 0;
+  pl.bgroups = part ? cgroups : 0;
   unsigned char* cur = base + used;
   auto carve = [&cur](size_t bytes) -> unsigned char* {
     unsigned char* p = bytes ? cur : nullptr;

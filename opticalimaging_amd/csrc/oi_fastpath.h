@@ -53,6 +53,7 @@ struct FpCoh {
   int nchan, nkern;
   int k0r, wr, k0c, wc;
   int groups;
+  int first, count;     // two-pass sum: the kernel groups [first, first + count) of this launch
   int qc;
   const float2* tw_l;  // exp(-2 pi i m / L) (stage twiddles and phase twist)
   const float2* tw_m;  // column-stage transform table
@@ -102,8 +103,9 @@ int ilt_update_theta(float* theta, const float* gt, float lr, int batch, size_t 
 size_t ilt_target_const_scratch(int batch);
 int ilt_target_const(const float* target, size_t npix, const float2* tband, size_t nband,
                      int batch, void* scratch, float* tconst, hipStream_t st);
-// Two-pass coherent sum: B holds batch * nkern * nchan * wc * L c64; R in
-// [img][group][q][t].  fp_two_pass_size_ok: the two-pass path's coarse grids;
+// Two-pass coherent sum of the kernel groups [c.first, c.first + c.count): B
+// holds batch * fp_two_pass_slots * wc * L c64; R in [img][group][q][t], all
+// c.groups of them.  fp_two_pass_size_ok: the two-pass path's coarse grids;
 // fp_split_size_ok: grids of the one-pass path that it serves better where a
 // plan holds B.
 bool fp_two_pass_size_ok(int l);
@@ -113,6 +115,11 @@ size_t fp_two_pass_lds(int L);
 constexpr int kTwoPassGroups = 64;
 // kernel groups (partial sums per image) of its row pass, at most kTwoPassGroups
 int fp_two_pass_groups(int L, int batch, int nkc);
+// (kernel, channel) pairs of `count` groups, at most: pair j groups + first + i
+// is slot j count + i of B
+inline int fp_two_pass_slots(int nkc, int groups, int count) {
+  return count < groups ? (nkc + groups - 1) / groups * count : nkc;
+}
 int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st);
 
 }  // namespace oi

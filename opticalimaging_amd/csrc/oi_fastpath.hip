@@ -663,17 +663,23 @@ template <class PL>
 __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ spec,
                                                      const float2* __restrict__ kern,
                                                      size_t spec_img, size_t kern_img, int nk,
-                                                     int nchan, int k0r, int wr, int wc,
+                                                     int nchan, int groups, int first, int count,
+                                                     int slots, int k0r, int wr, int wc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ B, int batch) {
   constexpr int L = PL::N, TL = PL::T, VL = PL::V, G = groups_per_block<PL>();
   extern __shared__ float2 lds[];
-  const int nxb = (wc + G - 1) / G, nkc = nk * nchan;
+  const int nxb = (wc + G - 1) / G;
   int w;
-  if (!xcd_item(blockIdx.x, nxb * nkc * batch, w)) return;   // uniform over the block
+  if (!xcd_item(blockIdx.x, nxb * slots * batch, w)) return;   // uniform over the block
   const int g = threadIdx.x % G, tg = threadIdx.x / G;
   const int c = w % nxb * G + g;
-  const int kc = (w / nxb) % nkc, img = w / (nxb * nkc);   // kc = k * nchan + channel
+  const int slot = (w / nxb) % slots, img = w / (nxb * slots);
+  int kc = slot;                                           // k * nchan + channel
+  if (count < groups) {                                    // uniform over the grid
+    kc = slot / count * groups + first + slot % count;
+    if (kc >= nk * nchan) return;                          // uniform over the block
+  }
   const int k = kc / nchan, ch = kc - k * nchan;
   const bool live = tg < TL && c < wc;
   const int t = tg < TL ? tg : 0;
@@ -695,7 +701,7 @@ __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ 
   }
   PL::template run_live_tab<false>(v, lds + g * (PL::LDS | 1), t, twt, live);
   if (!live) return;
-  float2* dst = B + ((size_t)img * nkc + kc) * L * wc + c;
+  float2* dst = B + ((size_t)img * slots + slot) * L * wc + c;
 #pragma unroll
   for (int m = 0; m < VL; ++m) dst[(size_t)(t + TL * m) * wc] = v[m];
 }
@@ -720,7 +726,8 @@ constexpr int brows_min_blocks() {
 }
 
 // Items (row group, image, kernel group); an item sums the (kernel, channel)
-// pairs kc = grp, grp + groups, ... into its own partial R[img][grp].  Images
+// pairs kc = grp, grp + groups, ... into its own partial R[img][grp], the same
+// whichever groups share the launch.  Images
 // slowest, as pass 1 writes them: an XCD reads what it wrote.
 // A wave is on its own: it loads its rows of B straight into registers (a row
 // is contiguous) and exchanges inside its own part of the LDS, so the loop has
@@ -735,7 +742,7 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
                                                      int wc, int qc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ R, int batch,
-                                                     int groups) {
+                                                     int groups, int first, int count, int slots) {
   constexpr int L = PL::N, TL = PL::T, VL = PL::V, GW = 64 / TL, RB = brows_rows<PL>();
   static_assert(VL <= 32, "row mask holds VL bits");
   extern __shared__ float2 lds[];
@@ -743,8 +750,8 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
   // their ends
   constexpr int NXR = (L + RB - 1) / RB;
   int w;
-  if (!xcd_item(blockIdx.x, NXR * batch * groups, w)) return;   // uniform over the block
-  const int xr = w % NXR, grp = (w / NXR) % groups, img = w / (NXR * groups);
+  if (!xcd_item(blockIdx.x, NXR * batch * count, w)) return;   // uniform over the block
+  const int xr = w % NXR, at = (w / NXR) % count, img = w / (NXR * count), grp = first + at;
   const int lane = threadIdx.x & 63, gw = lane / TL;
   const int t = gw < GW ? lane - gw * TL : 0;
   const int g = (threadIdx.x >> 6) * GW + (gw < GW ? gw : 0);
@@ -764,8 +771,8 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
   float acc[VL];
 #pragma unroll
   for (int m = 0; m < VL; ++m) acc[m] = 0.f;
-  const float2* src = B + ((size_t)img * nkc + grp) * L * wc + (size_t)(live ? row : 0) * wc;
-  const size_t step = (size_t)groups * L * wc;
+  const float2* src = B + ((size_t)img * slots + at) * L * wc + (size_t)(live ? row : 0) * wc;
+  const size_t step = (size_t)count * L * wc;
   float2 v[VL];
   for (int kc = grp; kc < nkc; kc += groups) {
 #pragma unroll
@@ -1308,17 +1315,19 @@ static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t 
   const size_t lds1 = bcols_lds<PL>();
   int rc = allow(k_fp_bcols<PL>, lds1);
   if (rc) return rc;
-  const int cols = ((a.wc + G - 1) / G) * c.nkern * c.nchan * a.batch;
+  const int slots = fp_two_pass_slots(c.nkern * c.nchan, c.groups, c.count);
+  const int cols = ((a.wc + G - 1) / G) * slots * a.batch;
   hipLaunchKernelGGL(k_fp_bcols<PL>, dim3(xcd_grid(cols)), dim3(kBlock), lds1, st, c.spec, c.kern,
-                     c.spec_img, c.kern_img, c.nkern, c.nchan, a.k0r, a.wr, a.wc, a.tw_l, B, a.batch);
+                     c.spec_img, c.kern_img, c.nkern, c.nchan, c.groups, c.first, c.count, slots,
+                     a.k0r, a.wr, a.wc, a.tw_l, B, a.batch);
   OI_LAUNCH_CHECK("fp_bcols");
   const size_t lds2 = two_pass_rows_lds<PL>();
   rc = allow(k_fp_brows<PL>, lds2);
   if (rc) return rc;
-  const int items = ((PL::N + RB - 1) / RB) * a.batch * c.groups;
+  const int items = ((PL::N + RB - 1) / RB) * a.batch * c.count;
   hipLaunchKernelGGL(k_fp_brows<PL>, dim3(xcd_grid(items)), dim3(kBlock), lds2, st, B,
                      c.nkern * c.nchan, a.k0c, a.wc, a.qc, a.tw_l, c.R, a.batch,
-                     c.groups);
+                     c.groups, c.first, c.count, slots);
   OI_LAUNCH_CHECK("fp_brows");
   return OI_OK;
 }

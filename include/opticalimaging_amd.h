@@ -196,8 +196,9 @@ int oi_pupil_crop(const void* spec, int nchan, int k0r, int wr, int k0c, int wc,
 
 /* Images of one spectrum under nsets kernel sets: out[s] is what
  * oi_coherent_image gives for (spec, kern[s]), up to the summation order of the
- * kernel groups, which is the plan's.  A plan with compile-time coarse kernels
- * takes max_batch sets per launch chain, any other one set.
+ * kernel groups.  A plan with compile-time coarse kernels takes max_batch sets
+ * per launch chain, in its own groups; any other one set, in no fewer groups than
+ * a plan for one image as far as its buffers hold them.
  * The foci of CalculateAbbeImage (CalculateAerialImage.py:46-92) are such sets.
  *   spec : c64 [nchan][wr][wc]
  *   kern : c64 [nsets][nkern][wr][wc]

@@ -68,7 +68,8 @@ int oi_version(void);
  * Geometry of one imaging problem.  Inputs to oi_plan_create: ny, nx, the
  * spectrum window, nchan (channels carried per image), max_batch, max_groups
  * (kernels are split into this many partial sums, fixed for the plan so a
- * result never depends on the batch it is computed in; 0 = choose),
+ * result never depends on the batch it is computed in; 0 = choose; coarse grids
+ * of 100 and 128 in two passes take no more than they would choose),
  * max_kernels (the largest kernel count any call on the plan passes; every
  * buffer that grows with it is allocated here, and calls with more kernels
  * fail with OI_ERR_INVALID; 0 = 256) and optionally lr, lc (coarse grid;

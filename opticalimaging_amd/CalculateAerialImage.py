@@ -61,11 +61,12 @@ def _abbe_images(field, source, scatter, projector, numerics, encoding):
     tens, kind, cin, live = encoding if encoding is not None else engine.field_encoding(h)
     ncomp = 3 if vector else 1
     foci = optics.focus_values(projector)
-    # One-pass coarse grids (2 band - 1 <= 128) image up to 16 foci per launch
-    # chain: 512^2, 196 points x 3 components, 5 foci: coherent sum 80 -> 47 us,
-    # band, columns and rows 90 -> 17 us.  Where 512 workgroups still have four
-    # kernels each, that many (two per CU) hide more latency than their partial
-    # sums cost: 47 us against 54 with 256.
+    # Coarse grids up to 128 image up to 16 foci per launch chain: 512^2, 196
+    # points x 3 components, 5 foci: coherent sum 80 -> 47 us, band, columns and
+    # rows 90 -> 17 us.  Where 512 workgroups of the one-pass sum (up to 81) still
+    # have four kernels each, that many (two per CU) hide more latency than their
+    # partial sums cost: 47 us against 54 with 256.  Sums in two passes take the
+    # fewer groups that they choose themselves.
     need = 2 * max(br, bc) - 1
     batch = max(1, min(len(foci), 16)) if need <= 128 and need < min(ny, nx) else 1
     nk = ncomp * src.n

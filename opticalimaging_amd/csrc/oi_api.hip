@@ -187,7 +187,10 @@ static size_t column_images(const oi_geometry& g, size_t B) {
   if (g.path != 1 || !fp_split_size_ok(g.lr) || g.wr > g.lr || g.wc > g.lr) return 0;
   const size_t one = column_bytes(g);
   if (one > kColumnsImage) return 0;
-  return B * one <= kColumnsPlan ? B : kColumnsPlan / one;
+  // chunks of equal length, as the groups are chosen for one: 16 images of 588
+  // kernels at 100 as 12 + 4, in the groups of 12, take 9 % longer than as 8 + 8
+  const size_t fit = kColumnsPlan / one, chunks = (B + fit - 1) / fit;
+  return (B + chunks - 1) / chunks;
 }
 
 // Kernel groups of the one-pass and the generic kernels for a launch of `images`.
@@ -304,8 +307,14 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
   g.rows = rows;  // the compile-time path keeps every coarse row in one block
   // Kernel groups: fixed per plan so an image's summation order never depends
   // on the batch it is computed in.  0 = enough groups for ~512 workgroups.
-  if (g.max_groups <= 0 && g.path == 1 && column_images(g, g.max_batch))
-    g.max_groups = fp_two_pass_groups(g.lr, (int)column_images(g, g.max_batch), g.max_kernels * g.nchan);
+  // Coarse 100 and 128 in two passes: a count asked for only bounds their own
+  // choice.  512 groups over the foci, which suit the one-pass kernel, took 4 and 5
+  // foci of 588 kernels 204 and 240 us at 100 and 209 and 246 at 128; their own
+  // 37, 30, 46 and 37 take 196, 235, 201 and 235.
+  if (g.path == 1 && column_images(g, g.max_batch)) {
+    const int own = fp_two_pass_groups(g.lr, (int)column_images(g, g.max_batch), g.max_kernels * g.nchan);
+    if (g.max_groups <= 0 || g.max_groups > own) g.max_groups = own;
+  }
   if (g.max_groups <= 0) g.max_groups = fill_groups(g, g.max_batch);
   return OI_OK;
 }

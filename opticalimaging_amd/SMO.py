@@ -99,9 +99,10 @@ class AbbeSourceProblem:
         nsrc = self.src.n
         # The float64 gradient takes <g, I> from this float32 image: image lengths
         # without register transforms keep the general kernels (a coarse grid of
-        # the caller's choice) and with them the rounding of that term.
+        # the caller's choice) and with them the rounding of that term.  Past a
+        # coarse grid of 128 the sum always was the two-pass one.
         lr = lc = 0
-        if not {self.ny, self.nx} <= _REGISTER_LENGTHS:
+        if 2 * max(br, bc) - 1 <= 128 and not {self.ny, self.nx} <= _REGISTER_LENGTHS:
             lr, lc = _coarse(2 * br - 1, self.ny), _coarse(2 * bc - 1, self.nx)
         self.plan = engine.Plan(self.ny, self.nx, k0r, wr, k0c, wc, nchan=self.C, max_batch=1,
                                 band_r=br, band_c=bc, lr=lr, lc=lc, max_kernels=self.ncomp * nsrc)

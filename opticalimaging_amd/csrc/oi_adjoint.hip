@@ -197,19 +197,26 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cfield_reg(const float2* __re
   const bool on = tg < T && kc < wc;
   const int t = tg < T ? tg : 0;
   const float2* sb = spec + (size_t)b * wr * wc + (on ? kc : 0);
-  const float2* kb = kern ? kern + (size_t)k * wr * wc + (on ? kc : 0) : nullptr;
+  const int r0 = pmod(t - k0r, L);                    // T m < L: ir = r0 + T m, less L once
+  auto row = [&](int m) {
+    const int ir = r0 + T * m;
+    return ir >= L ? ir - L : ir;
+  };
+  // every load at a valid address, as in the forward's k_fp_bcols; kernel x
+  // spectrum as it forms it, so that Ec holds the same bits as its buffer.  One
+  // test of kern for all values: a test for each left the loads waiting for one
+  // another (coarse 200, one kernel of 121 columns: 11.4 us, 7.4 so).
   float2 v[V];
 #pragma unroll
-  for (int m = 0; m < V; ++m) {
-    const int ir = pmod(t + T * m - k0r, L);
-    // every load at a valid address, as in the forward's k_fp_bcols; kernel x
-    // spectrum as it forms it, so that Ec holds the same bits as its buffer
-    const bool in = on && ir < wr;
-    const size_t at = in ? (size_t)ir * wc : 0;
-    float2 a = sb[at];
-    if (kb) a = reg::mul_rn(kb[at], a);
-    v[m] = in ? a : make_float2(0.f, 0.f);
+  for (int m = 0; m < V; ++m) v[m] = sb[on && row(m) < wr ? row(m) * wc : 0];
+  if (kern) {
+    const float2* kb = kern + (size_t)k * wr * wc + (on ? kc : 0);
+#pragma unroll
+    for (int m = 0; m < V; ++m) v[m] = reg::mul_rn(kb[on && row(m) < wr ? row(m) * wc : 0], v[m]);
   }
+#pragma unroll
+  for (int m = 0; m < V; ++m)
+    if (!(on && row(m) < wr)) v[m] = make_float2(0.f, 0.f);
   P::template run_live_tab<false>(v, lds + g * (P::LDS | 1), t, twt, on);
   if (!on) return;
   float2* out = Ec + ((size_t)b * nk + k) * L * wc + kc;

@@ -61,6 +61,10 @@ struct FpCoh {
 };
 
 bool fp_image_size_ok(int n);            // n has a register transform
+// the LDS holds the row transform's tile of a window of wc columns (real rows go
+// through it in pairs): 692 of 1024 points, 356 of 512.  True for lengths
+// without a register transform, whose products have no tile.
+bool fp_rows_fit(int nx, int wc, bool real);
 bool fp_coarse_size_ok(int l);
 // Radices (R1, R2) of the two-stage register transform of length n, false
 // when n has none.  Twiddle tables of length n carry 2n entries: [0, n) holds

@@ -1112,11 +1112,17 @@ static int allow(K kernel, size_t bytes) {
   return OI_OK;
 }
 
+// transform scratch + output tile [wc][2G + 1], or [wc][G + 1] of complex rows
+template <class P>
+static size_t rows_tile_lds(int wc, bool real) {
+  constexpr int G = groups_per_block<P>();
+  return rows_lds<P>() + (size_t)wc * ((real ? 2 * G : G) + 1) * sizeof(float2);
+}
+
 template <class P>
 static int run_rows(const FpArgs& a, hipStream_t st) {
   constexpr int G = groups_per_block<P>();
-  // transform scratch + output tile [wc][2G + 1]
-  const size_t lds = rows_lds<P>() + (size_t)a.wc * (2 * G + 1) * sizeof(float2);
+  const size_t lds = rows_tile_lds<P>(a.wc, true);
   // narrow form: H output pairs per thread cover the window [-H T, H T]
   int narrow = 0;
   if constexpr (P::STAGES == 2) {
@@ -1151,9 +1157,8 @@ static int run_rows(const FpArgs& a, hipStream_t st) {
                        static_cast<const float*>(a.field), a.ny, a.k0c, a.wc, a.tw_x, a.T,
                        (int)(a.kind == kFieldLogits));
   } else {
-    // its tile is [wc][G + 1]: at 512 points and windows up to 90 columns two
-    // workgroups share a CU instead of one
-    const size_t lds_c = rows_lds<P>() + (size_t)a.wc * (G + 1) * sizeof(float2);
+    // at 512 points and windows up to 90 columns two workgroups share a CU
+    const size_t lds_c = rows_tile_lds<P>(a.wc, false);
     int rc = allow(k_fp_rows_c64<P>, lds_c);
     if (rc) return rc;
     const int items = (a.ny + G - 1) / G * a.nchan * a.batch;
@@ -1528,6 +1533,13 @@ bool fp_image_size_ok(int n) {
   OI_IMAGE_PLANS(X)
 #undef X
   return false;
+}
+
+bool fp_rows_fit(int nx, int wc, bool real) {
+#define X(NN, PT) if (nx == NN) return fp::rows_tile_lds<fp::PT>(wc, real) <= kLdsLimit;
+  OI_IMAGE_PLANS(X)
+#undef X
+  return true;
 }
 
 bool fp_coarse_size_ok(int l) {

@@ -1,0 +1,35 @@
+"""Windows too wide for the LDS tile of the register row transform (nx = 1024: 692
+columns, nx = 512: 356) on bands that a two-pass coarse grid holds: image and
+gradient against float64.  Tolerances as for the other image transforms of these
+lengths."""
+import numpy as np
+import pytest
+import torch
+
+from opticalimaging_amd import engine
+from test_gpu_dft_sizes import GRAD_TOL, IMAGE_TOL, _gradient, _image
+
+pytestmark = pytest.mark.gpu
+
+
+def _set(ny, nx, wr, wc, bc, K):
+    """Kernels of bc columns anywhere in the window, and their full spectra."""
+    rng = np.random.default_rng(wc)
+    win = np.zeros((K, wr, wc), np.complex64)
+    for k in range(K):
+        j = (wc - bc) * k // max(1, K - 1)
+        win[k, :, j:j + bc] = (rng.standard_normal((wr, bc)) + 1j * rng.standard_normal((wr, bc))) / 8
+    full = np.zeros((K, ny, nx), np.complex128)
+    full[np.ix_(range(K), (np.arange(wr) - wr // 2) % ny, (np.arange(wc) - wc // 2) % nx)] = win
+    return engine.KernelSet(torch.as_tensor(win).cuda(), -(wr // 2), -(wc // 2), ny, nx, band=(wr, bc)), full
+
+
+@pytest.mark.parametrize("ny,nx,wr,wc,bc", [(1024, 1024, 30, 800, 440), (1024, 1024, 30, 692, 440),
+                                            (512, 512, 21, 380, 190), (512, 512, 21, 356, 190)])
+def test_image(gpu, ny, nx, wr, wc, bc):
+    ks, full = _set(ny, nx, wr, wc, bc, 3)
+    h = np.random.default_rng(ny).random((2, ny, nx)).astype(np.float32)
+    img = engine.socs_image(torch.as_tensor(h).cuda(), ks, pack_real=False).cpu().numpy()
+    for b in range(2):
+        ref = _image(full, h[b])
+        assert np.max(np.abs(img[b] - ref)) <= IMAGE_TOL * ref.max()

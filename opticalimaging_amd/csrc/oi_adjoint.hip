@@ -563,7 +563,7 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
   if (g.direct) return fail(OI_ERR_INVALID, "adjoint: no band spectrum on a direct plan");
   const int wgc = 2 * g.qc + 1, wgr = 2 * g.qr + 1;
   float2* Tg = static_cast<float2*>(work);     // the first region of the work buffer
-  if (adj_image_ok(g)) {
+  if (adj_image_ok(g) && fp_rows_fit(g.nx, wgc, true)) {
     // the fast path's transforms of the image sizes (same spectrum, scale and layout)
     FpArgs a{};
     a.field = img;

@@ -1,5 +1,6 @@
 // C ABI: error state, twiddle tables, imaging plans and the imaging entry
 // points (spectrum window, coherent image, SOCS image, full spectrum).
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -268,10 +269,12 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
   // when the window folds onto them without collisions.
   if (g.path == 0 && fast) {
     const int need = (2 * band_r - 1) > (2 * band_c - 1) ? 2 * band_r - 1 : 2 * band_c - 1;
-    // coarse grids past one workgroup's reach, and those the one-pass kernel
-    // does not serve when the two-pass table has them (144)
+    // coarse grids past one workgroup's reach, the smallest that holds the band
+    // and the window, and those the one-pass kernel does not serve when the
+    // two-pass table has them (144)
     const int L1 = fp_coarse_choose(need);
-    const int L = need > 144 ? fp_two_pass_choose(need, generic ? kTwoPassBatch : INT_MAX)
+    const int least = std::max(need, std::max(g.wr, g.wc));
+    const int L = need > 144 ? fp_two_pass_choose(least, generic ? kTwoPassBatch : INT_MAX)
                              : (L1 > 0 && !fp_one_pass_ok(L1) && fp_two_pass_size_ok(L1) ? L1 : 0);
     if (L > 0 && L < g.ny && L < g.nx && g.wr <= L && g.wc <= L &&
         fp_two_pass_lds(L) <= kLdsLimit &&

@@ -1,5 +1,6 @@
-"""Windows too wide for the LDS tile of the register row transform (nx = 1024: 692
-columns, nx = 512: 356) on bands that a two-pass coarse grid holds: image and
+"""Windows much wider than a kernel's band: past the smallest coarse grid of the
+band (the next one that holds the window serves), and too wide for the LDS tile of
+the register row transform (nx = 1024: 692 columns, nx = 512: 356).  Image and
 gradient against float64.  Tolerances as for the other image transforms of these
 lengths."""
 import numpy as np
@@ -33,6 +34,21 @@ def test_image(gpu, ny, nx, wr, wc, bc):
     for b in range(2):
         ref = _image(full, h[b])
         assert np.max(np.abs(img[b] - ref)) <= IMAGE_TOL * ref.max()
+
+
+@pytest.mark.parametrize("ny,nx,wr,wc,bc,coarse", [(512, 512, 30, 234, 90, 256), (648, 540, 31, 330, 95, 400),
+                                                   (1024, 640, 33, 401, 150, 450), (2048, 1024, 9, 577, 110, 900)])
+def test_coarse_grid_of_the_window(gpu, ny, nx, wr, wc, bc, coarse):
+    ks, full = _set(ny, nx, wr, wc, bc, 3)
+    info = engine.plan_for(ks, 1, 1).info()
+    assert (info["path"], info["lr"]) == (2, coarse)
+    h, g = np.random.default_rng(wc).random((2, ny, nx)).astype(np.float32)
+    hd, gd = torch.as_tensor(h[None]).cuda(), torch.as_tensor(g[None]).cuda()
+    ref = _image(full, h)
+    assert np.max(np.abs(engine.socs_image(hd, ks, pack_real=False).cpu().numpy()[0] - ref)) <= IMAGE_TOL * ref.max()
+    ref = _gradient(full, h, g)
+    out = engine.socs_adjoint(hd, gd, ks, pack_real=False).cpu().numpy()[0]
+    assert np.max(np.abs(out - ref)) <= GRAD_TOL * np.abs(ref).max()
 
 
 @pytest.mark.parametrize("ny,nx,wr,wc,bc", [(512, 512, 21, 190, 190), (1024, 1024, 30, 800, 440)])

@@ -563,7 +563,7 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
   if (g.direct) return fail(OI_ERR_INVALID, "adjoint: no band spectrum on a direct plan");
   const int wgc = 2 * g.qc + 1, wgr = 2 * g.qr + 1;
   float2* Tg = static_cast<float2*>(work);     // the first region of the work buffer
-  if (adj_image_ok(g) && fp_rows_fit(g.nx, wgc, true)) {
+  if (adj_image_ok(g)) {
     // the fast path's transforms of the image sizes (same spectrum, scale and layout)
     FpArgs a{};
     a.field = img;
@@ -580,6 +580,8 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
     a.wc = wgc;
     a.tw_x = g.fx.tw;
     a.tw_y = g.fy.tw;
+    a.fx = g.fx;
+    a.fy = g.fy;
     a.tab_x = g.tab_x;
     a.tab_y = g.tab_y;
     a.T = Tg;
@@ -595,7 +597,8 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
 
 bool adjoint_chain_ok(const AdjGeom& g) {
   const int qrm = adj_half(g.k0r, g.wr), qcm = adj_half(g.k0c, g.wc);
-  return adj_image_ok(g) && 2 * qrm + 1 <= g.ny && 2 * qcm + 1 <= g.nx;
+  return adj_image_ok(g) && fp_band_ok(g.ny, g.nx, qrm, qcm) && 2 * qrm + 1 <= g.ny &&
+         2 * qcm + 1 <= g.nx;
 }
 
 int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int batch,
@@ -704,6 +707,8 @@ int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int ba
     a.qc = qcm;
     a.tw_x = g.fx.tw;
     a.tw_y = g.fy.tw;
+    a.fx = g.fx;
+    a.fy = g.fy;
     a.tab_x = g.tab_x;
     a.tab_y = g.tab_y;
     a.Ihat = F;

@@ -479,6 +479,8 @@ static FpArgs fast_args(oi_plan* p, int batch, hipStream_t st) {
   a.qc = g.qc;
   a.tw_x = p->fx.tw;
   a.tw_y = p->fy.tw;
+  a.fx = p->fx;
+  a.fy = p->fy;
   a.tw_l = p->flr.tw;
   a.tab_x = p->tab_x;
   a.tab_y = p->tab_y;
@@ -556,11 +558,7 @@ static int spectrum_impl(oi_plan* p, const void* field, int kind, int cin, const
   int rc;
   const oi_geometry& g = p->g;
   mark(p, 0, st);
-  // windows past the register row transform's tile take the generic transforms
-  const bool real = kind == OI_FIELD_REAL || kind == kFieldLogits;
-  const bool fits = fp_rows_fit(g.nx, g.wc, real);
-  if (!fits && kind == kFieldLogits) return fail(OI_ERR_UNSUPPORTED, "window without the logits pass");
-  if (g.path && fits) {
+  if (g.path) {
     FpArgs a = fast_args(p, batch, st);
     a.field = field;
     a.kind = kind;
@@ -882,7 +880,7 @@ extern "C" int oi_socs_residual_adjoint(oi_plan* p, const float* mask, int batch
 // without the image (oi_ilt.hip states the identities).
 static bool band_residual_ok(const oi_plan* p) {
   // the loss's partial sums go to p->part (ny per image)
-  return p->g.nchan == 1 && !p->g.direct && residual_fused(p) && fp_rows_fit(p->g.nx, p->g.wc, true) &&
+  return p->g.nchan == 1 && !p->g.direct && residual_fused(p) && fp_rows_ok(p->g.nx, p->g.wc, true) &&
          ilt_band_blocks(p->g.qr, p->g.qc) <= p->g.ny;
 }
 

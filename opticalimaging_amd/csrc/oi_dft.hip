@@ -591,6 +591,23 @@ int dft_table_build(const float2* tw, int n, int amax, float* mem, DftTable& t, 
   return OI_OK;
 }
 
+// A product's time grows with the window, a transform's hardly.  8 x 1200 x 1200,
+// us as product and as transform, at windows of 240, 360, 480, 720 and 960: real
+// rows 42, 60, 80, 111, 143 and 79, 81, 85, 91, 112; complex rows 127, 187, 243,
+// 354, 462 and 128, 131, 135, 170, 192; spectrum columns 34, 69, 102, 214, 349 and
+// 39, 44, 60, 88, 118.  Odd lengths fold once instead of twice: real rows of 26 x
+// 675 x 675 at 236, 270 and 337 75, 107, 105 and 77, 77, 82; of 9 x 1125 x 1125 at
+// 281, 337 and 393 82, 82, 117 and 79, 80, 81.
+bool dft_window_ok(int n, int w, bool real) { return w <= (real && n % 2 == 0 ? 540 : 256); }
+
+// Band columns and image rows together, us as products and as transforms: 33 x 600
+// x 600 at half-widths of 150, 180, 210 and 240 124, 157, 207, 250 and 159, 160,
+// 188, 207; 8 x 1200 x 1200 at 180, 240 and 300 90, 136, 162 and 109, 140, 153; 3 x
+// 1920 x 1920 at 288 and 384 112, 173 and 110, 147.  Odd: 26 x 675 x 675 at 67, 101
+// and 135 80, 110, 154 and 100, 104, 143; 22 x 729 x 729 at 109 and 182 99, 177 and
+// 121, 166; 9 x 1125 x 1125 at 112 and 168 94, 145 and 99, 108.
+bool dft_band_ok(int n, int q) { return q <= (n % 2 ? 112 : 220); }
+
 int dft_rows(const FpArgs& a, hipStream_t st) {
   if (a.kind == kFieldLogits) return fail(OI_ERR_UNSUPPORTED, "image length without the logits pass");
   if (a.kind != OI_FIELD_REAL) {

@@ -28,6 +28,7 @@ struct CohArgs {
 
 struct InterpArgs {
   const float2* R;  // [B][groups][lr][qc+1]
+  const float2* band = nullptr;  // non-null, in R's place: [B][qc+1][2qr+1], scaled
   int groups;
   int lr, lc, ny, nx, qr, qc;
   float scale;      // 1 / (lr lc)

@@ -175,8 +175,8 @@ class AbbeSourceProblem:
             raise ValueError("grad_image must have the image's shape")
         img = self.image(V)
         lib = nat.load()
-        # zeros: the sum over an empty focus range
-        out = torch.zeros(self.nsrc, dtype=torch.float64, device=self.dev)
+        # the first focus writes it; the sum over an empty focus range is zero
+        out = (torch.empty if self.foci else torch.zeros)(self.nsrc, dtype=torch.float64, device=self.dev)
         work = torch.empty(int(lib.oi_source_gradient_work_bytes(self.nx, self.Lr, self.Lc)),
                            dtype=torch.uint8, device=self.dev)
         for i in range(len(self.foci)):

@@ -13,6 +13,7 @@ struct AdjGeom {
   int direct;
   FftDesc fx, fy, flr, flc;
   DftTable tab_x, tab_y;
+  int images;   // the plan's batch
 };
 
 size_t adjoint_work_bytes(const AdjGeom& g, int batch, int nkern);

@@ -582,6 +582,7 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
     a.tw_y = g.fy.tw;
     a.fx = g.fx;
     a.fy = g.fy;
+    a.images = g.images;
     a.tab_x = g.tab_x;
     a.tab_y = g.tab_y;
     a.T = Tg;
@@ -597,8 +598,7 @@ int adjoint_band_spectrum(const AdjGeom& g, const float* img, int batch, void* w
 
 bool adjoint_chain_ok(const AdjGeom& g) {
   const int qrm = adj_half(g.k0r, g.wr), qcm = adj_half(g.k0c, g.wc);
-  return adj_image_ok(g) && fp_band_ok(g.ny, g.nx, qrm, qcm) && 2 * qrm + 1 <= g.ny &&
-         2 * qcm + 1 <= g.nx;
+  return adj_image_ok(g) && 2 * qrm + 1 <= g.ny && 2 * qcm + 1 <= g.nx;
 }
 
 int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int batch,
@@ -709,6 +709,7 @@ int launch_adjoint(const AdjGeom& g, const float* gI, const float2* spec, int ba
     a.tw_y = g.fy.tw;
     a.fx = g.fx;
     a.fy = g.fy;
+    a.images = g.images;
     a.tab_x = g.tab_x;
     a.tab_y = g.tab_y;
     a.Ihat = F;

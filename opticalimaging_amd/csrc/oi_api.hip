@@ -102,6 +102,7 @@ constexpr int kStages = 5;
 
 struct oi_plan {
   oi_geometry g;
+  int images = 0;           // the batch that its kernels are chosen for
   FftDesc fx, fy, flr, flc, frows;
   TwiddlePool pool;
   float2* T = nullptr;
@@ -379,6 +380,7 @@ extern "C" int oi_plan_create(oi_geometry* geo, oi_plan** out) {
   oi_plan* p = new (std::nothrow) oi_plan();
   if (!p) return fail(OI_ERR_NOMEM, "plan_create: host allocation failed");
   p->g = g;
+  p->images = g.max_batch;
   int sizes[5] = {g.nx, g.ny, lr, lc, rows};
   FftDesc d[5];
   rc = make_twiddles(sizes, 5, d, p->pool);
@@ -481,6 +483,7 @@ static FpArgs fast_args(oi_plan* p, int batch, hipStream_t st) {
   a.tw_y = p->fy.tw;
   a.fx = p->fx;
   a.fy = p->fy;
+  a.images = p->images;
   a.tw_l = p->flr.tw;
   a.tab_x = p->tab_x;
   a.tab_y = p->tab_y;
@@ -853,6 +856,7 @@ static AdjGeom adj_geom(const oi_plan* p) {
   a.flc = p->flc;
   a.tab_x = p->tab_x;
   a.tab_y = p->tab_y;
+  a.images = p->images;
   return a;
 }
 
@@ -880,7 +884,7 @@ extern "C" int oi_socs_residual_adjoint(oi_plan* p, const float* mask, int batch
 // without the image (oi_ilt.hip states the identities).
 static bool band_residual_ok(const oi_plan* p) {
   // the loss's partial sums go to p->part (ny per image)
-  return p->g.nchan == 1 && !p->g.direct && residual_fused(p) && fp_rows_ok(p->g.nx, p->g.wc, true) &&
+  return p->g.nchan == 1 && !p->g.direct && residual_fused(p) && fp_rows_fit(p->g.nx, p->g.wc, true) &&
          ilt_band_blocks(p->g.qr, p->g.qc) <= p->g.ny;
 }
 
@@ -1153,6 +1157,7 @@ extern "C" int oi_socs_image_noalloc(const oi_geometry* geo, const void* field, 
   oi_plan pl;  // on the stack: pointers into `scratch`, nothing owned
   pl.g = g;
   pl.g.max_batch = chunk;
+  pl.images = batch;
   for (int i = 0; i < 5; ++i) {
     d[i].tw = reinterpret_cast<const float2*>(base + tw_off[i]);
     bool first = true;

@@ -23,11 +23,10 @@ struct FpArgs;
 size_t dft_table_bytes(int n, int amax);
 int dft_table_build(const float2* tw, int n, int amax, float* mem, DftTable& t, hipStream_t st);
 
-// A forward sum to a window of w orders is the faster as a product (the general
-// transforms take the others).
-bool dft_window_ok(int n, int w, bool real);
-// Likewise the image from a band of half-width q.
-bool dft_band_ok(int n, int q);
+// The stage is the faster as a product (the general transforms take the others).
+bool dft_rows_ok(const FpArgs& a);
+bool dft_cols_ok(const FpArgs& a);
+bool dft_ucols_ok(const FpArgs& a);
 
 // The launches of the register-transform kernels of the same stage.
 int dft_rows(const FpArgs& a, hipStream_t st);

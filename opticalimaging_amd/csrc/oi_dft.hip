@@ -591,22 +591,38 @@ int dft_table_build(const float2* tw, int n, int amax, float* mem, DftTable& t, 
   return OI_OK;
 }
 
-// A product's time grows with the window, a transform's hardly.  8 x 1200 x 1200,
-// us as product and as transform, at windows of 240, 360, 480, 720 and 960: real
-// rows 42, 60, 80, 111, 143 and 79, 81, 85, 91, 112; complex rows 127, 187, 243,
-// 354, 462 and 128, 131, 135, 170, 192; spectrum columns 34, 69, 102, 214, 349 and
-// 39, 44, 60, 88, 118.  Odd lengths fold once instead of twice: real rows of 26 x
-// 675 x 675 at 236, 270 and 337 75, 107, 105 and 77, 77, 82; of 9 x 1125 x 1125 at
-// 281, 337 and 393 82, 82, 117 and 79, 80, 81.
-bool dft_window_ok(int n, int w, bool real) { return w <= (real && n % 2 == 0 ? 540 : 256); }
+// A product's time grows with the orders, a transform's hardly; but where there is
+// too little to transform the general kernels leave the chip idle (about 25 us), and
+// a product of any width is ahead (one image of 405 x 405: rows 7 us, columns 10).
+// us as products and as transforms, 9 x 1125 x 1125 and 8 x 1200 x 1200:
+//   real rows, windows 281, 450, 787  81, 120, 192 and 77, 94, 112;  300, 480, 840
+//     60, 78, 132 and 80, 99, 114
+//   complex rows, the same  178, 296, 482 and 131, 167, 178;  153, 243, 411 and 133,
+//     168, 183;  at 112 and 120  59 and 128;  70 and 126
+//   spectrum columns, the same  49, 123, 339 and 40, 60, 106;  47, 102, 299 and 42,
+//     60, 107
+//   band columns, |qr| up to 112, 191, 281  33, 69, 141 and 25, 42, 52;  120, 204,
+//     300  26, 61, 92 and 25, 45, 55
+// Of 472 windows, batches and sizes from 225 to 1920 the choice takes 0.5 % (real
+// rows), 1.2, 1.1 and 1.7 % longer than the better form of each.  It goes by the
+// plan's batch: an image is the same in every call.
+static bool wide(int orders, int most, long long values, long long enough) {
+  return orders > most && values >= enough;
+}
 
-// Band columns and image rows together, us as products and as transforms: 33 x 600
-// x 600 at half-widths of 150, 180, 210 and 240 124, 157, 207, 250 and 159, 160,
-// 188, 207; 8 x 1200 x 1200 at 180, 240 and 300 90, 136, 162 and 109, 140, 153; 3 x
-// 1920 x 1920 at 288 and 384 112, 173 and 110, 147.  Odd: 26 x 675 x 675 at 67, 101
-// and 135 80, 110, 154 and 100, 104, 143; 22 x 729 x 729 at 109 and 182 99, 177 and
-// 121, 166; 9 x 1125 x 1125 at 112 and 168 94, 145 and 99, 108.
-bool dft_band_ok(int n, int q) { return q <= (n % 2 ? 112 : 220); }
+bool dft_rows_ok(const FpArgs& a) {
+  const long long values = (long long)a.ny * a.nx * a.images;
+  if (a.kind == OI_FIELD_C64_CHLAST) return !wide(a.wc, 256, values * a.nchan, 1000000);
+  return !wide(a.wc, a.nx % 2 ? 256 : 600, values / 2, 1000000);
+}
+
+bool dft_cols_ok(const FpArgs& a) {
+  return !wide(a.wr, 256, (long long)a.wc * a.ny * a.nchan * a.images, 600000);
+}
+
+bool dft_ucols_ok(const FpArgs& a) {
+  return !wide(2 * a.qr + 1, a.ny % 2 ? 160 : 256, (long long)(a.qc + 1) * a.ny * a.images, 300000);
+}
 
 int dft_rows(const FpArgs& a, hipStream_t st) {
   if (a.kind == kFieldLogits) return fail(OI_ERR_UNSUPPORTED, "image length without the logits pass");

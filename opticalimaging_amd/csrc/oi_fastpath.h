@@ -25,6 +25,7 @@ struct FpArgs {
   int kind, cin, nchan;
   Chans chans;
   int batch, ny, nx;
+  int images;     // the plan's batch: what its kernels are chosen for
   int k0r, wr, k0c, wc;
   int L;          // square coarse grid
   int qr, qc;     // band half-widths
@@ -62,13 +63,9 @@ struct FpCoh {
 };
 
 bool fp_image_size_ok(int n);            // n has a register transform
-// The fast form of the row stage serves a window of wc columns: the LDS holds the
-// register transform's tile (real rows go through it in pairs: 692 columns of 1024
-// points, 356 of 512), or the product is the faster one.  Likewise the columns.
-bool fp_rows_ok(int nx, int wc, bool real);
-bool fp_cols_ok(int ny, int wr);
-// Likewise the image from a band |qr| <= qr, q <= qc, both stages together.
-bool fp_band_ok(int ny, int nx, int qr, int qc);
+// The LDS holds the register row transform's tile of a window of wc columns (real
+// rows go through it in pairs: 692 of 1024 points, 356 of 512).
+bool fp_rows_fit(int nx, int wc, bool real);
 bool fp_coarse_size_ok(int l);
 // Radices (R1, R2) of the two-stage register transform of length n, false
 // when n has none.  Twiddle tables of length n carry 2n entries: [0, n) holds
@@ -80,15 +77,15 @@ int fp_coarse_choose(int need);          // smallest table size >= need, 0 if no
 size_t fp_coherent_lds(int L, int wr, int wc);
 int fp_coherent_rows_fit(int L);
 bool fp_one_pass_ok(int L);             // the one-pass coherent kernel serves L
-// marks stage 1 between its launches; a stage whose fast form does not serve the
-// window takes the general transforms (the same values to rounding, in the same
-// layout)
+// marks stage 1 between its launches; a stage whose window does not fit its
+// register transform, or is too wide for its product, takes the general transforms
+// (the same values to rounding, in the same layout)
 int fp_spectrum(const FpArgs& a, hipStream_t st);
 int fp_coherent(const FpArgs& a, const FpCoh& c, hipStream_t st);   // the one-pass coherent sum to R
 int fp_interp(const FpArgs& a, int groups, hipStream_t st);      // marks stages 4, 5
 // the band Ihat from partial sums R (the first kernel of fp_interp)
 int fp_band(const FpArgs& a, int groups, hipStream_t st);
-// interpolation column and row transforms of a band already in a.Ihat (fp_band_ok)
+// interpolation column and row transforms of a band already in a.Ihat
 int fp_band_image(const FpArgs& a, hipStream_t st);
 // row sets per workgroup and workgroups per image of the image-row pass for a
 // batch (its residual form writes one partial sum per workgroup)

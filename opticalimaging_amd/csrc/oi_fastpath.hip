@@ -1448,6 +1448,8 @@ static int stage_cols(const FpArgs& a, hipStream_t st) {
 #undef X
 }
 static int stage_ucols(const FpArgs& a, hipStream_t st) {
+  if (a.tab_y.fcos && !dft_ucols_ok(a))
+    return launch_band_cols(a.Ihat, a.qc + 1, a.qr, a.fy, a.batch, a.U, st);
 #define X(NN, PT) if (a.ny == NN) rc = fp::run_ucols<fp::PT>(a, st);
   OI_IMAGE_STAGE(a.ny, a.tab_y, X, dft_ucols)
 #undef X
@@ -1461,19 +1463,6 @@ static int stage_urows(const FpArgs& a, hipStream_t st) {
 int fp_interp(const FpArgs& a, int groups, hipStream_t st) {
   int rc = fp_band(a, groups, st);
   if (rc) return rc;
-  if (!fp_band_ok(a.ny, a.nx, a.qr, a.qc)) {   // never a residual's image: its lengths have transforms
-    InterpArgs g{};
-    g.band = a.Ihat;
-    g.ny = a.ny;
-    g.nx = a.nx;
-    g.qr = a.qr;
-    g.qc = a.qc;
-    g.fny = a.fy;
-    g.fnx = a.fx;
-    g.U = a.U;
-    g.out = a.out;
-    return launch_interp(g, a.batch, st, a.mark, a.mark_ctx);
-  }
   rc = stage_ucols(a, st);
   if (rc) return rc;
   if (a.mark) a.mark(a.mark_ctx, 4);
@@ -1548,17 +1537,11 @@ bool fp_image_size_ok(int n) {
   return false;
 }
 
-bool fp_rows_ok(int nx, int wc, bool real) {
+bool fp_rows_fit(int nx, int wc, bool real) {
 #define X(NN, PT) if (nx == NN) return fp::rows_tile_lds<fp::PT>(wc, real) <= kLdsLimit;
   OI_IMAGE_PLANS(X)
 #undef X
-  return dft_window_ok(nx, wc, real);
-}
-
-bool fp_cols_ok(int ny, int wr) { return fp_image_size_ok(ny) || dft_window_ok(ny, wr, false); }
-
-bool fp_band_ok(int ny, int nx, int qr, int qc) {
-  return (fp_image_size_ok(ny) || dft_band_ok(ny, qr)) && (fp_image_size_ok(nx) || dft_band_ok(nx, qc));
+  return true;
 }
 
 bool fp_coarse_size_ok(int l) {
@@ -1609,7 +1592,7 @@ int fp_coherent_rows_fit(int L) {
 int fp_spectrum(const FpArgs& a, hipStream_t st) {
   const bool real = a.kind != OI_FIELD_C64_CHLAST;
   int rc;
-  if (fp_rows_ok(a.nx, a.wc, real))
+  if (a.tab_x.fcos ? dft_rows_ok(a) : fp_rows_fit(a.nx, a.wc, real))
     rc = stage_rows(a, st);
   else if (a.kind == kFieldLogits)
     rc = fail(OI_ERR_UNSUPPORTED, "window without the logits pass");
@@ -1618,7 +1601,7 @@ int fp_spectrum(const FpArgs& a, hipStream_t st) {
                           a.wc, a.T, st);
   if (rc) return rc;
   if (a.mark) a.mark(a.mark_ctx, 1);
-  if (fp_cols_ok(a.ny, a.wr)) return stage_cols(a, st);
+  if (!a.tab_y.fcos || dft_cols_ok(a)) return stage_cols(a, st);
   return launch_spec_cols(a.T, a.batch * a.nchan, a.ny, a.nx, a.fy, a.k0r, a.wr, a.wc, a.spec, st);
 }
 

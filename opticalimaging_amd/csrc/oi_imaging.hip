@@ -309,26 +309,28 @@ __global__ __launch_bounds__(kThreads) void k_interp_cols(InterpArgs A, int ncol
 }
 
 // Rows: two image rows per complex transform (Hermitian extension of U).
-// The same from a band that another kernel left: Ihat[img][q][qr + qrm].
-__global__ __launch_bounds__(kThreads) void k_band_cols(InterpArgs A, int ncol) {
+// The columns from a band that another kernel left, Ihat[img][q][qr + qrm], in the
+// layout of the fast paths' row stages: U[img][q][y].
+__global__ __launch_bounds__(kThreads) void k_band_cols(const float2* __restrict__ Ihat, int nq, int qrm,
+                                                        FftDesc fy, int ncol, float2* __restrict__ U) {
   extern __shared__ float2 lds[];
-  const int ny = A.ny, nq = A.qc + 1, nb = 2 * A.qr + 1;
-  float2* o = lds;
-  float2* z = lds + ncol * ny;
+  const int ny = fy.n, nb = 2 * qrm + 1;
+  float2* a = lds;
+  float2* t = lds + ncol * ny;
   const int img = blockIdx.y, q0 = blockIdx.x * ncol;
+  const float2* src = Ihat + ((size_t)img * nq + q0) * nb;
   for (int e = threadIdx.x; e < ncol * ny; e += blockDim.x) {
     const int j = e / ny, y = e - j * ny;
-    const int k = y <= A.qr ? y + A.qr : y - ny + A.qr;      // negative: outside the band
+    const int k = y <= qrm ? y + qrm : y - ny + qrm;         // negative: outside the band
     const bool in = k >= 0 && q0 + j < nq;
-    const float2 v = A.band[((size_t)img * nq + (in ? q0 + j : 0)) * nb + (in ? k : 0)];
-    o[e] = in ? v : make_float2(0.f, 0.f);
+    const float2 v = src[in ? j * nb + k : 0];
+    a[e] = in ? v : make_float2(0.f, 0.f);
   }
   __syncthreads();
-  const float2* w = block_fft<false>(o, z, A.fny, ncol, ny);
-  for (int e = threadIdx.x; e < ncol * ny; e += blockDim.x) {
-    const int y = e / ncol, j = e - y * ncol;
-    if (q0 + j < nq) A.U[((size_t)img * ny + y) * nq + q0 + j] = w[j * ny + y];
-  }
+  const float2* z = block_fft<false>(a, t, fy, ncol, ny);
+  float2* dst = U + ((size_t)img * nq + q0) * ny;
+  const int end = (nq - q0 < ncol ? nq - q0 : ncol) * ny;
+  for (int e = threadIdx.x; e < end; e += blockDim.x) dst[e] = z[e];
 }
 
 __global__ __launch_bounds__(kThreads) void k_interp_rows(InterpArgs A, int nfft) {
@@ -368,15 +370,26 @@ __global__ __launch_bounds__(kThreads) void k_interp_rows(InterpArgs A, int nfft
   }
 }
 
+int launch_band_cols(const float2* Ihat, int nq, int qrm, const FftDesc& fy, int batch, float2* U,
+                     hipStream_t st) {
+  const int ncol = per_block(fy.n);
+  const size_t lds = fft_lds(ncol, fy.n);
+  int rc = allow_lds(k_band_cols, lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_band_cols, dim3((nq + ncol - 1) / ncol, batch), dim3(kThreads), lds, st, Ihat, nq, qrm,
+                     fy, ncol, U);
+  OI_LAUNCH_CHECK("band_cols");
+  return OI_OK;
+}
+
 int launch_interp(const InterpArgs& a, int batch, hipStream_t st, StageMark mark, void* ctx) {
-  const int L = a.lr > a.ny && !a.band ? a.lr : a.ny;
+  const int L = a.lr > a.ny ? a.lr : a.ny;
   const int ncol = per_block(L);
   size_t lds = fft_lds(ncol, L);
-  const auto cols = a.band ? k_band_cols : k_interp_cols;
-  int rc = allow_lds(cols, lds);
+  int rc = allow_lds(k_interp_cols, lds);
   if (rc) return rc;
   dim3 g1((a.qc + 1 + ncol - 1) / ncol, batch);
-  hipLaunchKernelGGL(cols, g1, dim3(kThreads), lds, st, a, ncol);
+  hipLaunchKernelGGL(k_interp_cols, g1, dim3(kThreads), lds, st, a, ncol);
   OI_LAUNCH_CHECK("interp_cols");
   if (mark) mark(ctx, 4);
   const int nfft = per_block(a.nx);

@@ -28,7 +28,6 @@ struct CohArgs {
 
 struct InterpArgs {
   const float2* R;  // [B][groups][lr][qc+1]
-  const float2* band = nullptr;  // non-null, in R's place: [B][qc+1][2qr+1], scaled
   int groups;
   int lr, lc, ny, nx, qr, qc;
   float scale;      // 1 / (lr lc)
@@ -47,6 +46,9 @@ int launch_coherent(const CohArgs& a, int batch, hipStream_t st);
 // mark(ctx, stage) is called after each of the two launches (stages 4, 5).
 typedef void (*StageMark)(void* ctx, int stage);
 int launch_interp(const InterpArgs& a, int batch, hipStream_t st, StageMark mark, void* ctx);
+// U[img][q][y] = sum_{|qr| <= qrm} Ihat[img][q][qr + qrm] e^{-2 pi i qr y / ny}
+int launch_band_cols(const float2* Ihat, int nq, int qrm, const FftDesc& fy, int batch, float2* U,
+                     hipStream_t st);
 int launch_group_sum(const float* Ic, int batch, int groups, size_t per_image, float* out,
                      hipStream_t st);
 int launch_full_rows(const void* field, int kind, int cin, const int* chans, int nchan,

@@ -74,44 +74,52 @@ def test_optimisation_steps(gpu):
 
 
 # windows on both sides of where products give way to transforms: real rows, complex
-# rows and columns, even and odd lengths
-@pytest.mark.parametrize("ny,nx,wr,wc,bc", [(600, 640, 256, 540, 200), (600, 640, 257, 541, 200),
-                                            (405, 405, 256, 256, 120), (405, 405, 257, 257, 120),
+# rows and columns, even and odd lengths, plans of many images and of one
+@pytest.mark.parametrize("ny,nx,wr,wc,bc", [(960, 1000, 256, 600, 200), (960, 1000, 257, 601, 200),
+                                            (600, 405, 256, 256, 120), (405, 600, 257, 257, 120),
                                             (729, 640, 256, 257, 120), (640, 729, 257, 256, 120)])
-@pytest.mark.parametrize("real", [True, False])
-def test_products_and_transforms(gpu, ny, nx, wr, wc, bc, real):
+@pytest.mark.parametrize("real,most", [(True, 16), (False, 16), (True, 2)])
+def test_products_and_transforms(gpu, ny, nx, wr, wc, bc, real, most):
     from opticalimaging_amd import _native as nat
     rng = np.random.default_rng(wc)
     f = rng.standard_normal((2, ny, nx, 2)).astype(np.float32)
     h = f[..., 0] if real else f[..., 0] + 1j * f[..., 1]
-    plan = engine.Plan(ny, nx, -(wr // 2), wr, -(wc // 2), wc, max_batch=2, band_r=min(wr, bc), band_c=bc, max_kernels=1)
+    plan = engine.Plan(ny, nx, -(wr // 2), wr, -(wc // 2), wc, max_batch=most, band_r=bc, band_c=bc, max_kernels=1)
     assert plan.info()["path"] == 2
-    out = torch.empty((2, wr, wc), dtype=torch.complex64, device="cuda")
     hd = torch.as_tensor(h if real else h[..., None]).cuda()
     chans, keep = nat.int_array([0])
     kind = nat.OI_FIELD_REAL if real else nat.OI_FIELD_C64_CHLAST
-    nat.check(nat.load().oi_spectrum_window(plan.handle, nat.ptr(hd), kind, 1, chans, 2, nat.ptr(out), nat.stream()))
+
+    def spectrum(x):
+        out = torch.empty((len(x), wr, wc), dtype=torch.complex64, device="cuda")
+        nat.check(nat.load().oi_spectrum_window(plan.handle, nat.ptr(x), kind, 1, chans, len(x), nat.ptr(out),
+                                                nat.stream()))
+        return out
+    out = spectrum(hd)
     ref = np.fft.ifft2(h.astype(np.complex128))
     ref = ref[:, (np.arange(wr) - wr // 2) % ny][:, :, (np.arange(wc) - wc // 2) % nx]
     # two transforms of one to seven hundred terms: half the image's tolerance
     assert np.max(np.abs(out.cpu().numpy() - ref)) <= IMAGE_TOL / 2 * np.abs(ref).max()
+    assert torch.equal(spectrum(hd[1:]), out[1:])          # whatever the call's batch
 
 
-@pytest.mark.parametrize("ny,nx,q", [(600, 640, 220), (600, 640, 221), (405, 675, 112), (405, 675, 113),
-                                     (512, 675, 113), (675, 512, 113), (729, 600, 90)])
+@pytest.mark.parametrize("ny,nx,q", [(600, 640, 127), (600, 640, 128), (405, 675, 79), (405, 675, 80),
+                                     (512, 675, 128), (675, 512, 128), (1125, 600, 90)])
 def test_band_products_and_transforms(gpu, ny, nx, q):
-    """Bands on both sides of where the image's products give way to transforms, by
-    the length of either axis, and the gradient's last stage with them."""
-    ks, full = _set(ny, nx, 2 * q + 1 if ny < 512 else 21, 2 * q + 1, q + 1, 2)
-    ks = engine.KernelSet(ks.win, ks.k0r, ks.k0c, ny, nx, band=(min(q + 1, ks.wr), q + 1))
-    if ny < 512:                         # rows of one band too
-        ks.win[:, q + 1:] = 0
-        full[:, (np.arange(q + 1, 2 * q + 1) - q) % ny] = 0
-    assert engine.plan_for(ks, 1, 2).info()["path"] == 2
-    h, g = np.random.default_rng(q).random((2, 2, ny, nx)).astype(np.float32)
+    """Bands on both sides of where the products of their columns give way to
+    transforms, and the gradient's last stage with them."""
+    rng = np.random.default_rng(q)
+    w = 2 * q + 1
+    win = np.zeros((2, w, w), np.complex64)
+    win[:, :q + 1, :q + 1] = (rng.standard_normal((2, q + 1, q + 1)) + 1j * rng.standard_normal((2, q + 1, q + 1))) / 8
+    full = np.zeros((2, ny, nx), np.complex128)
+    full[np.ix_(range(2), (np.arange(w) - q) % ny, (np.arange(w) - q) % nx)] = win
+    ks = engine.KernelSet(torch.as_tensor(win).cuda(), -q, -q, ny, nx, band=(q + 1, q + 1))
+    assert engine.plan_for(ks, 1, 10).info()["path"] == 2
+    h, g = rng.random((2, 10, ny, nx)).astype(np.float32)
     img = engine.socs_image(torch.as_tensor(h).cuda(), ks, pack_real=False).cpu().numpy()
     grad = engine.socs_adjoint(torch.as_tensor(h).cuda(), torch.as_tensor(g).cuda(), ks, pack_real=False).cpu().numpy()
-    for b in range(2):
+    for b in (0, 9):
         ref = _image(full, h[b])
         assert np.max(np.abs(img[b] - ref)) <= IMAGE_TOL * ref.max()
         ref = _gradient(full, h[b], g[b])

@@ -77,8 +77,8 @@ int oi_version(void);
  * Outputs filled by the library: max_groups (when 0), lr, lc, rows (coarse rows per workgroup),
  * direct (1 when the coarse grid equals the image grid), qr, qc (half-widths
  * of the intensity band carried from the coarse to the image grid), path
- * (1 when the image sizes and a square coarse grid have compile-time-size
- * kernels; then lr = lc).
+ * (1 or 2 when the coarse grid is square and has compile-time-size kernels; then
+ * lr = lc).
  *
  * The coarse grid must satisfy lr >= 2*band_r - 1 where band_r is the widest
  * row extent of any single coherent kernel's support (and likewise for
@@ -95,10 +95,14 @@ typedef struct oi_geometry {
   int rows;
   int direct;
   int qr, qc;
-  int path;       /* 0: generic kernels, or (image lengths without
-                   * compile-time transforms) matrix products; 1: compile-time-size kernels, one
-                     pass over the coarse grid; 2: compile-time-size kernels,
-                     two-pass coherent sum (coarse 144, 256 or 512)          */
+  int path;       /* 1, 2: compile-time-size coarse kernels.  1: coarse 16 to
+                     128, summed in one pass (100 and 128 in two), image lengths
+                     with compile-time transforms; 2: coarse 144, 200, 256, 324,
+                     400, 450, 512, 576, 900 or 1024, summed in two passes, any
+                     image length.  0: neither; the generic kernels, except
+                     that the coarse grids of 1 behind image lengths without
+                     compile-time transforms are reported so too (they have none
+                     of the fused image passes)                              */
   int max_kernels;
 } oi_geometry;
 

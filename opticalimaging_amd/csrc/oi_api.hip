@@ -266,8 +266,8 @@ static int plan_geometry(const oi_geometry& in, oi_geometry& g, bool generic = f
       g.lr = g.lc = lr = lc = L;
     }
   }
-  // Two-pass path: coarse grids beyond one workgroup's reach (L = 256, 512)
-  // when the window folds onto them without collisions.
+  // Two-pass path: coarse grids beyond one workgroup's reach (144 to 1024), when
+  // the window folds onto them without collisions.
   if (g.path == 0 && fast) {
     const int need = (2 * band_r - 1) > (2 * band_c - 1) ? 2 * band_r - 1 : 2 * band_c - 1;
     // coarse grids past one workgroup's reach, the smallest that holds the band

@@ -403,8 +403,8 @@ __global__ void k_diag(const double2* __restrict__ A, int n, double* __restrict_
 // (its inverse factor Linv_k kept), tile (I, J), k < J <= I, takes
 // A_IJ -= L_I L_J^T with L_I = A_Ik Linv_k^T formed in place by every tile (no
 // launch between panel and update), and tile (k + 1, k + 1) factors itself.
-// Bound by the 32 dependent pivots of each panel (about 13 us a launch, 0.1 ms
-// at n = 240, where the eigenvalues cost 4.1 ms); the factor is not kept.
+// Bound by the 32 dependent pivots of each panel (33 us a launch, 0.28 ms at n =
+// 240, where the eigenvalues cost 4.1 ms); the factor is not kept.
 constexpr int kCb = 32, kCs = kCb + 1;
 
 // In LDS: S (lower triangle) is factored, W = the factor's inverse.  False

@@ -644,7 +644,7 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
 }
 
 // ------------------------------------------------ two-pass coherent sum
-// For coarse grids too large for one workgroup (L = 256, 512).  Pass 1
+// For coarse grids whose tile no workgroup holds (100, 128, 144 to 1024).  Pass 1
 // transforms every window column of every (kernel, channel) into
 // B[img][kc][t][c] (row-major, t the coarse row); pass 2 gives each wavefront
 // 64 / T coarse rows, loops over all (kernel, channel) pairs reading its rows

@@ -231,7 +231,7 @@ def real_mask_kernels(ks: KernelSet, rel_tol: float = 1e-10) -> KernelSet:
     G = 0.5 * (G + G.transpose(0, 1))
     # r >= 2K - 1 (nothing to gain) follows when every eigenvalue exceeds half
     # the part of the trace that may be dropped: a Cholesky factorisation shows
-    # it in 0.2 ms at K = 120 where the eigenvalues take 4 (2 % above the half,
+    # it in 0.3 ms at K = 120 where the eigenvalues take 4 (2 % above the half,
     # far more than its rounding of 2K eps)
     if _sym_above(G, 0.51 * rel_tol):
         return ks

@@ -183,7 +183,8 @@ constexpr int rows_per_block() {
   return (kRegBlock / 64) * (64 / P::T);
 }
 
-template <class P>
+// KERN: kernel x spectrum; without: the spectrum alone (gamma's).
+template <class P, bool KERN>
 __global__ __launch_bounds__(kRegBlock) void k_adj_cfield_reg(const float2* __restrict__ spec,
                                                               const float2* __restrict__ kern,
                                                               int nk, int k0r, int wr, int wc,
@@ -197,26 +198,24 @@ __global__ __launch_bounds__(kRegBlock) void k_adj_cfield_reg(const float2* __re
   const bool on = tg < T && kc < wc;
   const int t = tg < T ? tg : 0;
   const float2* sb = spec + (size_t)b * wr * wc + (on ? kc : 0);
+  const float2* kb = KERN ? kern + (size_t)k * wr * wc + (on ? kc : 0) : nullptr;
   const int r0 = pmod(t - k0r, L);                    // T m < L: ir = r0 + T m, less L once
-  auto row = [&](int m) {
-    const int ir = r0 + T * m;
-    return ir >= L ? ir - L : ir;
-  };
-  // every load at a valid address, as in the forward's k_fp_bcols; kernel x
-  // spectrum as it forms it, so that Ec holds the same bits as its buffer.  One
-  // test of kern for all values: a test for each left the loads waiting for one
-  // another (coarse 200, one kernel of 121 columns: 11.4 us, 7.4 so).
   float2 v[V];
 #pragma unroll
-  for (int m = 0; m < V; ++m) v[m] = sb[on && row(m) < wr ? row(m) * wc : 0];
-  if (kern) {
-    const float2* kb = kern + (size_t)k * wr * wc + (on ? kc : 0);
-#pragma unroll
-    for (int m = 0; m < V; ++m) v[m] = reg::mul_rn(kb[on && row(m) < wr ? row(m) * wc : 0], v[m]);
+  for (int m = 0; m < V; ++m) {
+    int ir = r0 + T * m;
+    ir = ir >= L ? ir - L : ir;
+    // every load at a valid address, as in the forward's k_fp_bcols; kernel x
+    // spectrum as it forms it, so that Ec holds the same bits as its buffer.  KERN
+    // is a template argument: a test of the pointer at each value left the loads
+    // waiting for one another (coarse 200, one kernel of 121 columns: 11.4 us, 6.6
+    // without)
+    const bool in = on && ir < wr;
+    const int at = in ? ir * wc : 0;
+    float2 a = sb[at];
+    if constexpr (KERN) a = reg::mul_rn(kb[at], a);
+    v[m] = in ? a : make_float2(0.f, 0.f);
   }
-#pragma unroll
-  for (int m = 0; m < V; ++m)
-    if (!(on && row(m) < wr)) v[m] = make_float2(0.f, 0.f);
   P::template run_live_tab<false>(v, lds + g * (P::LDS | 1), t, twt, on);
   if (!on) return;
   float2* out = Ec + ((size_t)b * nk + k) * L * wc + kc;
@@ -348,11 +347,12 @@ static int adj_cfield_reg(int L, dim3 grid_y_z, const float2* spec, const float2
   if (L == NN) {                                                                               \
     using P = reg::GFFT<NN, A, B>;                                                             \
     constexpr int G = cols_per_block<P>();                                                     \
-    int rc = allow_lds_adj(k_adj_cfield_reg<P>, adj_cols_lds<P>());                             \
+    const auto run = kern ? k_adj_cfield_reg<P, true> : k_adj_cfield_reg<P, false>;            \
+    int rc = allow_lds_adj(run, adj_cols_lds<P>());                                            \
     if (rc) return rc;                                                                         \
     dim3 grid((wc + G - 1) / G, grid_y_z.y, grid_y_z.z);                                       \
-    hipLaunchKernelGGL(k_adj_cfield_reg<P>, grid, dim3(kRegBlock), adj_cols_lds<P>(), st, spec, \
-                       kern, nk, k0r, wr, wc, twt, Ec);                                        \
+    hipLaunchKernelGGL(run, grid, dim3(kRegBlock), adj_cols_lds<P>(), st, spec, kern, nk, k0r, \
+                       wr, wc, twt, Ec);                                                       \
     OI_LAUNCH_CHECK("adj_cfield_reg");                                                         \
     return OI_OK;                                                                              \
   }

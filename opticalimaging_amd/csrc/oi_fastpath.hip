@@ -658,25 +658,26 @@ __global__ __launch_bounds__(NT) void k_fp_coh(FpCoh A) {
 // share.  Bound by the stores of B and by arithmetic: 16 images x 12 kernels x
 // 107 columns of 256 in 17 us (42 MB; 20 with the blocks over all XCDs, 25 with
 // the exchange inside one wave, four columns each), 4 x 12 x 214 of 450 in 20
-// (27 with its loads under the window's condition).
-template <class PL>
+// (27 with its loads under the window's condition).  PART (both passes): some of the
+// kernel groups, where the allocation-free entry point holds no more at a time.
+template <class PL, bool PART>
 __global__ __launch_bounds__(kBlock) void k_fp_bcols(const float2* __restrict__ spec,
                                                      const float2* __restrict__ kern,
                                                      size_t spec_img, size_t kern_img, int nk,
                                                      int nchan, int groups, int first, int count,
-                                                     int slots, int k0r, int wr, int wc,
+                                                     int part_slots, int k0r, int wr, int wc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ B, int batch) {
   constexpr int L = PL::N, TL = PL::T, VL = PL::V, G = groups_per_block<PL>();
   extern __shared__ float2 lds[];
-  const int nxb = (wc + G - 1) / G;
+  const int nxb = (wc + G - 1) / G, slots = PART ? part_slots : nk * nchan;
   int w;
   if (!xcd_item(blockIdx.x, nxb * slots * batch, w)) return;   // uniform over the block
   const int g = threadIdx.x % G, tg = threadIdx.x / G;
   const int c = w % nxb * G + g;
   const int slot = (w / nxb) % slots, img = w / (nxb * slots);
   int kc = slot;                                           // k * nchan + channel
-  if (count < groups) {                                    // uniform over the grid
+  if constexpr (PART) {
     kc = slot / count * groups + first + slot % count;
     if (kc >= nk * nchan) return;                          // uniform over the block
   }
@@ -737,12 +738,12 @@ constexpr int brows_min_blocks() {
 // 56 -> 32; with the groups that brows_groups chooses 18, 21 (at L = 200) and 22.
 // Loading the next kernel's row ahead needs 32 more registers and
 // gives up a wave per SIMD for it: 21, 32 and 49 us.
-template <class PL>
+template <class PL, bool PART>
 __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(const float2* __restrict__ B, int nkc, int k0c,
                                                      int wc, int qc,
                                                      const float2* __restrict__ twt,
                                                      float2* __restrict__ R, int batch,
-                                                     int groups, int first, int count, int slots) {
+                                                     int groups, int first, int part, int part_slots) {
   constexpr int L = PL::N, TL = PL::T, VL = PL::V, GW = 64 / TL, RB = brows_rows<PL>();
   static_assert(VL <= 32, "row mask holds VL bits");
   extern __shared__ float2 lds[];
@@ -750,8 +751,9 @@ __global__ __launch_bounds__(kBlock, brows_min_blocks<PL>()) void k_fp_brows(con
   // their ends
   constexpr int NXR = (L + RB - 1) / RB;
   int w;
+  const int count = PART ? part : groups, slots = PART ? part_slots : nkc;
   if (!xcd_item(blockIdx.x, NXR * batch * count, w)) return;   // uniform over the block
-  const int xr = w % NXR, at = (w / NXR) % count, img = w / (NXR * count), grp = first + at;
+  const int xr = w % NXR, at = (w / NXR) % count, img = w / (NXR * count), grp = PART ? first + at : at;
   const int lane = threadIdx.x & 63, gw = lane / TL;
   const int t = gw < GW ? lane - gw * TL : 0;
   const int g = (threadIdx.x >> 6) * GW + (gw < GW ? gw : 0);
@@ -1314,23 +1316,23 @@ static size_t two_pass_rows_lds() {
   return (size_t)brows_rows<PL>() * PL::LDS * sizeof(float2);
 }
 
-template <class PL>
+template <class PL, bool PART>
 static int run_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st) {
   constexpr int G = groups_per_block<PL>(), RB = brows_rows<PL>();
   const size_t lds1 = bcols_lds<PL>();
-  int rc = allow(k_fp_bcols<PL>, lds1);
+  int rc = allow(k_fp_bcols<PL, PART>, lds1);
   if (rc) return rc;
   const int slots = fp_two_pass_slots(c.nkern * c.nchan, c.groups, c.count);
   const int cols = ((a.wc + G - 1) / G) * slots * a.batch;
-  hipLaunchKernelGGL(k_fp_bcols<PL>, dim3(xcd_grid(cols)), dim3(kBlock), lds1, st, c.spec, c.kern,
+  hipLaunchKernelGGL((k_fp_bcols<PL, PART>), dim3(xcd_grid(cols)), dim3(kBlock), lds1, st, c.spec, c.kern,
                      c.spec_img, c.kern_img, c.nkern, c.nchan, c.groups, c.first, c.count, slots,
                      a.k0r, a.wr, a.wc, a.tw_l, B, a.batch);
   OI_LAUNCH_CHECK("fp_bcols");
   const size_t lds2 = two_pass_rows_lds<PL>();
-  rc = allow(k_fp_brows<PL>, lds2);
+  rc = allow(k_fp_brows<PL, PART>, lds2);
   if (rc) return rc;
   const int items = ((PL::N + RB - 1) / RB) * a.batch * c.count;
-  hipLaunchKernelGGL(k_fp_brows<PL>, dim3(xcd_grid(items)), dim3(kBlock), lds2, st, B,
+  hipLaunchKernelGGL((k_fp_brows<PL, PART>), dim3(xcd_grid(items)), dim3(kBlock), lds2, st, B,
                      c.nkern * c.nchan, a.k0c, a.wc, a.qc, a.tw_l, c.R, a.batch,
                      c.groups, c.first, c.count, slots);
   OI_LAUNCH_CHECK("fp_brows");
@@ -1406,7 +1408,10 @@ size_t fp_two_pass_lds(int L) {
 
 int fp_two_pass(const FpArgs& a, const FpCoh& c, float2* B, hipStream_t st) {
   int rc = OI_ERR_UNSUPPORTED;
-#define X(NN, A, B_) if (a.L == NN) rc = fp::run_two_pass<reg::GFFT<NN, A, B_>>(a, c, B, st);
+#define X(NN, A, B_)                                                                       \
+  if (a.L == NN)                                                                          \
+    rc = c.count < c.groups ? fp::run_two_pass<reg::GFFT<NN, A, B_>, true>(a, c, B, st)   \
+                            : fp::run_two_pass<reg::GFFT<NN, A, B_>, false>(a, c, B, st);
   OI_TWO_PASS_PLANS(X)
   OI_SPLIT_PLANS(X)
 #undef X

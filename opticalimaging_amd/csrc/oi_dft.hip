@@ -606,22 +606,23 @@ int dft_table_build(const float2* tw, int n, int amax, float* mem, DftTable& t, 
 // Of 472 windows, batches and sizes from 225 to 1920 the choice takes 0.5 % (real
 // rows), 1.2, 1.1 and 1.7 % longer than the better form of each.  It goes by the
 // plan's batch: an image is the same in every call.
-static bool wide(int orders, int most, long long values, long long enough) {
-  return orders > most && values >= enough;
+// Lines past 10240 points do not fit the transforms' LDS and stay products.
+static bool wide(int n, int orders, int most, long long values, long long enough) {
+  return orders > most && values >= enough && 2 * (size_t)n * sizeof(float2) <= kLdsLimit;
 }
 
 bool dft_rows_ok(const FpArgs& a) {
   const long long values = (long long)a.ny * a.nx * a.images;
-  if (a.kind == OI_FIELD_C64_CHLAST) return !wide(a.wc, 256, values * a.nchan, 1000000);
-  return !wide(a.wc, a.nx % 2 ? 256 : 600, values / 2, 1000000);
+  if (a.kind == OI_FIELD_C64_CHLAST) return !wide(a.nx, a.wc, 256, values * a.nchan, 1000000);
+  return !wide(a.nx, a.wc, a.nx % 2 ? 256 : 600, values / 2, 1000000);
 }
 
 bool dft_cols_ok(const FpArgs& a) {
-  return !wide(a.wr, 256, (long long)a.wc * a.ny * a.nchan * a.images, 600000);
+  return !wide(a.ny, a.wr, 256, (long long)a.wc * a.ny * a.nchan * a.images, 600000);
 }
 
 bool dft_ucols_ok(const FpArgs& a) {
-  return !wide(2 * a.qr + 1, a.ny % 2 ? 160 : 256, (long long)(a.qc + 1) * a.ny * a.images, 300000);
+  return !wide(a.ny, 2 * a.qr + 1, a.ny % 2 ? 160 : 256, (long long)(a.qc + 1) * a.ny * a.images, 300000);
 }
 
 int dft_rows(const FpArgs& a, hipStream_t st) {

@@ -124,3 +124,20 @@ def test_band_products_and_transforms(gpu, ny, nx, q):
         assert np.max(np.abs(img[b] - ref)) <= IMAGE_TOL * ref.max()
         ref = _gradient(full, h[b], g[b])
         assert np.max(np.abs(grad[b] - ref)) <= GRAD_TOL * np.abs(ref).max()
+
+
+def test_lines_past_the_transforms(gpu):
+    """12000 points stay products at any window: no LDS holds their transform."""
+    from opticalimaging_amd import _native as nat
+    ny, nx, wc = 960, 12000, 300
+    rng = np.random.default_rng(5)
+    win = (rng.standard_normal((1, 9, wc)) + 1j * rng.standard_normal((1, 9, wc))).astype(np.complex64)
+    full = np.zeros((1, ny, nx), np.complex128)
+    full[np.ix_([0], (np.arange(9) - 4) % ny, (np.arange(wc) - 150) % nx)] = win
+    ks = engine.KernelSet(torch.as_tensor(win).cuda(), -4, -150, ny, nx)
+    info = engine.plan_for(ks, 1, 1).info()
+    assert (info["path"], info["lr"]) == (2, 900)
+    h = (rng.standard_normal((1, ny, nx)) + 1j * rng.standard_normal((1, ny, nx))).astype(np.complex64)
+    img = engine.socs_image(torch.as_tensor(h[..., None]).cuda(), ks, kind=nat.OI_FIELD_C64_CHLAST).cpu().numpy()
+    ref = _image(full, h[0])
+    assert np.max(np.abs(img[0] - ref)) <= IMAGE_TOL * ref.max()
